@@ -923,21 +923,36 @@ def _group_bounds(lb: str, k: int, ngroups: int) -> str:
         return LAUNCH_BOUNDS["lb1" if k == ngroups - 1 else "lb2"]
     return LAUNCH_BOUNDS[lb]
 
-# Candidate schedules per build: (kind, partition, launch bounds).
-# Candidate schedules built per workload: the plain one-thread-per-point schedule first (the
-# fallback for input that is not 16-byte aligned), then the tuned workgroup-tiled schedules
-# and their nearest alternatives.  Schedules the autotuner measured slower on every workload
-# are no longer built (their timings stay in the tuned tables under nrpy_amd/autotune/).
+# Candidate schedules built per workload, from the general to the preferred one: a patch runs
+# the last of its list that takes its size (``default_schedule`` in bhah_hip.hip) until another
+# is selected.  The plain one-thread-per-point schedule comes first (any size and alignment).
+# What decides between the forms, measured per launch on MI355X:
+#   * _dmo takes rows of any length; _dma needs even ones and has a box two values narrower
+#     where the stencils reach NGHOSTS: rhs fd6 752 against 820 us at 192x96x96, 208 against 207
+#     at 128x64x64 and 127x63x62 (the plain schedule: 1032 us there).
+#   * Small workgroups suit the kernels whose boxes are small: a wave then waits for its own
+#     box instead of three other waves', and several workgroups of a CU are at different
+#     points.  Ricci fd6, 64 threads against 256: 314 against 360 us at 192x96x96; fd4: 35.4
+#     against 41.0 at 96x48x48; phi-symmetric: 23.0 against 29.4 at 256x64x16.  rhs
+#     phi-symmetric (no xx2 halo): 42.9 against 59.3.  The 3D right-hand side's boxes reach
+#     three or four points every way; there a 64-thread tile stages nine boxes' worth of
+#     halo and loses (99 against 75 us, fd4 at 96x48x48).
 FULL_CANDIDATES = {
     "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_mi_xcd", "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk",
+            "p1_lb1_sj_L16x4x4x1_d4_dmo_rb1_io_pg_ub_sa_lr40_di_mi_blk_xcd",
             "p1_lb1_sj_L16x4x4x1_d4_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk"],
-    "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg2_mi_xcd", "r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_lr40_mi_xcd"],
+    "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_lr40_mi_xcd",
+              "r1_lb1_sj_L16x2x2x1_d3_dmo_rb1_io_pg_lr40_di_mi_xcd", "r1_lb1_sj_L16x2x2x1_d3_dma_rb1_io_pg_lr40_di_mi_xcd"],
+}
+FULL_FD4_CANDIDATES = {
+    "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d4_dmo_rb1_io_pg_ub_sa_lr40_di_mi_xcd"],
+    "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x1x1_d3_dmo_rb1_io_pg_lr40_di_mi_xcd"],
 }
 SMALL_CANDIDATES = {"rhs": ["p1_lb1", "p1_lb1_sl_lf_pf16_u32_w2", "p1_lb1_sj_L16x8x2x1_d3_dma_rb1",
                             "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8", "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8_ub",
-                            "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8_ub_mi"],
-                    "ricci": ["r1_lb1", "r1_lb1_pf16_u32", "r1_lb1_sj_L16x4x4x1_d2_dma_xcd",
-                              "r1_lb1_sj_L16x8x2x1_d3_dma_rb1", "r1_lb1_sj_L16x8x2x1_d3_dma_rb1_mi"]}
+                            "p1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_ub_lr40_di_mi_xcd"],
+                    "ricci": ["r1_lb1", "r1_lb1_pf16_u32", "r1_lb1_sj_L16x8x2x1_d3_dma_rb1",
+                              "r1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_lr40_di_mi_xcd"]}
 
 CAND_SIG = ("dim3 g, dim3 b, hipStream_t s, const double *in, const double *aux, double *out, "
             "const double *rfm0, const double *rfm1, bhah_kparams p")
@@ -960,13 +975,17 @@ LDS_PIN_MACRO = """#ifndef BHAH_PIN
 class _LdsEmitter(StencilEmitter):
     """Stencil expressions reading a workgroup's LDS box ``sh`` around box index ``c``."""
 
-    def __init__(self, spec: specs.Spec, fd_order: int, centre: str, BX: int, BY: int, base: int = 0):
+    def __init__(self, spec: specs.Spec, fd_order: int, centre: str, BX: int, BY: int, base: int = 0,
+                 odd_rows: bool = False):
         super().__init__(spec, fd_order)
-        self.centre, self.BX, self.BY, self.base = centre, BX, BY, base
+        self.centre, self.BX, self.BY, self.base, self.odd_rows = centre, BX, BY, base, odd_rows
 
     def load(self, gf: str, off: Tuple[int, int, int]) -> str:
         o = self.base + off[0] + self.BX * off[1] + self.BX * self.BY * off[2]
-        return f"sh[{self.centre}{f' + {o}' if o > 0 else (f' - {-o}' if o < 0 else '')}]"
+        # with odd_rows a row's place in the box depends on the parity of its offset from the
+        # thread's own row
+        c = self.centre + (("", "y", "z", "w")[(off[1] & 1) + 2 * (off[2] & 1)] if self.odd_rows else "")
+        return f"sh[{c}{f' + {o}' if o > 0 else (f' - {-o}' if o < 0 else '')}]"
 
 
 def _lds_tile_order(xcd: bool, zfirst: bool, blocked: bool = False) -> str:
@@ -980,7 +999,8 @@ def _lds_tile_order(xcd: bool, zfirst: bool, blocked: bool = False) -> str:
     grids that do not divide into such blocks keep the linear order."""
     if not (xcd or zfirst or blocked):
         return "  const unsigned bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;"
-    lin = ("((n & 7u) == 0u) ? (h & 7u) * (n >> 3) + (h >> 3) : h" if xcd else "h")
+    # n = 8 q + r tiles: XCD k takes q, or q + 1 of them for k < r
+    lin = ("(h & 7u) * (n >> 3) + min((int)(h & 7u), (int)(n & 7u)) + (h >> 3)" if xcd else "h")
     dec = ("bz = l % gz;\n    bx = (l / gz) % gx;\n    by = l / (gz * gx);" if zfirst else
            "bx = l % gx;\n    by = (l / gx) % gy;\n    bz = l / (gx * gy);")
     if blocked:
@@ -1017,16 +1037,31 @@ LDS_DMA_MACROS = """#ifndef BHAH_DMA16
 """
 
 
-def _lds_offsets(dma: bool, H: int, SH: int, NJ: int, NL: int) -> str:
+def _lds_offsets(dma: bool, H: int, HZ: int, SH: int, NJ: int, NL: int, odd_rows: bool = False) -> str:
     """Per-thread global offsets of the box elements it loads.  Indices are clamped into
     the array, so partial tiles at the upper interior edge read valid (unused) points."""
+    if odd_rows:
+        # Each box row starts at the even flat index at or below its first point, so every
+        # pair is 16-byte aligned whatever the parity of Nx0.  A pair may run past its row's
+        # end (into the next row: valid memory, unused values); only past the gridfunction's
+        # end is it clamped (Ntot is even, checked by the host).
+        return f"""  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  unsigned pofs[{NJ}];
+#pragma unroll
+  for (int j = 0; j < {NJ}; j++) {{
+    const int e = 2 * (tid + NT * j);
+    const int ex = e % BX, ey = (e / BX) % BY, ez = e / (BX * BY);
+    const int g1 = min(o1 - {H} + ey, p.Nx1 - 1), g2 = min(o2 - {HZ} + ez, p.Nx2 - 1);
+    const int row = (o0 - {H} + (int)s1 * g1 + (int)s2 * g2) & ~1;
+    pofs[j] = 8u * (unsigned)min(row + ex, (int)Ntot - 2);
+  }}"""
     if not dma:
         return f"""  int ofs[NL];
 #pragma unroll
   for (int j = 0; j < NL; j++) {{
     const int e = tid + NT * j;
     const int ex = e % BX, ey = (e / BX) % BY, ez = e / (BX * BY);
-    const int g0 = min(o0 - {H} + ex, p.Nx0 - 1), g1 = min(o1 - {H} + ey, p.Nx1 - 1), g2 = min(o2 - {H} + ez, p.Nx2 - 1);
+    const int g0 = min(o0 - {H} + ex, p.Nx0 - 1), g1 = min(o1 - {H} + ey, p.Nx1 - 1), g2 = min(o2 - {HZ} + ez, p.Nx2 - 1);
     ofs[j] = g0 + (int)s1 * g1 + (int)s2 * g2;
   }}"""
     # pair j of this thread: box elements 2q, 2q + 1 (q = tid + NT j) are xx0 neighbours
@@ -1041,7 +1076,7 @@ def _lds_offsets(dma: bool, H: int, SH: int, NJ: int, NL: int) -> str:
   for (int j = 0; j < {NJ}; j++) {{
     const int e = 2 * (tid + NT * j);
     const int ex = e % BX, ey = (e / BX) % BY, ez = e / (BX * BY);
-    const int g0 = min(o0 - {H + SH} + ex, p.Nx0 - 2), g1 = min(o1 - {H} + ey, p.Nx1 - 1), g2 = min(o2 - {H} + ez, p.Nx2 - 1);
+    const int g0 = min(o0 - {H + SH} + ex, p.Nx0 - 2), g1 = min(o1 - {H} + ey, p.Nx1 - 1), g2 = min(o2 - {HZ} + ez, p.Nx2 - 1);
     pofs[j] = 8u * (unsigned)(g0 + (int)s1 * g1 + (int)s2 * g2);
   }}"""
 
@@ -1122,7 +1157,7 @@ def _int_line_sum(W: Dict[int, int], pts: Dict[int, str], mirror: str) -> Tuple[
     return f"({' + '.join(parts)})", fl
 
 
-_SH_REF = re.compile(r"sh\[c\d+(?: [+-] \d+)?\]")
+_SH_REF = re.compile(r"sh\[c\d+[yzw]?(?: [+-] \d+)?\]")
 
 
 def _batch_lds_reads(stmts: List[Tuple[str, List[str]]], nmax: int, prefix: str) -> List[Tuple[str, List[str]]]:
@@ -1184,7 +1219,8 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
                depth: int = 1, zfirst: bool = False, group: int = 1, dma: bool = False,
                one_barrier: bool = False, ensemble: str = "", interleave: bool = False,
                pin_group: int = -1, branchless_upwind: bool = False, blocked: bool = False,
-               sym_lines: bool = False, read_batch: int = 0, dma_spread: bool = False) -> Tuple[str, str, int]:
+               sym_lines: bool = False, read_batch: int = 0, dma_spread: bool = False,
+               odd_rows: bool = False) -> Tuple[str, str, int]:
     """One workgroup-tiled kernel.  Each gridfunction with derivatives is staged, one at a
     time, from global memory into a halo box in LDS: ``group`` gridfunctions per
     barrier-separated phase, with the loads of the next ``depth`` phases in flight while
@@ -1197,7 +1233,13 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
     with explicit vmcnt waits counted per phase (``one_barrier``: one barrier per phase,
     refilling the slot the previous phase read).  The box's xx0 origin is rounded down
     to an even index (every pair 16-byte aligned), which needs an even Nx0 (checked by the
-    host).
+    host).  With ``odd_rows`` every row's own origin is rounded down to an even flat index
+    instead, which any Nx0 allows: a row then starts in its box at its first point or one
+    point before, and the reads go through four base indices, by the parity of the row's
+    distance in xx1 and xx2 from the thread's own row.
+
+    The box has a halo along xx2 only where the kernel differentiates along xx2 (a
+    phi-symmetric build does not).
 
     With ``ensemble`` (a kernel name) the source also holds the batched-ensemble form: the
     per-tile code as a device function and a kernel walking (member, tile) records, tiles in
@@ -1241,6 +1283,7 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
             line_cf.setdefault(key, {})["up" if d.op == "dupD" else "ko"] = cidx[c]
             line_out[key] = g_out
     H = fd.ghost_zones(fd_order) if terms else fd_order // 2
+    HZ = H if any(2 in d.dirs for d in dused) or any(k[1] == 2 for k in line_out) else 0
     staged = [g for g in sub.gfs if any(d.gf == g for d in dused) or any(k[0] == g for k in line_out)]
     if interleave:
         # spread the gridfunctions with mixed second derivatives (several times the LDS reads
@@ -1258,7 +1301,9 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
     SH = ((fd.ghost_zones(fd_order) - H) & 1) if dma else 0
     if dma and TX % 2:
         raise ValueError("DMA staging needs an even tile width")
-    BX, BY, BZ = TX + 2 * H + 2 * SH, TY + 2 * H, TZ + 2 * H
+    if odd_rows and not dma:
+        raise ValueError("odd_rows is a form of the DMA staging")
+    BX, BY, BZ = TX + 2 * H + (2 if odd_rows else 2 * SH), TY + 2 * H, TZ + 2 * HZ
     NB = BX * BY * BZ
     NL = (NB + NT - 1) // NT
     NJ = (NB // 2 + NT - 1) // NT  # 16-byte DMA loads per thread per box
@@ -1294,9 +1339,16 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
   const int lx = tid % {TX}, ly = (tid / {TX}) % {TY}, lz = tid / {TX * TY};
   const long s1 = p.s1, s2 = p.s2, Ntot = p.Ntot;
   const int o0 = p.NG + (int)bx * {TX}, o1 = p.NG + (int)by * {TY}, o2 = p.NG + (int)bz * {TZ};
-{_lds_offsets(dma, H, SH, NJ, NL)}""")
+{_lds_offsets(dma, H, HZ, SH, NJ, NL, odd_rows)}""")
     for k in range(P):
-        a(f"  const int c{k} = (lx + {H + SH}) + BX * (ly + {H}) + BX * BY * (lz + {k * ZS + H});")
+        if not odd_rows:
+            a(f"  const int c{k} = (lx + {H + SH}) + BX * (ly + {H}) + BX * BY * (lz + {k * ZS + HZ});")
+            continue
+        # q: 1 where the row of this thread's point starts at an odd flat index
+        a(f"""  const int c{k}b = (lx + {H}) + BX * (ly + {H}) + BX * BY * (lz + {k * ZS + HZ});
+  const int q{k} = (o0 - {H} + (int)s1 * (o1 + ly) + (int)s2 * (o2 + lz + {k * ZS})) & 1;
+  const int c{k} = c{k}b + q{k}, c{k}y = c{k}b + (q{k} ^ ((int)s1 & 1)), c{k}z = c{k}b + (q{k} ^ ((int)s2 & 1)),
+            c{k}w = c{k}b + (q{k} ^ ((int)(s1 + s2) & 1));""")
     # Upwind sums are formed with integer weights (their common denominator DU moved into
     # one uniform scale per direction): an FP64 multiply-add takes an integer weight as an
     # instruction literal, where a weight such as 1/30 needs a register pair loaded first.
@@ -1380,7 +1432,7 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
                     pins.clear()
 
             for k in range(P):
-                st = _LdsEmitter(sub, fd_order, f"c{k}", BX, BY, box(ph, q))
+                st = _LdsEmitter(sub, fd_order, f"c{k}", BX, BY, box(ph, q), odd_rows)
                 stmts: List[Tuple[str, List[str]]] = []  # (statement, values it forms)
                 if g in ovr and g in used:
                     stmts.append((f"  double V{k}_{g} = {st.load(g, (0, 0, 0))};", [f"V{k}_{g}"]))
@@ -1638,11 +1690,11 @@ def candidate_tu(v: specs.Variant, fd_order: int, kind: str, cand: str, ensemble
                                          depth=next((int(o[1:]) for o in opts if o[0] == "d" and o[1:].isdigit()), 1),
                                          zfirst="zf" in opts, blocked="blk" in opts,
                                          group=next((int(o[1:]) for o in opts if o[0] == "g" and o[1:].isdigit()), 1),
-                                         dma="dma" in opts, one_barrier="rb1" in opts, ensemble=ename,
+                                         dma="dma" in opts or "dmo" in opts, one_barrier="rb1" in opts, ensemble=ename,
                                          interleave="io" in opts,
                                          branchless_upwind="ub" in opts, sym_lines="sa" in opts,
                                          read_batch=next((int(o[2:]) for o in opts if o[:2] == "lr" and o[2:].isdigit()), 0),
-                                         dma_spread="di" in opts,
+                                         dma_spread="di" in opts, odd_rows="dmo" in opts,
                                          pin_group=next((int(o[2:] or 0) for o in opts if o[:2] == "pg" and o[2:].isdigit() or o == "pg"), -1))
             kernels.append(src)
             calls.append(launch)
@@ -2061,7 +2113,7 @@ extern "C" hipError_t launch_wave_rhs_rk_{tag}(dim3 g, dim3 b, hipStream_t s, co
 BSSN_BUILDS = [
     (specs.VARIANTS[0], 4, SMALL_CANDIDATES, True),
     (specs.VARIANTS[1], 6, FULL_CANDIDATES, False),
-    (specs.VARIANTS[1], 4, SMALL_CANDIDATES, False),
+    (specs.VARIANTS[1], 4, FULL_FD4_CANDIDATES, False),
 ]
 WAVE_BUILDS = [4]
 COORD_ENUM = {"Cartesian": 0, "Spherical": 1, "SinhSpherical": 2}

@@ -1219,6 +1219,35 @@ int noalloc_scratch(double **out) {
   return BHAH_OK;
 }
 
+// Whether schedule `nm` can run on patch P: BHAH_OK, or an error naming the size it cannot take.
+int schedule_fits(const bhah_patch *P, const char *nm) {
+  if (strstr(nm, "_u32") && P->Ntot * 24 * 8 >= (1L << 31))
+    return fail(BHAH_ERR_UNSUPPORTED, "schedule %s addresses arrays below 2 GiB only", nm);
+  // Staged schedules named _dmo round every row's origin to an even flat index, which only needs
+  // gridfunctions of even length; those named _dma take rows of even length.
+  if (strstr(nm, "_dmo") && ((P->Ntot & 1) || P->Ntot >= (1L << 29)))
+    return fail(BHAH_ERR_UNSUPPORTED, "schedule %s needs an even number of gridpoints below 2^29 (have %ld)", nm,
+                P->Ntot);
+  if (strstr(nm, "_dma") && (P->Nx[0] & 1))
+    return fail(BHAH_ERR_UNSUPPORTED, "schedule %s loads xx0 pairs and needs an even Nx0 (have %d)", nm, P->Nx[0]);
+  if (strstr(nm, "_dma") && P->Ntot * 8 >= (1L << 32))
+    return fail(BHAH_ERR_UNSUPPORTED, "schedule %s addresses a gridfunction below 4 GiB only", nm);
+  return BHAH_OK;
+}
+
+// The schedule a patch starts with: the last candidate of its build that takes its size (the
+// generator lists them from the general to the preferred form).
+int default_schedule(const bhah_patch *P, const BssnCandidate *c, int n) {
+  const std::string before = g_last_error;
+  int i = n - 1;
+  while (i > 0 && schedule_fits(P, c[i].name)) i--;
+  g_last_error = before;
+  return i;
+}
+
+// Whether schedule `nm` fills its boxes with 16-byte loads (its input must be 16-byte aligned).
+bool pair_loads(const char *nm) { return strstr(nm, "_dma") || strstr(nm, "_dmo"); }
+
 // L2 and RMS columns of diags_integration_write_row (diagnostics_volume_integration_helpers.h:332-345).
 void finish_volume_integrals(const double sums[VI_SUMS], bhah_volume_integrals *r) {
   for (int q = 0; q < BHAH_DIAG_NUM_RECIPES; q++) {
@@ -1654,6 +1683,12 @@ static int patch_upload(bhah_patch *P, const std::vector<double> &rfm0, const st
     bhah_hip_patch_destroy(P);
     return fail(BHAH_ERR_HIP, "hipMalloc failed");
   }
+  if (P->k) {
+    P->rhs_choice = default_schedule(P, P->k->rhs, P->k->n_rhs);
+    P->rhs_dma = pair_loads(P->k->rhs[P->rhs_choice].name);
+    P->ricci_choice = default_schedule(P, P->k->ricci, P->k->n_ricci);
+    P->ricci_dma = pair_loads(P->k->ricci[P->ricci_choice].name);
+  }
   P->stream = nullptr;  // default (null) stream unless set
   *out = P;
   return BHAH_OK;
@@ -2041,13 +2076,9 @@ int bhah_hip_patch_select_schedule(bhah_patch *P, int kind, int index) {
   if (n < 0) return n;
   if (index < 0 || index >= n) return fail(BHAH_ERR_ARG, "schedule index %d out of range [0,%d)", index, n);
   const char *nm = (kind == BHAH_KERNEL_RHS ? P->k->rhs : P->k->ricci)[index].name;
-  if (strstr(nm, "_u32") && P->Ntot * 24 * 8 >= (1L << 31))
-    return fail(BHAH_ERR_UNSUPPORTED, "schedule %s addresses arrays below 2 GiB only", nm);
-  const bool dma = strstr(nm, "_dma") != nullptr;
-  if (dma && (P->Nx[0] & 1))
-    return fail(BHAH_ERR_UNSUPPORTED, "schedule %s loads xx0 pairs and needs an even Nx0 (have %d)", nm, P->Nx[0]);
-  if (dma && P->Ntot * 8 >= (1L << 32))
-    return fail(BHAH_ERR_UNSUPPORTED, "schedule %s addresses a gridfunction below 4 GiB only", nm);
+  const int rc = schedule_fits(P, nm);
+  if (rc) return rc;
+  const bool dma = pair_loads(nm);
   if (kind == BHAH_KERNEL_RHS) {
     P->rhs_choice = index;
     P->rhs_dma = dma;
@@ -2564,7 +2595,9 @@ int ensemble_build_items(bhah_ensemble *E) {
 }
 
 // Tile list of a selected LDS-tiled schedule (kind 0: rhs, 1: Ricci): every member's interior
-// in the schedule's own TX x TY x TZ tiles.
+// in the schedule's own TX x TY x TZ tiles.  Workgroups go round-robin over the 8 XCDs, so the
+// list is dealt out such that XCD k walks its k-th contiguous eighth: neighbouring tiles, whose
+// halos overlap, then share an L2.
 int ensemble_build_lds_items(bhah_ensemble *E, int kind) {
   const BssnCandidate &c = kind == 0 ? E->k->rhs[E->rhs_choice] : E->k->ricci[E->ricci_choice];
   hipFree(E->d_lds[kind]);
@@ -2580,9 +2613,12 @@ int ensemble_build_lds_items(bhah_ensemble *E, int kind) {
       for (int by = 0; by < t1; by++)
         for (int bx = 0; bx < t0; bx++) v.push_back({m, bx, by, bz});
   }
+  const size_t n = v.size();
+  std::vector<bhah_item> order(n);
+  for (size_t h = 0; h < n; h++) order[h] = v[(h & 7) * (n >> 3) + std::min(h & 7, n & 7) + (h >> 3)];
   int rc;
-  if ((rc = upload(v, &E->d_lds[kind]))) return rc;
-  E->n_lds[kind] = (int)v.size();
+  if ((rc = upload(order, &E->d_lds[kind]))) return rc;
+  E->n_lds[kind] = (int)n;
   return BHAH_OK;
 }
 
@@ -2590,7 +2626,7 @@ int ensemble_enqueue_step(bhah_ensemble *E) {
   const int in_s[4] = {0, 2, 3, 2}, k_s[4] = {2, 3, 2, 3};
   const BssnCandidate &ric = E->k->ricci[E->ricci_choice], &rhs = E->k->rhs[E->rhs_choice];
   const dim3 tb(E->tile_x, E->tile_y, 1);
-  if (!E->aligned16 && (strstr(ric.name, "_dma") || strstr(rhs.name, "_dma")))
+  if (!E->aligned16 && (pair_loads(ric.name) || pair_loads(rhs.name)))
     return fail(BHAH_ERR_UNSUPPORTED, "schedules with 16-byte pair loads need 16-byte aligned member arrays");
   // LDS-tiled schedules walk their own tile lists (the launcher sets the workgroup size)
   const bhah_item *ric_items = ric.lds[0] ? E->d_lds[1] : E->d_int, *rhs_items = rhs.lds[0] ? E->d_lds[0] : E->d_int;
@@ -2783,12 +2819,8 @@ int bhah_hip_ensemble_select_schedule(bhah_ensemble *E, int kind, int index) {
   const BssnCandidate &c = (kind == BHAH_KERNEL_RHS ? E->k->rhs : E->k->ricci)[index];
   if (!c.ens) return fail(BHAH_ERR_UNSUPPORTED, "schedule %s has no batched form", c.name);
   for (const bhah_patch *P : E->P) {
-    if (strstr(c.name, "_u32") && P->Ntot * 24 * 8 >= (1L << 31))
-      return fail(BHAH_ERR_UNSUPPORTED, "schedule %s addresses arrays below 2 GiB only", c.name);
-    if (strstr(c.name, "_dma") && (P->Nx[0] & 1))
-      return fail(BHAH_ERR_UNSUPPORTED, "schedule %s loads xx0 pairs and needs an even Nx0 in every member", c.name);
-    if (strstr(c.name, "_dma") && P->Ntot * 8 >= (1L << 32))
-      return fail(BHAH_ERR_UNSUPPORTED, "schedule %s addresses a gridfunction below 4 GiB only", c.name);
+    const int rc = schedule_fits(P, c.name);
+    if (rc) return rc;
   }
   if (kind == BHAH_KERNEL_RHS) E->rhs_choice = index;
   else E->ricci_choice = index;

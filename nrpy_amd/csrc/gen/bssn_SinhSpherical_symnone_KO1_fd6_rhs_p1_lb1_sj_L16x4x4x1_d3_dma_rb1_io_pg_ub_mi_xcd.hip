@@ -41,7 +41,7 @@ bssn_rhs_SinhSpherical_symnone_KO1_fd6_p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_m
   {
     const unsigned gx = gridDim.x, gy = gridDim.y, gz = gridDim.z, n = gx * gy * gz;
     const unsigned h = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-    const unsigned l = ((n & 7u) == 0u) ? (h & 7u) * (n >> 3) + (h >> 3) : h;
+    const unsigned l = (h & 7u) * (n >> 3) + min((int)(h & 7u), (int)(n & 7u)) + (h >> 3);
     bx = l % gx;
     by = (l / gx) % gy;
     bz = l / (gx * gy);

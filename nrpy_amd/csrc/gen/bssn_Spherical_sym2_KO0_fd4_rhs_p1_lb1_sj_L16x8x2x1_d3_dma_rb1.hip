@@ -32,29 +32,29 @@
 #define Rational_3_4 (3.0 / 4.0)
 #define Rational_4_3 (4.0 / 3.0)
 
-// bhah-dma-issue bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0: 0:5 1:5 2:5 3:5 4:5 5:5 6:5 7:5 8:5 9:5 10:5 11:5 12:5 13:5 14:5 15:5 16:5 17:5 18:5 19:5 20:5 21:5 22:5 23:5
-// bhah-dma-issue bssn_ens_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0: 0:5 1:5 2:5 3:5 4:5 5:5 6:5 7:5 8:5 9:5 10:5 11:5 12:5 13:5 14:5 15:5 16:5 17:5 18:5 19:5 20:5 21:5 22:5 23:5
+// bhah-dma-issue bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0: 0:2 1:2 2:2 3:2 4:2 5:2 6:2 7:2 8:2 9:2 10:2 11:2 12:2 13:2 14:2 15:2 16:2 17:2 18:2 19:2 20:2 21:2 22:2 23:2
+// bhah-dma-issue bssn_ens_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0: 0:2 1:2 2:2 3:2 4:2 5:2 6:2 7:2 8:2 9:2 10:2 11:2 12:2 13:2 14:2 15:2 16:2 17:2 18:2 19:2 20:2 21:2 22:2 23:2
 extern "C" __global__ void __launch_bounds__(256)
 bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *__restrict__ in, const double *__restrict__ aux, double *__restrict__ out,
         const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p) {
-  __shared__ double sh[7680];
+  __shared__ double sh[3072];
   const unsigned bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
-  // Tile of 16x8x2 interior points; halo box 22x14x8 = 2464 values per gridfunction.
-  constexpr int BX = 22, BY = 14, NB = 2464, NT = 256, NL = 10;
+  // Tile of 16x8x2 interior points; halo box 22x14x2 = 616 values per gridfunction.
+  constexpr int BX = 22, BY = 14, NB = 616, NT = 256, NL = 3;
   const int tid = (int)threadIdx.x;
   const int lx = tid % 16, ly = (tid / 16) % 8, lz = tid / 128;
   const long s1 = p.s1, s2 = p.s2, Ntot = p.Ntot;
   const int o0 = p.NG + (int)bx * 16, o1 = p.NG + (int)by * 8, o2 = p.NG + (int)bz * 2;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  unsigned pofs[5];
+  unsigned pofs[2];
 #pragma unroll
-  for (int j = 0; j < 5; j++) {
+  for (int j = 0; j < 2; j++) {
     const int e = 2 * (tid + NT * j);
     const int ex = e % BX, ey = (e / BX) % BY, ez = e / (BX * BY);
-    const int g0 = min(o0 - 3 + ex, p.Nx0 - 2), g1 = min(o1 - 3 + ey, p.Nx1 - 1), g2 = min(o2 - 3 + ez, p.Nx2 - 1);
+    const int g0 = min(o0 - 3 + ex, p.Nx0 - 2), g1 = min(o1 - 3 + ey, p.Nx1 - 1), g2 = min(o2 - 0 + ez, p.Nx2 - 1);
     pofs[j] = 8u * (unsigned)(g0 + (int)s1 * g1 + (int)s2 * g2);
   }
-  const int c0 = (lx + 3) + BX * (ly + 3) + BX * BY * (lz + 3);
+  const int c0 = (lx + 3) + BX * (ly + 3) + BX * BY * (lz + 0);
   const double ius0 = p.invdxx0 * (1.0 / 12.0), nius0 = -ius0, ikos0 = p.invdxx0 * (1.0 / 64.0);
   const double ius1 = p.invdxx1 * (1.0 / 12.0), nius1 = -ius1, ikos1 = p.invdxx1 * (1.0 / 64.0);
   const double ius2 = p.invdxx2 * (1.0 / 12.0), nius2 = -ius2, ikos2 = p.invdxx2 * (1.0 / 64.0);
@@ -100,20 +100,20 @@ bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *
   {
     const char *src = (const char *)(in + 0 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
   {
     const char *src = (const char *)(in + 1 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
   // ---- aDD00
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(0);
   {
     const char *src = (const char *)(in + 2 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_aDD00 = sh[c0];
   BHAH_PIN(V0_aDD00);
@@ -122,40 +122,40 @@ bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *
   V0_lin_aDD00 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_aDD00);
   // ---- aDD01
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(1);
   {
     const char *src = (const char *)(in + 3 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_aDD01 = sh[c0 + 2560];
+  double V0_aDD01 = sh[c0 + 1024];
   BHAH_PIN(V0_aDD01);
-  V0_lin_aDD01 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_aDD01 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_aDD01);
-  V0_lin_aDD01 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_aDD01 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_aDD01);
   // ---- aDD02
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(2);
   {
     const char *src = (const char *)(in + 4 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_aDD02 = sh[c0 + 5120];
+  double V0_aDD02 = sh[c0 + 2048];
   BHAH_PIN(V0_aDD02);
-  V0_lin_aDD02 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_aDD02 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_aDD02);
-  V0_lin_aDD02 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_aDD02 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_aDD02);
   // ---- aDD11
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(3);
   {
     const char *src = (const char *)(in + 5 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_aDD11 = sh[c0];
   BHAH_PIN(V0_aDD11);
@@ -164,40 +164,40 @@ bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *
   V0_lin_aDD11 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_aDD11);
   // ---- aDD12
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(4);
   {
     const char *src = (const char *)(in + 6 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_aDD12 = sh[c0 + 2560];
+  double V0_aDD12 = sh[c0 + 1024];
   BHAH_PIN(V0_aDD12);
-  V0_lin_aDD12 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_aDD12 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_aDD12);
-  V0_lin_aDD12 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_aDD12 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_aDD12);
   // ---- aDD22
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(5);
   {
     const char *src = (const char *)(in + 7 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_aDD22 = sh[c0 + 5120];
+  double V0_aDD22 = sh[c0 + 2048];
   BHAH_PIN(V0_aDD22);
-  V0_lin_aDD22 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_aDD22 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_aDD22);
-  V0_lin_aDD22 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_aDD22 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_aDD22);
   // ---- alpha
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(6);
   {
     const char *src = (const char *)(in + 8 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_alpha = sh[c0];
   BHAH_PIN(V0_alpha);
@@ -216,40 +216,40 @@ bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *
   V0_lin_alpha += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_alpha);
   // ---- betU0
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(7);
   {
     const char *src = (const char *)(in + 9 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_betU0 = sh[c0 + 2560];
+  double V0_betU0 = sh[c0 + 1024];
   BHAH_PIN(V0_betU0);
-  V0_lin_betU0 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_betU0 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_betU0);
-  V0_lin_betU0 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_betU0 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_betU0);
   // ---- betU1
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(8);
   {
     const char *src = (const char *)(in + 10 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_betU1 = sh[c0 + 5120];
+  double V0_betU1 = sh[c0 + 2048];
   BHAH_PIN(V0_betU1);
-  V0_lin_betU1 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_betU1 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_betU1);
-  V0_lin_betU1 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_betU1 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_betU1);
   // ---- betU2
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(9);
   {
     const char *src = (const char *)(in + 11 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_betU2 = sh[c0];
   BHAH_PIN(V0_betU2);
@@ -258,54 +258,54 @@ bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *
   V0_lin_betU2 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_betU2);
   // ---- cf
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(10);
   {
     const char *src = (const char *)(in + 12 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_cf = sh[c0 + 2560];
+  double V0_cf = sh[c0 + 1024];
   BHAH_PIN(V0_cf);
-  double V0_cf_dD0 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2561] - sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] - sh[c0 + 2558]));
+  double V0_cf_dD0 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 1025] - sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] - sh[c0 + 1022]));
   BHAH_PIN(V0_cf_dD0);
-  double V0_cf_dD1 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2582] - sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] - sh[c0 + 2516]));
+  double V0_cf_dD1 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 1046] - sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] - sh[c0 + 980]));
   BHAH_PIN(V0_cf_dD1);
-  double V0_cf_dDD00 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 2560] + (4.0 / 3.0) * (sh[c0 + 2561] + sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] + sh[c0 + 2558]));
+  double V0_cf_dDD00 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 1024] + (4.0 / 3.0) * (sh[c0 + 1025] + sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] + sh[c0 + 1022]));
   BHAH_PIN(V0_cf_dDD00);
-  double V0_cf_dDD01 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 2583] - sh[c0 + 2539]) - (sh[c0 + 2581] - sh[c0 + 2537])) + (-1.0 / 18.0) * ((sh[c0 + 2605] - sh[c0 + 2517]) - (sh[c0 + 2603] - sh[c0 + 2515])) + (-1.0 / 18.0) * ((sh[c0 + 2584] - sh[c0 + 2540]) - (sh[c0 + 2580] - sh[c0 + 2536])) + (1.0 / 144.0) * ((sh[c0 + 2606] - sh[c0 + 2518]) - (sh[c0 + 2602] - sh[c0 + 2514])));
+  double V0_cf_dDD01 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 1047] - sh[c0 + 1003]) - (sh[c0 + 1045] - sh[c0 + 1001])) + (-1.0 / 18.0) * ((sh[c0 + 1069] - sh[c0 + 981]) - (sh[c0 + 1067] - sh[c0 + 979])) + (-1.0 / 18.0) * ((sh[c0 + 1048] - sh[c0 + 1004]) - (sh[c0 + 1044] - sh[c0 + 1000])) + (1.0 / 144.0) * ((sh[c0 + 1070] - sh[c0 + 982]) - (sh[c0 + 1066] - sh[c0 + 978])));
   BHAH_PIN(V0_cf_dDD01);
-  double V0_cf_dDD11 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 2560] + (4.0 / 3.0) * (sh[c0 + 2582] + sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] + sh[c0 + 2516]));
+  double V0_cf_dDD11 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 1024] + (4.0 / 3.0) * (sh[c0 + 1046] + sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] + sh[c0 + 980]));
   BHAH_PIN(V0_cf_dDD11);
-  V0_lin_cf += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_cf += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_cf);
-  V0_lin_cf += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_cf += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_cf);
   // ---- hDD00
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(11);
   {
     const char *src = (const char *)(in + 13 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_hDD00 = sh[c0 + 5120];
+  double V0_hDD00 = sh[c0 + 2048];
   BHAH_PIN(V0_hDD00);
-  double V0_hDD_dD000 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 5121] - sh[c0 + 5119]) + (-1.0 / 12.0) * (sh[c0 + 5122] - sh[c0 + 5118]));
+  double V0_hDD_dD000 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2049] - sh[c0 + 2047]) + (-1.0 / 12.0) * (sh[c0 + 2050] - sh[c0 + 2046]));
   BHAH_PIN(V0_hDD_dD000);
-  double V0_hDD_dD001 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 5142] - sh[c0 + 5098]) + (-1.0 / 12.0) * (sh[c0 + 5164] - sh[c0 + 5076]));
+  double V0_hDD_dD001 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2070] - sh[c0 + 2026]) + (-1.0 / 12.0) * (sh[c0 + 2092] - sh[c0 + 2004]));
   BHAH_PIN(V0_hDD_dD001);
-  V0_lin_hDD00 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_hDD00 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_hDD00);
-  V0_lin_hDD00 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_hDD00 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_hDD00);
   // ---- hDD01
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(12);
   {
     const char *src = (const char *)(in + 14 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_hDD01 = sh[c0];
   BHAH_PIN(V0_hDD01);
@@ -318,48 +318,48 @@ bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *
   V0_lin_hDD01 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_hDD01);
   // ---- hDD02
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(13);
   {
     const char *src = (const char *)(in + 15 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_hDD02 = sh[c0 + 2560];
+  double V0_hDD02 = sh[c0 + 1024];
   BHAH_PIN(V0_hDD02);
-  double V0_hDD_dD020 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2561] - sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] - sh[c0 + 2558]));
+  double V0_hDD_dD020 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 1025] - sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] - sh[c0 + 1022]));
   BHAH_PIN(V0_hDD_dD020);
-  double V0_hDD_dD021 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2582] - sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] - sh[c0 + 2516]));
+  double V0_hDD_dD021 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 1046] - sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] - sh[c0 + 980]));
   BHAH_PIN(V0_hDD_dD021);
-  V0_lin_hDD02 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_hDD02 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_hDD02);
-  V0_lin_hDD02 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_hDD02 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_hDD02);
   // ---- hDD11
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(14);
   {
     const char *src = (const char *)(in + 16 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_hDD11 = sh[c0 + 5120];
+  double V0_hDD11 = sh[c0 + 2048];
   BHAH_PIN(V0_hDD11);
-  double V0_hDD_dD110 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 5121] - sh[c0 + 5119]) + (-1.0 / 12.0) * (sh[c0 + 5122] - sh[c0 + 5118]));
+  double V0_hDD_dD110 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2049] - sh[c0 + 2047]) + (-1.0 / 12.0) * (sh[c0 + 2050] - sh[c0 + 2046]));
   BHAH_PIN(V0_hDD_dD110);
-  double V0_hDD_dD111 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 5142] - sh[c0 + 5098]) + (-1.0 / 12.0) * (sh[c0 + 5164] - sh[c0 + 5076]));
+  double V0_hDD_dD111 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2070] - sh[c0 + 2026]) + (-1.0 / 12.0) * (sh[c0 + 2092] - sh[c0 + 2004]));
   BHAH_PIN(V0_hDD_dD111);
-  V0_lin_hDD11 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_hDD11 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_hDD11);
-  V0_lin_hDD11 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_hDD11 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_hDD11);
   // ---- hDD12
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(15);
   {
     const char *src = (const char *)(in + 17 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_hDD12 = sh[c0];
   BHAH_PIN(V0_hDD12);
@@ -372,44 +372,44 @@ bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *
   V0_lin_hDD12 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_hDD12);
   // ---- hDD22
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(16);
   {
     const char *src = (const char *)(in + 18 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_hDD22 = sh[c0 + 2560];
+  double V0_hDD22 = sh[c0 + 1024];
   BHAH_PIN(V0_hDD22);
-  double V0_hDD_dD220 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2561] - sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] - sh[c0 + 2558]));
+  double V0_hDD_dD220 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 1025] - sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] - sh[c0 + 1022]));
   BHAH_PIN(V0_hDD_dD220);
-  double V0_hDD_dD221 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2582] - sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] - sh[c0 + 2516]));
+  double V0_hDD_dD221 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 1046] - sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] - sh[c0 + 980]));
   BHAH_PIN(V0_hDD_dD221);
-  V0_lin_hDD22 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_hDD22 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_hDD22);
-  V0_lin_hDD22 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_hDD22 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_hDD22);
   // ---- lambdaU0
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(17);
   {
     const char *src = (const char *)(in + 19 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_lambdaU0 = sh[c0 + 5120];
+  double V0_lambdaU0 = sh[c0 + 2048];
   BHAH_PIN(V0_lambdaU0);
-  V0_lin_lambdaU0 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_lambdaU0 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_lambdaU0);
-  V0_lin_lambdaU0 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_lambdaU0 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_lambdaU0);
   // ---- lambdaU1
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(18);
   {
     const char *src = (const char *)(in + 20 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_lambdaU1 = sh[c0];
   BHAH_PIN(V0_lambdaU1);
@@ -418,44 +418,44 @@ bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *
   V0_lin_lambdaU1 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_lambdaU1);
   // ---- lambdaU2
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(19);
   {
     const char *src = (const char *)(in + 21 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_lambdaU2 = sh[c0 + 2560];
+  double V0_lambdaU2 = sh[c0 + 1024];
   BHAH_PIN(V0_lambdaU2);
-  V0_lin_lambdaU2 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_lambdaU2 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_lambdaU2);
-  V0_lin_lambdaU2 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_lambdaU2 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_lambdaU2);
   // ---- trK
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(20);
   {
     const char *src = (const char *)(in + 22 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_trK = sh[c0 + 5120];
+  double V0_trK = sh[c0 + 2048];
   BHAH_PIN(V0_trK);
-  double V0_trK_dD0 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 5121] - sh[c0 + 5119]) + (-1.0 / 12.0) * (sh[c0 + 5122] - sh[c0 + 5118]));
+  double V0_trK_dD0 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2049] - sh[c0 + 2047]) + (-1.0 / 12.0) * (sh[c0 + 2050] - sh[c0 + 2046]));
   BHAH_PIN(V0_trK_dD0);
-  double V0_trK_dD1 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 5142] - sh[c0 + 5098]) + (-1.0 / 12.0) * (sh[c0 + 5164] - sh[c0 + 5076]));
+  double V0_trK_dD1 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2070] - sh[c0 + 2026]) + (-1.0 / 12.0) * (sh[c0 + 2092] - sh[c0 + 2004]));
   BHAH_PIN(V0_trK_dD1);
-  V0_lin_trK += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_trK += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_trK);
-  V0_lin_trK += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_trK += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_trK);
   // ---- vetU0
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(21);
   {
     const char *src = (const char *)(in + 23 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_vetU0 = sh[c0];
   BHAH_PIN(V0_vetU0);
@@ -474,42 +474,42 @@ bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *
   V0_lin_vetU0 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_vetU0);
   // ---- vetU1
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(22);
-  double V0_vetU1 = sh[c0 + 2560];
+  double V0_vetU1 = sh[c0 + 1024];
   BHAH_PIN(V0_vetU1);
-  double V0_vetU_dD10 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2561] - sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] - sh[c0 + 2558]));
+  double V0_vetU_dD10 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 1025] - sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] - sh[c0 + 1022]));
   BHAH_PIN(V0_vetU_dD10);
-  double V0_vetU_dD11 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2582] - sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] - sh[c0 + 2516]));
+  double V0_vetU_dD11 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 1046] - sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] - sh[c0 + 980]));
   BHAH_PIN(V0_vetU_dD11);
-  double V0_vetU_dDD100 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 2560] + (4.0 / 3.0) * (sh[c0 + 2561] + sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] + sh[c0 + 2558]));
+  double V0_vetU_dDD100 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 1024] + (4.0 / 3.0) * (sh[c0 + 1025] + sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] + sh[c0 + 1022]));
   BHAH_PIN(V0_vetU_dDD100);
-  double V0_vetU_dDD101 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 2583] - sh[c0 + 2539]) - (sh[c0 + 2581] - sh[c0 + 2537])) + (-1.0 / 18.0) * ((sh[c0 + 2605] - sh[c0 + 2517]) - (sh[c0 + 2603] - sh[c0 + 2515])) + (-1.0 / 18.0) * ((sh[c0 + 2584] - sh[c0 + 2540]) - (sh[c0 + 2580] - sh[c0 + 2536])) + (1.0 / 144.0) * ((sh[c0 + 2606] - sh[c0 + 2518]) - (sh[c0 + 2602] - sh[c0 + 2514])));
+  double V0_vetU_dDD101 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 1047] - sh[c0 + 1003]) - (sh[c0 + 1045] - sh[c0 + 1001])) + (-1.0 / 18.0) * ((sh[c0 + 1069] - sh[c0 + 981]) - (sh[c0 + 1067] - sh[c0 + 979])) + (-1.0 / 18.0) * ((sh[c0 + 1048] - sh[c0 + 1004]) - (sh[c0 + 1044] - sh[c0 + 1000])) + (1.0 / 144.0) * ((sh[c0 + 1070] - sh[c0 + 982]) - (sh[c0 + 1066] - sh[c0 + 978])));
   BHAH_PIN(V0_vetU_dDD101);
-  double V0_vetU_dDD111 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 2560] + (4.0 / 3.0) * (sh[c0 + 2582] + sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] + sh[c0 + 2516]));
+  double V0_vetU_dDD111 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 1024] + (4.0 / 3.0) * (sh[c0 + 1046] + sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] + sh[c0 + 980]));
   BHAH_PIN(V0_vetU_dDD111);
-  V0_lin_vetU1 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_vetU1 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_vetU1);
-  V0_lin_vetU1 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_vetU1 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_vetU1);
   // ---- vetU2
   BHAH_VMWAIT(0);
   BHAH_BARRIER_PHASE(23);
-  double V0_vetU2 = sh[c0 + 5120];
+  double V0_vetU2 = sh[c0 + 2048];
   BHAH_PIN(V0_vetU2);
-  double V0_vetU_dD20 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 5121] - sh[c0 + 5119]) + (-1.0 / 12.0) * (sh[c0 + 5122] - sh[c0 + 5118]));
+  double V0_vetU_dD20 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2049] - sh[c0 + 2047]) + (-1.0 / 12.0) * (sh[c0 + 2050] - sh[c0 + 2046]));
   BHAH_PIN(V0_vetU_dD20);
-  double V0_vetU_dD21 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 5142] - sh[c0 + 5098]) + (-1.0 / 12.0) * (sh[c0 + 5164] - sh[c0 + 5076]));
+  double V0_vetU_dD21 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2070] - sh[c0 + 2026]) + (-1.0 / 12.0) * (sh[c0 + 2092] - sh[c0 + 2004]));
   BHAH_PIN(V0_vetU_dD21);
-  double V0_vetU_dDD200 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 5120] + (4.0 / 3.0) * (sh[c0 + 5121] + sh[c0 + 5119]) + (-1.0 / 12.0) * (sh[c0 + 5122] + sh[c0 + 5118]));
+  double V0_vetU_dDD200 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 2048] + (4.0 / 3.0) * (sh[c0 + 2049] + sh[c0 + 2047]) + (-1.0 / 12.0) * (sh[c0 + 2050] + sh[c0 + 2046]));
   BHAH_PIN(V0_vetU_dDD200);
-  double V0_vetU_dDD201 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 5143] - sh[c0 + 5099]) - (sh[c0 + 5141] - sh[c0 + 5097])) + (-1.0 / 18.0) * ((sh[c0 + 5165] - sh[c0 + 5077]) - (sh[c0 + 5163] - sh[c0 + 5075])) + (-1.0 / 18.0) * ((sh[c0 + 5144] - sh[c0 + 5100]) - (sh[c0 + 5140] - sh[c0 + 5096])) + (1.0 / 144.0) * ((sh[c0 + 5166] - sh[c0 + 5078]) - (sh[c0 + 5162] - sh[c0 + 5074])));
+  double V0_vetU_dDD201 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 2071] - sh[c0 + 2027]) - (sh[c0 + 2069] - sh[c0 + 2025])) + (-1.0 / 18.0) * ((sh[c0 + 2093] - sh[c0 + 2005]) - (sh[c0 + 2091] - sh[c0 + 2003])) + (-1.0 / 18.0) * ((sh[c0 + 2072] - sh[c0 + 2028]) - (sh[c0 + 2068] - sh[c0 + 2024])) + (1.0 / 144.0) * ((sh[c0 + 2094] - sh[c0 + 2006]) - (sh[c0 + 2090] - sh[c0 + 2002])));
   BHAH_PIN(V0_vetU_dDD201);
-  double V0_vetU_dDD211 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 5120] + (4.0 / 3.0) * (sh[c0 + 5142] + sh[c0 + 5098]) + (-1.0 / 12.0) * (sh[c0 + 5164] + sh[c0 + 5076]));
+  double V0_vetU_dDD211 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 2048] + (4.0 / 3.0) * (sh[c0 + 2070] + sh[c0 + 2026]) + (-1.0 / 12.0) * (sh[c0 + 2092] + sh[c0 + 2004]));
   BHAH_PIN(V0_vetU_dDD211);
-  V0_lin_vetU2 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_vetU2 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_vetU2);
-  V0_lin_vetU2 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_vetU2 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_vetU2);
   {
     const int i0 = o0 + lx, i1 = o1 + ly, i2 = o2 + lz + 0;
@@ -957,22 +957,22 @@ bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const double *
 static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0_tile(const double *__restrict__ in, const double *__restrict__ aux,
         double *__restrict__ out, const double *__restrict__ rfm0, const double *__restrict__ rfm1,
         const bhah_kparams p, const unsigned bx, const unsigned by, const unsigned bz, double *sh) {
-  // Tile of 16x8x2 interior points; halo box 22x14x8 = 2464 values per gridfunction.
-  constexpr int BX = 22, BY = 14, NB = 2464, NT = 256, NL = 10;
+  // Tile of 16x8x2 interior points; halo box 22x14x2 = 616 values per gridfunction.
+  constexpr int BX = 22, BY = 14, NB = 616, NT = 256, NL = 3;
   const int tid = (int)threadIdx.x;
   const int lx = tid % 16, ly = (tid / 16) % 8, lz = tid / 128;
   const long s1 = p.s1, s2 = p.s2, Ntot = p.Ntot;
   const int o0 = p.NG + (int)bx * 16, o1 = p.NG + (int)by * 8, o2 = p.NG + (int)bz * 2;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  unsigned pofs[5];
+  unsigned pofs[2];
 #pragma unroll
-  for (int j = 0; j < 5; j++) {
+  for (int j = 0; j < 2; j++) {
     const int e = 2 * (tid + NT * j);
     const int ex = e % BX, ey = (e / BX) % BY, ez = e / (BX * BY);
-    const int g0 = min(o0 - 3 + ex, p.Nx0 - 2), g1 = min(o1 - 3 + ey, p.Nx1 - 1), g2 = min(o2 - 3 + ez, p.Nx2 - 1);
+    const int g0 = min(o0 - 3 + ex, p.Nx0 - 2), g1 = min(o1 - 3 + ey, p.Nx1 - 1), g2 = min(o2 - 0 + ez, p.Nx2 - 1);
     pofs[j] = 8u * (unsigned)(g0 + (int)s1 * g1 + (int)s2 * g2);
   }
-  const int c0 = (lx + 3) + BX * (ly + 3) + BX * BY * (lz + 3);
+  const int c0 = (lx + 3) + BX * (ly + 3) + BX * BY * (lz + 0);
   const double ius0 = p.invdxx0 * (1.0 / 12.0), nius0 = -ius0, ikos0 = p.invdxx0 * (1.0 / 64.0);
   const double ius1 = p.invdxx1 * (1.0 / 12.0), nius1 = -ius1, ikos1 = p.invdxx1 * (1.0 / 64.0);
   const double ius2 = p.invdxx2 * (1.0 / 12.0), nius2 = -ius2, ikos2 = p.invdxx2 * (1.0 / 64.0);
@@ -1018,20 +1018,20 @@ static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj
   {
     const char *src = (const char *)(in + 0 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
   {
     const char *src = (const char *)(in + 1 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
   // ---- aDD00
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(0);
   {
     const char *src = (const char *)(in + 2 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_aDD00 = sh[c0];
   BHAH_PIN(V0_aDD00);
@@ -1040,40 +1040,40 @@ static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj
   V0_lin_aDD00 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_aDD00);
   // ---- aDD01
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(1);
   {
     const char *src = (const char *)(in + 3 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_aDD01 = sh[c0 + 2560];
+  double V0_aDD01 = sh[c0 + 1024];
   BHAH_PIN(V0_aDD01);
-  V0_lin_aDD01 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_aDD01 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_aDD01);
-  V0_lin_aDD01 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_aDD01 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_aDD01);
   // ---- aDD02
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(2);
   {
     const char *src = (const char *)(in + 4 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_aDD02 = sh[c0 + 5120];
+  double V0_aDD02 = sh[c0 + 2048];
   BHAH_PIN(V0_aDD02);
-  V0_lin_aDD02 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_aDD02 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_aDD02);
-  V0_lin_aDD02 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_aDD02 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_aDD02);
   // ---- aDD11
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(3);
   {
     const char *src = (const char *)(in + 5 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_aDD11 = sh[c0];
   BHAH_PIN(V0_aDD11);
@@ -1082,40 +1082,40 @@ static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj
   V0_lin_aDD11 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_aDD11);
   // ---- aDD12
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(4);
   {
     const char *src = (const char *)(in + 6 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_aDD12 = sh[c0 + 2560];
+  double V0_aDD12 = sh[c0 + 1024];
   BHAH_PIN(V0_aDD12);
-  V0_lin_aDD12 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_aDD12 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_aDD12);
-  V0_lin_aDD12 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_aDD12 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_aDD12);
   // ---- aDD22
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(5);
   {
     const char *src = (const char *)(in + 7 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_aDD22 = sh[c0 + 5120];
+  double V0_aDD22 = sh[c0 + 2048];
   BHAH_PIN(V0_aDD22);
-  V0_lin_aDD22 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_aDD22 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_aDD22);
-  V0_lin_aDD22 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_aDD22 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_aDD22);
   // ---- alpha
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(6);
   {
     const char *src = (const char *)(in + 8 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_alpha = sh[c0];
   BHAH_PIN(V0_alpha);
@@ -1134,40 +1134,40 @@ static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj
   V0_lin_alpha += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_alpha);
   // ---- betU0
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(7);
   {
     const char *src = (const char *)(in + 9 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_betU0 = sh[c0 + 2560];
+  double V0_betU0 = sh[c0 + 1024];
   BHAH_PIN(V0_betU0);
-  V0_lin_betU0 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_betU0 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_betU0);
-  V0_lin_betU0 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_betU0 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_betU0);
   // ---- betU1
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(8);
   {
     const char *src = (const char *)(in + 10 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_betU1 = sh[c0 + 5120];
+  double V0_betU1 = sh[c0 + 2048];
   BHAH_PIN(V0_betU1);
-  V0_lin_betU1 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_betU1 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_betU1);
-  V0_lin_betU1 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_betU1 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_betU1);
   // ---- betU2
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(9);
   {
     const char *src = (const char *)(in + 11 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_betU2 = sh[c0];
   BHAH_PIN(V0_betU2);
@@ -1176,54 +1176,54 @@ static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj
   V0_lin_betU2 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_betU2);
   // ---- cf
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(10);
   {
     const char *src = (const char *)(in + 12 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_cf = sh[c0 + 2560];
+  double V0_cf = sh[c0 + 1024];
   BHAH_PIN(V0_cf);
-  double V0_cf_dD0 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2561] - sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] - sh[c0 + 2558]));
+  double V0_cf_dD0 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 1025] - sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] - sh[c0 + 1022]));
   BHAH_PIN(V0_cf_dD0);
-  double V0_cf_dD1 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2582] - sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] - sh[c0 + 2516]));
+  double V0_cf_dD1 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 1046] - sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] - sh[c0 + 980]));
   BHAH_PIN(V0_cf_dD1);
-  double V0_cf_dDD00 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 2560] + (4.0 / 3.0) * (sh[c0 + 2561] + sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] + sh[c0 + 2558]));
+  double V0_cf_dDD00 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 1024] + (4.0 / 3.0) * (sh[c0 + 1025] + sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] + sh[c0 + 1022]));
   BHAH_PIN(V0_cf_dDD00);
-  double V0_cf_dDD01 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 2583] - sh[c0 + 2539]) - (sh[c0 + 2581] - sh[c0 + 2537])) + (-1.0 / 18.0) * ((sh[c0 + 2605] - sh[c0 + 2517]) - (sh[c0 + 2603] - sh[c0 + 2515])) + (-1.0 / 18.0) * ((sh[c0 + 2584] - sh[c0 + 2540]) - (sh[c0 + 2580] - sh[c0 + 2536])) + (1.0 / 144.0) * ((sh[c0 + 2606] - sh[c0 + 2518]) - (sh[c0 + 2602] - sh[c0 + 2514])));
+  double V0_cf_dDD01 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 1047] - sh[c0 + 1003]) - (sh[c0 + 1045] - sh[c0 + 1001])) + (-1.0 / 18.0) * ((sh[c0 + 1069] - sh[c0 + 981]) - (sh[c0 + 1067] - sh[c0 + 979])) + (-1.0 / 18.0) * ((sh[c0 + 1048] - sh[c0 + 1004]) - (sh[c0 + 1044] - sh[c0 + 1000])) + (1.0 / 144.0) * ((sh[c0 + 1070] - sh[c0 + 982]) - (sh[c0 + 1066] - sh[c0 + 978])));
   BHAH_PIN(V0_cf_dDD01);
-  double V0_cf_dDD11 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 2560] + (4.0 / 3.0) * (sh[c0 + 2582] + sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] + sh[c0 + 2516]));
+  double V0_cf_dDD11 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 1024] + (4.0 / 3.0) * (sh[c0 + 1046] + sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] + sh[c0 + 980]));
   BHAH_PIN(V0_cf_dDD11);
-  V0_lin_cf += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_cf += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_cf);
-  V0_lin_cf += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_cf += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_cf);
   // ---- hDD00
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(11);
   {
     const char *src = (const char *)(in + 13 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_hDD00 = sh[c0 + 5120];
+  double V0_hDD00 = sh[c0 + 2048];
   BHAH_PIN(V0_hDD00);
-  double V0_hDD_dD000 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 5121] - sh[c0 + 5119]) + (-1.0 / 12.0) * (sh[c0 + 5122] - sh[c0 + 5118]));
+  double V0_hDD_dD000 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2049] - sh[c0 + 2047]) + (-1.0 / 12.0) * (sh[c0 + 2050] - sh[c0 + 2046]));
   BHAH_PIN(V0_hDD_dD000);
-  double V0_hDD_dD001 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 5142] - sh[c0 + 5098]) + (-1.0 / 12.0) * (sh[c0 + 5164] - sh[c0 + 5076]));
+  double V0_hDD_dD001 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2070] - sh[c0 + 2026]) + (-1.0 / 12.0) * (sh[c0 + 2092] - sh[c0 + 2004]));
   BHAH_PIN(V0_hDD_dD001);
-  V0_lin_hDD00 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_hDD00 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_hDD00);
-  V0_lin_hDD00 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_hDD00 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_hDD00);
   // ---- hDD01
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(12);
   {
     const char *src = (const char *)(in + 14 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_hDD01 = sh[c0];
   BHAH_PIN(V0_hDD01);
@@ -1236,48 +1236,48 @@ static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj
   V0_lin_hDD01 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_hDD01);
   // ---- hDD02
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(13);
   {
     const char *src = (const char *)(in + 15 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_hDD02 = sh[c0 + 2560];
+  double V0_hDD02 = sh[c0 + 1024];
   BHAH_PIN(V0_hDD02);
-  double V0_hDD_dD020 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2561] - sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] - sh[c0 + 2558]));
+  double V0_hDD_dD020 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 1025] - sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] - sh[c0 + 1022]));
   BHAH_PIN(V0_hDD_dD020);
-  double V0_hDD_dD021 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2582] - sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] - sh[c0 + 2516]));
+  double V0_hDD_dD021 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 1046] - sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] - sh[c0 + 980]));
   BHAH_PIN(V0_hDD_dD021);
-  V0_lin_hDD02 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_hDD02 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_hDD02);
-  V0_lin_hDD02 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_hDD02 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_hDD02);
   // ---- hDD11
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(14);
   {
     const char *src = (const char *)(in + 16 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_hDD11 = sh[c0 + 5120];
+  double V0_hDD11 = sh[c0 + 2048];
   BHAH_PIN(V0_hDD11);
-  double V0_hDD_dD110 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 5121] - sh[c0 + 5119]) + (-1.0 / 12.0) * (sh[c0 + 5122] - sh[c0 + 5118]));
+  double V0_hDD_dD110 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2049] - sh[c0 + 2047]) + (-1.0 / 12.0) * (sh[c0 + 2050] - sh[c0 + 2046]));
   BHAH_PIN(V0_hDD_dD110);
-  double V0_hDD_dD111 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 5142] - sh[c0 + 5098]) + (-1.0 / 12.0) * (sh[c0 + 5164] - sh[c0 + 5076]));
+  double V0_hDD_dD111 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2070] - sh[c0 + 2026]) + (-1.0 / 12.0) * (sh[c0 + 2092] - sh[c0 + 2004]));
   BHAH_PIN(V0_hDD_dD111);
-  V0_lin_hDD11 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_hDD11 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_hDD11);
-  V0_lin_hDD11 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_hDD11 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_hDD11);
   // ---- hDD12
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(15);
   {
     const char *src = (const char *)(in + 17 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_hDD12 = sh[c0];
   BHAH_PIN(V0_hDD12);
@@ -1290,44 +1290,44 @@ static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj
   V0_lin_hDD12 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_hDD12);
   // ---- hDD22
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(16);
   {
     const char *src = (const char *)(in + 18 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_hDD22 = sh[c0 + 2560];
+  double V0_hDD22 = sh[c0 + 1024];
   BHAH_PIN(V0_hDD22);
-  double V0_hDD_dD220 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2561] - sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] - sh[c0 + 2558]));
+  double V0_hDD_dD220 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 1025] - sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] - sh[c0 + 1022]));
   BHAH_PIN(V0_hDD_dD220);
-  double V0_hDD_dD221 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2582] - sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] - sh[c0 + 2516]));
+  double V0_hDD_dD221 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 1046] - sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] - sh[c0 + 980]));
   BHAH_PIN(V0_hDD_dD221);
-  V0_lin_hDD22 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_hDD22 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_hDD22);
-  V0_lin_hDD22 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_hDD22 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_hDD22);
   // ---- lambdaU0
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(17);
   {
     const char *src = (const char *)(in + 19 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_lambdaU0 = sh[c0 + 5120];
+  double V0_lambdaU0 = sh[c0 + 2048];
   BHAH_PIN(V0_lambdaU0);
-  V0_lin_lambdaU0 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_lambdaU0 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_lambdaU0);
-  V0_lin_lambdaU0 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_lambdaU0 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_lambdaU0);
   // ---- lambdaU1
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(18);
   {
     const char *src = (const char *)(in + 20 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_lambdaU1 = sh[c0];
   BHAH_PIN(V0_lambdaU1);
@@ -1336,44 +1336,44 @@ static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj
   V0_lin_lambdaU1 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_lambdaU1);
   // ---- lambdaU2
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(19);
   {
     const char *src = (const char *)(in + 21 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 0 + 2 * (NT * j + 64 * wv));
   }
-  double V0_lambdaU2 = sh[c0 + 2560];
+  double V0_lambdaU2 = sh[c0 + 1024];
   BHAH_PIN(V0_lambdaU2);
-  V0_lin_lambdaU2 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_lambdaU2 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_lambdaU2);
-  V0_lin_lambdaU2 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_lambdaU2 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_lambdaU2);
   // ---- trK
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(20);
   {
     const char *src = (const char *)(in + 22 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 2560 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 1024 + 2 * (NT * j + 64 * wv));
   }
-  double V0_trK = sh[c0 + 5120];
+  double V0_trK = sh[c0 + 2048];
   BHAH_PIN(V0_trK);
-  double V0_trK_dD0 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 5121] - sh[c0 + 5119]) + (-1.0 / 12.0) * (sh[c0 + 5122] - sh[c0 + 5118]));
+  double V0_trK_dD0 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2049] - sh[c0 + 2047]) + (-1.0 / 12.0) * (sh[c0 + 2050] - sh[c0 + 2046]));
   BHAH_PIN(V0_trK_dD0);
-  double V0_trK_dD1 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 5142] - sh[c0 + 5098]) + (-1.0 / 12.0) * (sh[c0 + 5164] - sh[c0 + 5076]));
+  double V0_trK_dD1 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2070] - sh[c0 + 2026]) + (-1.0 / 12.0) * (sh[c0 + 2092] - sh[c0 + 2004]));
   BHAH_PIN(V0_trK_dD1);
-  V0_lin_trK += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_trK += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_trK);
-  V0_lin_trK += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_trK += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_trK);
   // ---- vetU0
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(21);
   {
     const char *src = (const char *)(in + 23 * Ntot);
 #pragma unroll
-    for (int j = 0; j < 5; j++) BHAH_DMA16O(src, pofs[j], sh + 5120 + 2 * (NT * j + 64 * wv));
+    for (int j = 0; j < 2; j++) BHAH_DMA16O(src, pofs[j], sh + 2048 + 2 * (NT * j + 64 * wv));
   }
   double V0_vetU0 = sh[c0];
   BHAH_PIN(V0_vetU0);
@@ -1392,42 +1392,42 @@ static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj
   V0_lin_vetU0 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 66] + -6.0 * sh[c0 + 44] + -3.0 * sh[c0 - 22] + 18.0 * sh[c0 + 22] + -10.0 * sh[c0])) : (nius1 * (sh[c0 - 66] + -6.0 * sh[c0 - 44] + 18.0 * sh[c0 - 22] + -3.0 * sh[c0 + 22] + -10.0 * sh[c0])));
   BHAH_PIN(V0_lin_vetU0);
   // ---- vetU1
-  BHAH_VMWAIT(5);
+  BHAH_VMWAIT(2);
   BHAH_BARRIER_PHASE(22);
-  double V0_vetU1 = sh[c0 + 2560];
+  double V0_vetU1 = sh[c0 + 1024];
   BHAH_PIN(V0_vetU1);
-  double V0_vetU_dD10 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2561] - sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] - sh[c0 + 2558]));
+  double V0_vetU_dD10 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 1025] - sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] - sh[c0 + 1022]));
   BHAH_PIN(V0_vetU_dD10);
-  double V0_vetU_dD11 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2582] - sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] - sh[c0 + 2516]));
+  double V0_vetU_dD11 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 1046] - sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] - sh[c0 + 980]));
   BHAH_PIN(V0_vetU_dD11);
-  double V0_vetU_dDD100 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 2560] + (4.0 / 3.0) * (sh[c0 + 2561] + sh[c0 + 2559]) + (-1.0 / 12.0) * (sh[c0 + 2562] + sh[c0 + 2558]));
+  double V0_vetU_dDD100 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 1024] + (4.0 / 3.0) * (sh[c0 + 1025] + sh[c0 + 1023]) + (-1.0 / 12.0) * (sh[c0 + 1026] + sh[c0 + 1022]));
   BHAH_PIN(V0_vetU_dDD100);
-  double V0_vetU_dDD101 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 2583] - sh[c0 + 2539]) - (sh[c0 + 2581] - sh[c0 + 2537])) + (-1.0 / 18.0) * ((sh[c0 + 2605] - sh[c0 + 2517]) - (sh[c0 + 2603] - sh[c0 + 2515])) + (-1.0 / 18.0) * ((sh[c0 + 2584] - sh[c0 + 2540]) - (sh[c0 + 2580] - sh[c0 + 2536])) + (1.0 / 144.0) * ((sh[c0 + 2606] - sh[c0 + 2518]) - (sh[c0 + 2602] - sh[c0 + 2514])));
+  double V0_vetU_dDD101 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 1047] - sh[c0 + 1003]) - (sh[c0 + 1045] - sh[c0 + 1001])) + (-1.0 / 18.0) * ((sh[c0 + 1069] - sh[c0 + 981]) - (sh[c0 + 1067] - sh[c0 + 979])) + (-1.0 / 18.0) * ((sh[c0 + 1048] - sh[c0 + 1004]) - (sh[c0 + 1044] - sh[c0 + 1000])) + (1.0 / 144.0) * ((sh[c0 + 1070] - sh[c0 + 982]) - (sh[c0 + 1066] - sh[c0 + 978])));
   BHAH_PIN(V0_vetU_dDD101);
-  double V0_vetU_dDD111 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 2560] + (4.0 / 3.0) * (sh[c0 + 2582] + sh[c0 + 2538]) + (-1.0 / 12.0) * (sh[c0 + 2604] + sh[c0 + 2516]));
+  double V0_vetU_dDD111 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 1024] + (4.0 / 3.0) * (sh[c0 + 1046] + sh[c0 + 1002]) + (-1.0 / 12.0) * (sh[c0 + 1068] + sh[c0 + 980]));
   BHAH_PIN(V0_vetU_dDD111);
-  V0_lin_vetU1 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2563] + -6.0 * sh[c0 + 2562] + -3.0 * sh[c0 + 2559] + 18.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])) : (nius0 * (sh[c0 + 2557] + -6.0 * sh[c0 + 2558] + 18.0 * sh[c0 + 2559] + -3.0 * sh[c0 + 2561] + -10.0 * sh[c0 + 2560])));
+  V0_lin_vetU1 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 1027] + -6.0 * sh[c0 + 1026] + -3.0 * sh[c0 + 1023] + 18.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])) : (nius0 * (sh[c0 + 1021] + -6.0 * sh[c0 + 1022] + 18.0 * sh[c0 + 1023] + -3.0 * sh[c0 + 1025] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_vetU1);
-  V0_lin_vetU1 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2626] + -6.0 * sh[c0 + 2604] + -3.0 * sh[c0 + 2538] + 18.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])) : (nius1 * (sh[c0 + 2494] + -6.0 * sh[c0 + 2516] + 18.0 * sh[c0 + 2538] + -3.0 * sh[c0 + 2582] + -10.0 * sh[c0 + 2560])));
+  V0_lin_vetU1 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 1090] + -6.0 * sh[c0 + 1068] + -3.0 * sh[c0 + 1002] + 18.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])) : (nius1 * (sh[c0 + 958] + -6.0 * sh[c0 + 980] + 18.0 * sh[c0 + 1002] + -3.0 * sh[c0 + 1046] + -10.0 * sh[c0 + 1024])));
   BHAH_PIN(V0_lin_vetU1);
   // ---- vetU2
   BHAH_VMWAIT(0);
   BHAH_BARRIER_PHASE(23);
-  double V0_vetU2 = sh[c0 + 5120];
+  double V0_vetU2 = sh[c0 + 2048];
   BHAH_PIN(V0_vetU2);
-  double V0_vetU_dD20 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 5121] - sh[c0 + 5119]) + (-1.0 / 12.0) * (sh[c0 + 5122] - sh[c0 + 5118]));
+  double V0_vetU_dD20 = p.invdxx0 * ((2.0 / 3.0) * (sh[c0 + 2049] - sh[c0 + 2047]) + (-1.0 / 12.0) * (sh[c0 + 2050] - sh[c0 + 2046]));
   BHAH_PIN(V0_vetU_dD20);
-  double V0_vetU_dD21 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 5142] - sh[c0 + 5098]) + (-1.0 / 12.0) * (sh[c0 + 5164] - sh[c0 + 5076]));
+  double V0_vetU_dD21 = p.invdxx1 * ((2.0 / 3.0) * (sh[c0 + 2070] - sh[c0 + 2026]) + (-1.0 / 12.0) * (sh[c0 + 2092] - sh[c0 + 2004]));
   BHAH_PIN(V0_vetU_dD21);
-  double V0_vetU_dDD200 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 5120] + (4.0 / 3.0) * (sh[c0 + 5121] + sh[c0 + 5119]) + (-1.0 / 12.0) * (sh[c0 + 5122] + sh[c0 + 5118]));
+  double V0_vetU_dDD200 = p.invdxx0 * p.invdxx0 * ((-5.0 / 2.0) * sh[c0 + 2048] + (4.0 / 3.0) * (sh[c0 + 2049] + sh[c0 + 2047]) + (-1.0 / 12.0) * (sh[c0 + 2050] + sh[c0 + 2046]));
   BHAH_PIN(V0_vetU_dDD200);
-  double V0_vetU_dDD201 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 5143] - sh[c0 + 5099]) - (sh[c0 + 5141] - sh[c0 + 5097])) + (-1.0 / 18.0) * ((sh[c0 + 5165] - sh[c0 + 5077]) - (sh[c0 + 5163] - sh[c0 + 5075])) + (-1.0 / 18.0) * ((sh[c0 + 5144] - sh[c0 + 5100]) - (sh[c0 + 5140] - sh[c0 + 5096])) + (1.0 / 144.0) * ((sh[c0 + 5166] - sh[c0 + 5078]) - (sh[c0 + 5162] - sh[c0 + 5074])));
+  double V0_vetU_dDD201 = p.invdxx0 * p.invdxx1 * ((4.0 / 9.0) * ((sh[c0 + 2071] - sh[c0 + 2027]) - (sh[c0 + 2069] - sh[c0 + 2025])) + (-1.0 / 18.0) * ((sh[c0 + 2093] - sh[c0 + 2005]) - (sh[c0 + 2091] - sh[c0 + 2003])) + (-1.0 / 18.0) * ((sh[c0 + 2072] - sh[c0 + 2028]) - (sh[c0 + 2068] - sh[c0 + 2024])) + (1.0 / 144.0) * ((sh[c0 + 2094] - sh[c0 + 2006]) - (sh[c0 + 2090] - sh[c0 + 2002])));
   BHAH_PIN(V0_vetU_dDD201);
-  double V0_vetU_dDD211 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 5120] + (4.0 / 3.0) * (sh[c0 + 5142] + sh[c0 + 5098]) + (-1.0 / 12.0) * (sh[c0 + 5164] + sh[c0 + 5076]));
+  double V0_vetU_dDD211 = p.invdxx1 * p.invdxx1 * ((-5.0 / 2.0) * sh[c0 + 2048] + (4.0 / 3.0) * (sh[c0 + 2070] + sh[c0 + 2026]) + (-1.0 / 12.0) * (sh[c0 + 2092] + sh[c0 + 2004]));
   BHAH_PIN(V0_vetU_dDD211);
-  V0_lin_vetU2 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 5123] + -6.0 * sh[c0 + 5122] + -3.0 * sh[c0 + 5119] + 18.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])) : (nius0 * (sh[c0 + 5117] + -6.0 * sh[c0 + 5118] + 18.0 * sh[c0 + 5119] + -3.0 * sh[c0 + 5121] + -10.0 * sh[c0 + 5120])));
+  V0_lin_vetU2 += L0_coef[0] * ((L0_beta[0] > 0.0) ? (ius0 * (sh[c0 + 2051] + -6.0 * sh[c0 + 2050] + -3.0 * sh[c0 + 2047] + 18.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])) : (nius0 * (sh[c0 + 2045] + -6.0 * sh[c0 + 2046] + 18.0 * sh[c0 + 2047] + -3.0 * sh[c0 + 2049] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_vetU2);
-  V0_lin_vetU2 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 5186] + -6.0 * sh[c0 + 5164] + -3.0 * sh[c0 + 5098] + 18.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])) : (nius1 * (sh[c0 + 5054] + -6.0 * sh[c0 + 5076] + 18.0 * sh[c0 + 5098] + -3.0 * sh[c0 + 5142] + -10.0 * sh[c0 + 5120])));
+  V0_lin_vetU2 += L0_coef[1] * ((L0_beta[1] > 0.0) ? (ius1 * (sh[c0 + 2114] + -6.0 * sh[c0 + 2092] + -3.0 * sh[c0 + 2026] + 18.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])) : (nius1 * (sh[c0 + 1982] + -6.0 * sh[c0 + 2004] + 18.0 * sh[c0 + 2026] + -3.0 * sh[c0 + 2070] + -10.0 * sh[c0 + 2048])));
   BHAH_PIN(V0_lin_vetU2);
   {
     const int i0 = o0 + lx, i1 = o1 + ly, i2 = o2 + lz + 0;
@@ -1874,7 +1874,7 @@ static __device__ __forceinline__ void bssn_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj
 extern "C" __global__ void __launch_bounds__(256)
 bssn_ens_rhs_Spherical_sym2_KO0_fd4_p1_lb1_sj_L16x8x2x1_d3_dma_rb1_g0(const bhah_member *__restrict__ mem, const bhah_item *__restrict__ items, const int nitems,
         const int in_sel, const int aux_sel, const int out_sel) {
-  __shared__ double sh[7680];
+  __shared__ double sh[3072];
   for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
     const bhah_item w = items[it];
     const bhah_member *M = &mem[w.m];
