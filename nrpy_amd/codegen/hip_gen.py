@@ -838,17 +838,17 @@ def _upwind_prologue(spec: specs.Spec, fd_order: int, rationals, tables: bool = 
     return "\n".join(lines)
 
 
-def detgamma_inline(v: specs.Variant, rationals, src: str) -> str:
+def detgamma_inline(v: specs.Variant, rationals, src: str, first: int = 0) -> str:
     """Inline det(gammabar) enforcement on hDD values held in ``nxt[]``.
 
-    ``src`` names the array of 24 next-stage values (EVOL order).
+    ``src`` names the array of next-stage values (EVOL order from gridfunction ``first`` on).
     """
     spec = specs.detgamma_spec(v)
     pr = emit.DoublePrinter(rationals)
     centre, _, _, rfm, _ = spec.classify()
     lines = ["  {"]
     for n in centre:
-        lines.append(f"    const double {n} = {src}[{bssn.EVOL_GFS.index(n)}];")
+        lines.append(f"    const double {n} = {src}[{bssn.EVOL_GFS.index(n) - first}];")
     for n in rfm:
         lines.append(f"    const double {n} = {RFM_EXPR[specs.RFM_SYMBOLS.index(n)]};")
     replaced, reduced = sp.cse([e for _, e in spec.outputs], symbols=sp.numbered_symbols("dg"), order="none")
@@ -859,7 +859,7 @@ def detgamma_inline(v: specs.Variant, rationals, src: str) -> str:
         lines.append(f"    const double new_{gf} = {pr.doprint(e)};")
         outs.append(gf)
     for gf in outs:
-        lines.append(f"    {src}[{bssn.EVOL_GFS.index(gf)}] = new_{gf};")
+        lines.append(f"    {src}[{bssn.EVOL_GFS.index(gf) - first}] = new_{gf};")
     lines.append("  }")
     return "\n".join(lines)
 
@@ -1754,6 +1754,293 @@ extern "C" hipError_t launch_bssn_ens_{kind}_{tag}_{cand}({ENS_SIG}) {{
     return head + consts + "\n" + "".join(kernels) + "".join(ens_kernels) + undefs + "\n" + launcher, total
 
 
+# The RK4 substep update with det(gammabar) enforcement of the next stage, over all points in
+# array order.  Bound by memory traffic (768-960 B per point).  Work is split into four groups of
+# six gridfunctions (hDD, which det enforcement couples, and three of the others), a workgroup per
+# (chunk of points, group): four times the workgroups of a thread that owns all 24, which a
+# small grid needs to fill the chip, and a quarter of the registers, so more loads are in
+# flight per CU.  NP points per thread: 2 with 16-byte loads and stores (even Ntot, 16-byte
+# aligned arrays), else 1.
+#
+# INNER: the pass takes the inner-parity boundary condition of the right-hand side with it
+# (apply_bcs_inner_only__openmp.c:3-57).  At an inner ghost point k is the value at the point's
+# source with the parity sign, and so is every earlier k and their running sum: the running sum
+# of an inner ghost point is not kept, its source's is read in the last stage (which only reads
+# it).  kin is only read by this pass.  The maps (bhah_patch::d_inner_map, d_inner_pairs in
+# bhah_hip.hip) name the sources; a pair of points whose sources lie in one aligned pair (every
+# pair of a four-ghost-zone grid with even rows) takes them with one 16-byte load a gridfunction,
+# any other pair with two 8-byte loads.
+#
+# Against one thread for all 24 gridfunctions and a separate inner copy where the pairs' sources are
+# apart, per substep in whole steps: 4.9 us against 19.5 + 5.6 at 72x12x2, 18.8 against 46.5 at
+# 64x32x32 fd6, 216 against 297 + 75 for a 64-member ensemble (63% of its points are inner ghosts),
+# 365 against 387 at 192x96x96 fd6 (1.9 GB: 5.1 TB/s).
+RK_PASS = r"""
+typedef double bhah_d2 __attribute__((ext_vector_type(2)));
+namespace rk_@TAG@ {
+constexpr int PAR[24] = {@PAR@};
+// gridfunction j of group G
+constexpr __host__ __device__ int gf(int G, int j) {
+  return G == 0 ? 11 + j : G == 1 ? j : G == 2 ? (j < 5 ? 6 + j : 17) : 18 + j;
+}
+// NP consecutive values; NT: with the non-temporal hint
+template <int NP>
+struct Vec;
+template <>
+struct Vec<1> {
+  double v[1];
+  template <bool NT>
+  static __device__ __forceinline__ Vec ld(const double *q) {
+    return {{NT ? __builtin_nontemporal_load(q) : *q}};
+  }
+  template <bool NT>
+  __device__ __forceinline__ void st(double *q) const {
+    if (NT) __builtin_nontemporal_store(v[0], q);
+    else *q = v[0];
+  }
+};
+template <>
+struct Vec<2> {
+  double v[2];
+  template <bool NT>
+  static __device__ __forceinline__ Vec ld(const double *q) {
+    const bhah_d2 t = NT ? __builtin_nontemporal_load((const bhah_d2 *)q) : *(const bhah_d2 *)q;
+    return {{t.x, t.y}};
+  }
+  template <bool NT>
+  __device__ __forceinline__ void st(double *q) const {
+    bhah_d2 t;
+    t.x = v[0];
+    t.y = v[1];
+    if (NT) __builtin_nontemporal_store(t, (bhah_d2 *)q);
+    else *(bhah_d2 *)q = t;
+  }
+};
+// Where this thread's points find the right-hand side: a point or an aligned pair (from, code), or,
+// for a pair whose sources are apart, two points with their parity masks.
+struct Source {
+  long from, s0, s1;
+  unsigned code, m0, m1;
+  bool split, ghost;  // ghost: every point of this thread is an inner ghost point
+};
+template <int NP>
+__device__ __forceinline__ Source find_source(const int2 *map, const int2 *pairs, long q) {
+  Source S;
+  const int2 m = (NP == 2) ? pairs[q] : map[q];
+  S.split = NP == 2 && m.y < 0;
+  S.code = (unsigned)m.y;
+  S.from = (long)m.x * NP;
+  S.s0 = S.s1 = 0;
+  S.m0 = S.m1 = 0;
+  S.ghost = S.from != q * NP;
+  if (S.split) {
+    const int4 t = ((const int4 *)map)[q];
+    S.s0 = t.x;
+    S.m0 = (unsigned)t.y;
+    S.s1 = t.z;
+    S.m1 = (unsigned)t.w;
+    S.ghost = S.s0 != 2 * q && S.s1 != 2 * q + 1;
+  }
+  return S;
+}
+// The six gridfunctions of group G of f at this thread's sources, with their parity signs.
+template <int G, int NP, bool NT>
+__device__ __forceinline__ void at_source(Vec<NP> (&r)[6], const double *f, const long Ntot, const Source &S) {
+  if (NP == 2 && S.split) {
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+      r[j].v[0] = f[gf(G, j) * Ntot + S.s0];
+      r[j].v[NP - 1] = f[gf(G, j) * Ntot + S.s1];
+    }
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+      r[j].v[0] = ((S.m0 >> PAR[gf(G, j)]) & 1u) ? -r[j].v[0] : r[j].v[0];
+      r[j].v[NP - 1] = ((S.m1 >> PAR[gf(G, j)]) & 1u) ? -r[j].v[NP - 1] : r[j].v[NP - 1];
+    }
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 6; j++) r[j] = Vec<NP>::template ld<NT>(f + gf(G, j) * Ntot + S.from);
+#pragma unroll
+  for (int j = 0; j < 6; j++) {
+    const int t = PAR[gf(G, j)];
+    if (NP == 1) {
+      r[j].v[0] = ((S.code >> t) & 1u) ? -r[j].v[0] : r[j].v[0];
+    } else {
+      const double a = (S.code & 1u) ? r[j].v[NP - 1] : r[j].v[0], b = (S.code & 2u) ? r[j].v[NP - 1] : r[j].v[0];
+      r[j].v[0] = ((S.code >> (4 + t)) & 1u) ? -a : a;
+      r[j].v[NP - 1] = ((S.code >> (16 + t)) & 1u) ? -b : b;
+    }
+  }
+}
+template <int G, int NP, bool INNER, bool NT>
+__device__ __forceinline__ void group(const double *__restrict__ kin, const double *y_n, double *y_run, double *out,
+                                      const double *__restrict__ rfm0, const double *__restrict__ rfm1,
+                                      const bhah_kparams &p, const int2 *__restrict__ map,
+                                      const int2 *__restrict__ pairs, const long q) {
+  const long Ntot = p.Ntot, idx = q * NP;
+  constexpr int N = 6;
+  const double dt = p.dt;
+  Vec<NP> k[N], y[N], r[N];
+  Source S;
+  S.ghost = false;
+  if (INNER) {
+    S = find_source<NP>(map, pairs, q);
+    at_source<G, NP, NT>(k, kin, Ntot, S);
+  } else {
+#pragma unroll
+    for (int j = 0; j < N; j++) k[j] = Vec<NP>::template ld<NT>(kin + gf(G, j) * Ntot + idx);
+  }
+  const bool ghost = S.ghost;
+#pragma unroll
+  for (int j = 0; j < N; j++) y[j] = Vec<NP>::template ld<NT>(y_n + gf(G, j) * Ntot + idx);
+  // RK4 substep update (register_all_MoL_step_forward_in_time.c:4-103), in registers.
+  if (p.substep == 4) {
+    if (INNER && ghost) {
+      at_source<G, NP, true>(r, y_run, Ntot, S);
+    } else {
+#pragma unroll
+      for (int j = 0; j < N; j++) r[j] = Vec<NP>::template ld<true>(y_run + gf(G, j) * Ntot + idx);
+    }
+#pragma unroll
+    for (int j = 0; j < N; j++)
+#pragma unroll
+      for (int e = 0; e < NP; e++) y[j].v[e] = (1.0 / 6.0) * dt * k[j].v[e] + y[j].v[e] + r[j].v[e];
+  } else {
+    if (!ghost) {
+      if (p.substep == 1) {
+#pragma unroll
+        for (int j = 0; j < N; j++)
+#pragma unroll
+          for (int e = 0; e < NP; e++) r[j].v[e] = (1.0 / 6.0) * dt * k[j].v[e];
+      } else {
+#pragma unroll
+        for (int j = 0; j < N; j++) r[j] = Vec<NP>::template ld<true>(y_run + gf(G, j) * Ntot + idx);
+#pragma unroll
+        for (int j = 0; j < N; j++)
+#pragma unroll
+          for (int e = 0; e < NP; e++) r[j].v[e] = (1.0 / 3.0) * dt * k[j].v[e] + r[j].v[e];
+      }
+#pragma unroll
+      for (int j = 0; j < N; j++) r[j].template st<true>(y_run + gf(G, j) * Ntot + idx);
+    }
+    const double a = (p.substep == 3) ? 1.0 : (1.0 / 2.0);
+#pragma unroll
+    for (int j = 0; j < N; j++)
+#pragma unroll
+      for (int e = 0; e < NP; e++) y[j].v[e] = a * dt * k[j].v[e] + y[j].v[e];
+  }
+  if (G == 0) {
+#pragma unroll
+    for (int e = 0; e < NP; e++) {
+      const unsigned long u = (unsigned long)(idx + e), row = u / (unsigned)p.Nx0;
+      const int i0 = (int)(u - row * (unsigned)p.Nx0), i1 = (int)(row % (unsigned)p.Nx1);
+      double nxt[N];
+#pragma unroll
+      for (int j = 0; j < N; j++) nxt[j] = y[j].v[e];
+@DET@
+#pragma unroll
+      for (int j = 0; j < N; j++) y[j].v[e] = nxt[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < N; j++) y[j].template st<NT>(out + gf(G, j) * Ntot + idx);
+}
+template <int NP, bool INNER, bool NT>
+__device__ __forceinline__ void any_group(int G, const double *__restrict__ kin, const double *y_n, double *y_run,
+                                          double *out, const double *__restrict__ rfm0,
+                                          const double *__restrict__ rfm1, const bhah_kparams &p,
+                                          const int2 *__restrict__ map, const int2 *__restrict__ pairs,
+                                          const long q) {
+  if (q * NP >= p.Ntot) return;
+  if (G == 0) group<0, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+  else if (G == 1) group<1, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+  else if (G == 2) group<2, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+  else group<3, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+}
+}  // namespace rk_@TAG@
+template <int NP, bool INNER, bool NT>
+__global__ void __launch_bounds__(256)
+bssn_rk_det_@TAG@(const double *__restrict__ kin, const double *y_n, double *y_run, double *out,
+                  const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p,
+                  const int2 *__restrict__ map, const int2 *__restrict__ pairs) {
+  rk_@TAG@::any_group<NP, INNER, NT>((int)(blockIdx.x & 3u), kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs,
+                                 (long)(blockIdx.x >> 2) * blockDim.x + threadIdx.x);
+}
+"""
+RK_PASS_LAUNCH = r"""
+static hipError_t rk_det_launch_@TAG@(hipStream_t s, const double *kin, const double *y_n, double *y_run, double *out,
+    const double *rfm0, const double *rfm1, const bhah_kparams &p, const int2 *map, const int2 *pairs) {
+  const int np = (!(p.Ntot & 1) && !((reinterpret_cast<uintptr_t>(kin) | reinterpret_cast<uintptr_t>(y_n) |
+                                      reinterpret_cast<uintptr_t>(y_run) | reinterpret_cast<uintptr_t>(out)) & 15))
+                     ? 2
+                     : 1;
+  const long units = p.Ntot / np;
+  // 256 threads a workgroup where that gives every CU several; 64 on small grids
+  const unsigned nt = units >= (1L << 17) ? 256 : 64;
+  const dim3 g(4u * (unsigned)((units + nt - 1) / nt));
+  // The running sum is not read again before the next substep, so it always streams past the
+  // caches.  The other arrays (five stage arrays in all) are read by the next kernels: caching
+  // them gains where a good part of them stays in the 256 MB last-level cache (7229 -> 6947 us
+  // per four steps at 127x63x62 fd6, 0.64 GB; 2297 -> 2003 at 256x64x16, 0.39 GB; 6958 -> 6925
+  // for an ensemble of 1.5 GB) and loses where none does (23493 -> 23839 at 192x96x96, 2.1 GB).
+  const bool nt_all = p.Ntot * (5 * 24 * 8L) > 1800000000L;
+#define RK_LAUNCH(NP_, IN_, NT_)                                                                                     \
+  if (np == NP_ && (map != nullptr) == IN_ && nt_all == NT_)                                                         \
+    hipLaunchKernelGGL((bssn_rk_det_@TAG@<NP_, IN_, NT_>), g, dim3(nt), 0, s, kin, y_n, y_run, out, rfm0, rfm1, p,   \
+                       map, pairs)
+  RK_LAUNCH(1, false, false);
+  RK_LAUNCH(1, false, true);
+  RK_LAUNCH(1, true, false);
+  RK_LAUNCH(1, true, true);
+  RK_LAUNCH(2, false, false);
+  RK_LAUNCH(2, false, true);
+  RK_LAUNCH(2, true, false);
+  RK_LAUNCH(2, true, true);
+#undef RK_LAUNCH
+  return hipGetLastError();
+}
+extern "C" hipError_t launch_bssn_rk_det_@TAG@(hipStream_t s, const double *kin, const double *y_n, double *y_run,
+    double *out, const double *rfm0, const double *rfm1, bhah_kparams p) {
+  return rk_det_launch_@TAG@(s, kin, y_n, y_run, out, rfm0, rfm1, p, nullptr, nullptr);
+}
+// The RK pass with the inner boundary condition folded in.
+extern "C" hipError_t launch_bssn_rk_det_inner_@TAG@(hipStream_t s, const double *kin, const double *y_n,
+    double *y_run, double *out, const double *rfm0, const double *rfm1, bhah_kparams p, const int *map,
+    const int *pairs) {
+  return rk_det_launch_@TAG@(s, kin, y_n, y_run, out, rfm0, rfm1, p, reinterpret_cast<const int2 *>(map),
+                             reinterpret_cast<const int2 *>(pairs));
+}
+"""
+RK_PASS_ENSEMBLE = r"""
+// Records are (member, chunk): 256 consecutive units of NP points of the member's arrays, in array
+// order; each is walked by four consecutive workgroups, one per group of gridfunctions.
+template <int NP>
+__global__ void __launch_bounds__(256)
+bssn_ens_rk_det_@TAG@(const bhah_member *__restrict__ mem, const bhah_item *__restrict__ items, const int nitems,
+                      const int k_sel, const int out_sel, const int substep) {
+  for (int it = blockIdx.x; it < 4 * nitems; it += gridDim.x) {
+    const bhah_item w = items[it >> 2];
+    const bhah_member *M = &mem[w.m];
+    bhah_kparams p = M->kp;
+    p.substep = substep;
+    rk_@TAG@::any_group<NP, true, false>(it & 3, M->arr[k_sel], M->arr[0], M->arr[1], M->arr[out_sel], M->rfm0, M->rfm1, p,
+                                  reinterpret_cast<const int2 *>(M->inner_map),
+                                  reinterpret_cast<const int2 *>(M->inner_pairs), (long)w.bx * 256 + threadIdx.x);
+  }
+}
+"""
+RK_PASS_ENSEMBLE_LAUNCH = r"""extern "C" hipError_t launch_bssn_ens_rk_det_@TAG@(dim3 g, hipStream_t s, const bhah_member *mem,
+    const bhah_item *items, int nitems, int k_sel, int out_sel, int substep, int np) {
+  if (np == 2)
+    hipLaunchKernelGGL(bssn_ens_rk_det_@TAG@<2>, g, dim3(256), 0, s, mem, items, nitems, k_sel, out_sel, substep);
+  else
+    hipLaunchKernelGGL(bssn_ens_rk_det_@TAG@<1>, g, dim3(256), 0, s, mem, items, nitems, k_sel, out_sel, substep);
+  return hipGetLastError();
+}
+"""
+
+
 def bssn_kernels(v: specs.Variant, fd_order: int, ensemble: bool = False) -> str:
     """Kernels shared by every schedule: RK4+det pass, det enforcement, constraints
     (and, for ensemble builds, the batched RK4+det pass)."""
@@ -1761,208 +2048,12 @@ def bssn_kernels(v: specs.Variant, fd_order: int, ensemble: bool = False) -> str
     rats: Dict[str, str] = {}
     ngf = len(bssn.EVOL_GFS)
     # ---- RK4 substep update + det(gammabar) enforcement, all points, one streaming pass
-    det = detgamma_inline(v, rats, "nxt")
-    # One thread per point in array order (every lane of every wave on consecutive
-    # addresses, no partial rows); every array is streamed once, so loads and stores
-    # carry the non-temporal hint.
-    rk_nt = RK_EPILOGUE
-    for a, b in (("y_run[g * Ntot + idx] = (1.0 / 6.0) * dt * k;",
-                  "__builtin_nontemporal_store((1.0 / 6.0) * dt * k, &y_run[g * Ntot + idx]);"),
-                 ("(1.0 / 6.0) * dt * k + y_n[g * Ntot + idx] + y_run[g * Ntot + idx];",
-                  "(1.0 / 6.0) * dt * k + __builtin_nontemporal_load(&y_n[g * Ntot + idx]) + "
-                  "__builtin_nontemporal_load(&y_run[g * Ntot + idx]);"),
-                 ("y_run[g * Ntot + idx] = (1.0 / 3.0) * dt * k + y_run[g * Ntot + idx];",
-                  "__builtin_nontemporal_store((1.0 / 3.0) * dt * k + __builtin_nontemporal_load(&y_run[g * Ntot + idx]), "
-                  "&y_run[g * Ntot + idx]);"),
-                 ("a * dt * k + y_n[g * Ntot + idx];", "a * dt * k + __builtin_nontemporal_load(&y_n[g * Ntot + idx]);")):
-        assert a in rk_nt, a
-        rk_nt = rk_nt.replace(a, b)
-    rkdet = f"""
-extern "C" __global__ void __launch_bounds__(256)
-bssn_rk_det_{tag}(const double *__restrict__ kin, const double *y_n, double *__restrict__ y_run, double *out,
-                  const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p) {{
-  const long Ntot = p.Ntot;
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= Ntot) return;
-  const int i0 = (int)(idx % p.Nx0), i1 = (int)((idx / p.Nx0) % p.Nx1);
-  constexpr int NGF = {ngf};
-  double kk[NGF], ctr[NGF];
-#pragma unroll
-  for (int g = 0; g < NGF; g++) {{
-    kk[g] = __builtin_nontemporal_load(&kin[g * Ntot + idx]);
-    ctr[g] = (p.substep == 1) ? __builtin_nontemporal_load(&y_n[g * Ntot + idx]) : 0.0;
-  }}
-{rk_nt}
-{det}
-#pragma unroll
-  for (int g = 0; g < NGF; g++) __builtin_nontemporal_store(nxt[g], &out[g * Ntot + idx]);
-}}
-"""
-    # Two consecutive points per thread with 16-byte loads and stores: twice the bytes per
-    # request of every array stream.  Same arithmetic per point as the pass above; the
-    # launcher takes it when Ntot is even and every array is 16-byte aligned.
-    rkdet += f"""
-typedef double bhah_d2 __attribute__((ext_vector_type(2)));
-extern "C" __global__ void __launch_bounds__(256)
-bssn_rk_det2_{tag}(const double *__restrict__ kin, const double *y_n, double *__restrict__ y_run, double *out,
-                   const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p) {{
-  const long Ntot = p.Ntot;
-  const long idx2 = ((long)blockIdx.x * 256 + threadIdx.x) * 2;
-  if (idx2 >= Ntot) return;
-  constexpr int NGF = {ngf};
-  const bhah_d2 *K2 = (const bhah_d2 *)(kin + idx2), *YN2 = (const bhah_d2 *)(y_n + idx2);
-  bhah_d2 *YR2 = (bhah_d2 *)(y_run + idx2), *OUT2 = (bhah_d2 *)(out + idx2);
-  const long S2 = Ntot / 2;  // gridfunction stride in pairs
-  // RK4 substep update (register_all_MoL_step_forward_in_time.c:4-103), in registers.
-  const double dt = p.dt;
-  bhah_d2 nx2[NGF];
-  if (p.substep == 1) {{
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {{
-      const bhah_d2 k = __builtin_nontemporal_load(&K2[g * S2]);
-      __builtin_nontemporal_store((1.0 / 6.0) * dt * k, &YR2[g * S2]);
-      nx2[g] = (1.0 / 2.0) * dt * k + __builtin_nontemporal_load(&YN2[g * S2]);
-    }}
-  }} else if (p.substep == 4) {{
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {{
-      const bhah_d2 k = __builtin_nontemporal_load(&K2[g * S2]);
-      nx2[g] = (1.0 / 6.0) * dt * k + __builtin_nontemporal_load(&YN2[g * S2]) + __builtin_nontemporal_load(&YR2[g * S2]);
-    }}
-  }} else {{
-    const double a = (p.substep == 2) ? (1.0 / 2.0) : 1.0;
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {{
-      const bhah_d2 k = __builtin_nontemporal_load(&K2[g * S2]);
-      __builtin_nontemporal_store((1.0 / 3.0) * dt * k + __builtin_nontemporal_load(&YR2[g * S2]), &YR2[g * S2]);
-      nx2[g] = a * dt * k + __builtin_nontemporal_load(&YN2[g * S2]);
-    }}
-  }}
-#pragma unroll
-  for (int h = 0; h < 2; h++) {{
-    const long idx = idx2 + h;
-    const int i0 = (int)(idx % p.Nx0), i1 = (int)((idx / p.Nx0) % p.Nx1);
-    double nxt[NGF];
-#pragma unroll
-    for (int g = 0; g < NGF; g++) nxt[g] = nx2[g][h];
-{det}
-#pragma unroll
-    for (int g = 0; g < NGF; g++) nx2[g][h] = nxt[g];
-  }}
-#pragma unroll
-  for (int g = 0; g < NGF; g++) __builtin_nontemporal_store(nx2[g], &OUT2[g * S2]);
-}}
-"""
-    # The same pass with the inner-parity boundary condition of the right-hand side folded in:
-    # at an inner ghost point k is the value at its source point with the parity sign
-    # (apply_bcs_inner_only__openmp.c:3-57).  kin is only read by this pass, so the value is the
-    # one the separate copy would have stored there: the same k, bit for bit.  Each pair of points
-    # reads its k from one 16-byte-aligned source pair (its own pair away from the inner ghost
-    # zones), so a gridfunction costs one 16-byte load, as in the pass above.
-    rkdet += f"""
-extern "C" __global__ void __launch_bounds__(256)
-bssn_rk_deti2_{tag}(const double *__restrict__ kin, const double *y_n, double *__restrict__ y_run, double *out,
-                    const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p,
-                    const int2 *__restrict__ pmap, const int *__restrict__ gfpar) {{
-  const long Ntot = p.Ntot;
-  const long q = (long)blockIdx.x * 256 + threadIdx.x;  // pair index
-  const long idx2 = q * 2;
-  if (idx2 >= Ntot) return;
-  constexpr int NGF = {ngf};
-  const bhah_d2 *K2 = (const bhah_d2 *)kin, *YN2 = (const bhah_d2 *)(y_n + idx2);
-  bhah_d2 *YR2 = (bhah_d2 *)(y_run + idx2), *OUT2 = (bhah_d2 *)(out + idx2);
-  const long S2 = Ntot / 2;  // gridfunction stride in pairs
-  // source pair; code bit 0 / bit 1: point 0 / point 1 takes the source pair's second value;
-  // bits 4-15 / 16-27: the parity-type masks of points 0 / 1 (bit t set: type t flips sign)
-  const int2 pm = pmap[q];
-  const long sp = pm.x;
-  const unsigned code = (unsigned)pm.y;
-#define BHAH_KPAIR(g)                                                                               \\
-  ({{                                                                                               \\
-    const bhah_d2 v_ = __builtin_nontemporal_load(&K2[(g) * S2 + sp]);                              \\
-    const unsigned par_ = (unsigned)gfpar[g];                                                       \\
-    const double a_ = (code & 1u) ? v_.y : v_.x, b_ = (code & 2u) ? v_.y : v_.x;                    \\
-    bhah_d2 k_;                                                                                     \\
-    k_.x = ((code >> (4 + par_)) & 1u) ? -a_ : a_;                                                  \\
-    k_.y = ((code >> (16 + par_)) & 1u) ? -b_ : b_;                                                 \\
-    k_;                                                                                             \\
-  }})
-  const double dt = p.dt;
-  bhah_d2 nx2[NGF];
-  if (p.substep == 1) {{
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {{
-      const bhah_d2 k = BHAH_KPAIR(g);
-      __builtin_nontemporal_store((1.0 / 6.0) * dt * k, &YR2[g * S2]);
-      nx2[g] = (1.0 / 2.0) * dt * k + __builtin_nontemporal_load(&YN2[g * S2]);
-    }}
-  }} else if (p.substep == 4) {{
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {{
-      const bhah_d2 k = BHAH_KPAIR(g);
-      nx2[g] = (1.0 / 6.0) * dt * k + __builtin_nontemporal_load(&YN2[g * S2]) + __builtin_nontemporal_load(&YR2[g * S2]);
-    }}
-  }} else {{
-    const double a = (p.substep == 2) ? (1.0 / 2.0) : 1.0;
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {{
-      const bhah_d2 k = BHAH_KPAIR(g);
-      __builtin_nontemporal_store((1.0 / 3.0) * dt * k + __builtin_nontemporal_load(&YR2[g * S2]), &YR2[g * S2]);
-      nx2[g] = a * dt * k + __builtin_nontemporal_load(&YN2[g * S2]);
-    }}
-  }}
-#undef BHAH_KPAIR
-#pragma unroll
-  for (int h = 0; h < 2; h++) {{
-    const long idx = idx2 + h;
-    const int i0 = (int)(idx % p.Nx0), i1 = (int)((idx / p.Nx0) % p.Nx1);
-    double nxt[NGF];
-#pragma unroll
-    for (int g = 0; g < NGF; g++) nxt[g] = nx2[g][h];
-{det}
-#pragma unroll
-    for (int g = 0; g < NGF; g++) nx2[g][h] = nxt[g];
-  }}
-#pragma unroll
-  for (int g = 0; g < NGF; g++) __builtin_nontemporal_store(nx2[g], &OUT2[g * S2]);
-}}
-"""
-    ens_rk = ""
-    if ensemble:
-        ens_rk = f"""
-// Records are (member, chunk): 256 consecutive points of the member's arrays, in array order
-// (the single-patch pass's indexing and non-temporal hints).
-static __device__ __forceinline__ void bssn_ens_rk_det_{tag}_tile(const double *__restrict__ kin, const double *y_n,
-        double *__restrict__ y_run, double *out, const double *__restrict__ rfm0, const double *__restrict__ rfm1,
-        const bhah_kparams p, const int chunk) {{
-  const long Ntot = p.Ntot;
-  const long idx = (long)chunk * 256 + (threadIdx.x + blockDim.x * threadIdx.y);
-  if (idx >= Ntot) return;
-  const int i0 = (int)(idx % p.Nx0), i1 = (int)((idx / p.Nx0) % p.Nx1);
-  constexpr int NGF = {ngf};
-  double kk[NGF], ctr[NGF];
-#pragma unroll
-  for (int g = 0; g < NGF; g++) {{
-    kk[g] = __builtin_nontemporal_load(&kin[g * Ntot + idx]);
-    ctr[g] = (p.substep == 1) ? __builtin_nontemporal_load(&y_n[g * Ntot + idx]) : 0.0;
-  }}
-{rk_nt}
-{det}
-#pragma unroll
-  for (int g = 0; g < NGF; g++) __builtin_nontemporal_store(nxt[g], &out[g * Ntot + idx]);
-}}
-extern "C" __global__ void __launch_bounds__(256)
-bssn_ens_rk_det_{tag}(const bhah_member *__restrict__ mem, const bhah_item *__restrict__ items, const int nitems,
-                      const int k_sel, const int out_sel, const int substep) {{
-  for (int it = blockIdx.x; it < nitems; it += gridDim.x) {{
-    const bhah_item w = items[it];
-    const bhah_member *M = &mem[w.m];
-    bhah_kparams p = M->kp;
-    p.substep = substep;
-    bssn_ens_rk_det_{tag}_tile(M->arr[k_sel], M->arr[0], M->arr[1], M->arr[out_sel], M->rfm0, M->rfm1, p, w.bx);
-  }}
-}}
-"""
+    h0 = bssn.EVOL_GFS.index("hDD00")
+    det = detgamma_inline(v, rats, "nxt", h0)
+    par = [bssn.parity_type(g) for g in bssn.EVOL_GFS]
+    rkdet = RK_PASS.replace("@TAG@", tag).replace("@DET@", det).replace("@PAR@", ", ".join(map(str, par)))
+    assert [bssn.EVOL_GFS.index(f"hDD{i}{j}") - h0 for i in range(3) for j in range(i, 3)] == list(range(6)) and h0 == 11
+    ens_rk = RK_PASS_ENSEMBLE.replace("@TAG@", tag) if ensemble else ""
     # ---- det enforcement over all points (standalone ABI call)
     dspec = specs.detgamma_spec(v)
     det_all = f"""
@@ -2008,35 +2099,8 @@ bssn_initial_lambda_{tag}(double *gfs, const double *__restrict__ rfm0, const do
     head = [f"// ---- BSSN kernels: {v.coord}, symmetry axes '{v.symmetry_axes}', KO={v.enable_KO}, fd_order={fd_order}"]
     consts = "\n".join(f"#define {k} ({v})" for k, v in sorted(rats.items()))
     undefs = "\n".join(f"#undef {k}" for k in sorted(rats))
-    launch = f"""
+    launch = RK_PASS_LAUNCH.replace("@TAG@", tag) + f"""
 // Host-side launchers (one translation unit per variant; no relocatable device code needed).
-extern "C" hipError_t launch_bssn_rk_det_{tag}(dim3 g, dim3 b, hipStream_t s, const double *kin, const double *y_n,
-    double *y_run, double *out, const double *rfm0, const double *rfm1, bhah_kparams p) {{
-  (void)g;
-  (void)b;
-  const bool pairs = !(p.Ntot & 1) && !((reinterpret_cast<uintptr_t>(kin) | reinterpret_cast<uintptr_t>(y_n) |
-                                         reinterpret_cast<uintptr_t>(y_run) | reinterpret_cast<uintptr_t>(out)) & 15);
-  if (pairs)
-    hipLaunchKernelGGL(bssn_rk_det2_{tag}, dim3((unsigned)((p.Ntot / 2 + 255) / 256)), dim3(256), 0, s, kin, y_n, y_run,
-                       out, rfm0, rfm1, p);
-  else
-    hipLaunchKernelGGL(bssn_rk_det_{tag}, dim3((unsigned)((p.Ntot + 255) / 256)), dim3(256), 0, s, kin, y_n, y_run,
-                       out, rfm0, rfm1, p);
-  return hipGetLastError();
-}}
-// The RK pass with the inner boundary condition folded in: pairs only (even Ntot, 16-byte aligned
-// arrays); a call that does not meet that returns hipErrorInvalidValue and launches nothing.
-extern "C" hipError_t launch_bssn_rk_det_inner_{tag}(hipStream_t s, const double *kin, const double *y_n,
-    double *y_run, double *out, const double *rfm0, const double *rfm1, bhah_kparams p, const int *pmap,
-    const int *gfpar) {{
-  if ((p.Ntot & 1) || ((reinterpret_cast<uintptr_t>(kin) | reinterpret_cast<uintptr_t>(y_n) |
-                        reinterpret_cast<uintptr_t>(y_run) | reinterpret_cast<uintptr_t>(out) |
-                        reinterpret_cast<uintptr_t>(pmap)) & 15))
-    return hipErrorInvalidValue;
-  hipLaunchKernelGGL(bssn_rk_deti2_{tag}, dim3((unsigned)((p.Ntot / 2 + 255) / 256)), dim3(256), 0, s, kin, y_n, y_run,
-                     out, rfm0, rfm1, p, reinterpret_cast<const int2 *>(pmap), gfpar);
-  return hipGetLastError();
-}}
 extern "C" hipError_t launch_bssn_constraints_{tag}(dim3 g, dim3 b, hipStream_t s, const double *in,
     const double *aux, double *diag, const double *rfm0, const double *rfm1, bhah_kparams p) {{
   hipLaunchKernelGGL(bssn_constraints_{tag}, g, b, 0, s, in, aux, diag, rfm0, rfm1, p);
@@ -2054,12 +2118,7 @@ extern "C" hipError_t launch_bssn_initial_lambda_{tag}(dim3 g, dim3 b, hipStream
 }}
 """
     if ensemble:
-        launch += f"""extern "C" hipError_t launch_bssn_ens_rk_det_{tag}(dim3 g, dim3 b, hipStream_t s, const bhah_member *mem,
-    const bhah_item *items, int nitems, int k_sel, int out_sel, int substep) {{
-  hipLaunchKernelGGL(bssn_ens_rk_det_{tag}, g, b, 0, s, mem, items, nitems, k_sel, out_sel, substep);
-  return hipGetLastError();
-}}
-"""
+        launch += RK_PASS_ENSEMBLE_LAUNCH.replace("@TAG@", tag)
     return "\n".join(head) + "\n" + consts + "\n" + rkdet + ens_rk + det_all + cons + undefs + "\n" + launch
 
 
@@ -2201,11 +2260,11 @@ def generate(outdir: str) -> List[str]:
             ]
         if ens:
             table_decl.append(
-                f'extern "C" hipError_t launch_bssn_ens_rk_det_{tag}(dim3, dim3, hipStream_t, const bhah_member *, '
-                f"const bhah_item *, int, int, int, int);"
+                f'extern "C" hipError_t launch_bssn_ens_rk_det_{tag}(dim3, hipStream_t, const bhah_member *, '
+                f"const bhah_item *, int, int, int, int, int);"
             )
         table_decl.append(
-            f'extern "C" hipError_t launch_bssn_rk_det_{tag}(dim3, dim3, hipStream_t, const double *, const double *, '
+            f'extern "C" hipError_t launch_bssn_rk_det_{tag}(hipStream_t, const double *, const double *, '
             f"double *, double *, const double *, const double *, bhah_kparams);"
         )
         table_decl.append(

@@ -23,6 +23,8 @@ struct bhah_member {
   double *arr[5];
   int coord;
   double AMPL, SINHW;
+  const double *rad;  // r(xx0), dxx0/dr
+  const int *inner_map, *inner_pairs;  // sources of the inner points, for the RK pass
 };
 
 // One unit of batched work: member index and tile coordinates (tile along

@@ -42,16 +42,16 @@ struct BssnKernels {
   int n_rhs;
   const BssnCandidate *ricci;
   int n_ricci;
-  hipError_t (*rk_det)(dim3, dim3, hipStream_t, const double *, const double *, double *, double *, const double *,
+  hipError_t (*rk_det)(hipStream_t, const double *, const double *, double *, double *, const double *,
                        const double *, bhah_kparams);
-  // the same pass taking the inner-parity boundary condition of k with it (pairs of points only)
+  // the same pass taking the inner-parity boundary condition of k with it (per-point map, pair map)
   hipError_t (*rk_det_inner)(hipStream_t, const double *, const double *, double *, double *, const double *,
                              const double *, bhah_kparams, const int *, const int *);
   hipError_t (*detgamma)(dim3, dim3, hipStream_t, double *, const double *, const double *, bhah_kparams);
   hipError_t (*constraints)(dim3, dim3, hipStream_t, const double *, const double *, double *, const double *,
                             const double *, bhah_kparams);
   hipError_t (*initial_lambda)(dim3, dim3, hipStream_t, double *, const double *, const double *, bhah_kparams);
-  hipError_t (*ens_rk_det)(dim3, dim3, hipStream_t, const bhah_member *, const bhah_item *, int, int, int, int);
+  hipError_t (*ens_rk_det)(dim3, hipStream_t, const bhah_member *, const bhah_item *, int, int, int, int, int);
   // reverse-mode kernels of one RK4 step (builds with adjoints only)
   int (*adj_nslots)(void);
   hipError_t (*adj_rhs)(dim3, dim3, hipStream_t, const double *, const double *, const double *, double *,
@@ -113,11 +113,12 @@ struct bhah_patch {
   double *d_rfm0 = nullptr, *d_rfm1 = nullptr, *d_xx0 = nullptr, *d_xx1 = nullptr, *d_xx2 = nullptr;
   int *d_inner_dst = nullptr, *d_inner_src = nullptr;
   unsigned short *d_inner_mask = nullptr;  // bit t set: parity type t flips sign
-  // per pair of points (2q, 2q+1): the 16-byte-aligned pair that holds the sources of both
-  // points' right-hand sides (the pair itself away from inner ghost points) and a code: bit 0 /
-  // bit 1 set when point 0 / point 1 takes that pair's second value, bits 4-15 / 16-27 the parity
-  // masks of points 0 / 1.  Null when some pair's sources are not in one aligned pair.
-  int *d_inner_pairs = nullptr;
+  // Where the RK pass finds k of inner ghost points.  d_inner_map: (source, parity mask) of every
+  // point.  d_inner_pairs (even Ntot), per pair of points (2q, 2q+1): where one 16-byte-aligned
+  // pair holds the sources of both (the pair itself away from inner ghost points) that pair and a
+  // code: bit 0 / bit 1 set when point 0 / point 1 takes its second value, bits 4-15 / 16-27 the
+  // parity masks of points 0 / 1; otherwise a negative code, and the points' own records hold.
+  int *d_inner_map = nullptr, *d_inner_pairs = nullptr;
   // the MoL step takes the inner boundary condition of k inside the RK pass (environment
   // BHAH_HIP_SEPARATE_INNER_BC=1 at patch creation keeps the separate copy, for comparison)
   bool fold_inner = true;
@@ -128,6 +129,7 @@ struct bhah_patch {
   int16_t *d_outer[8][3] = {};
   int *d_rad_lines = nullptr;  // (i1, i2) per radial line when the outer points form lines
   int n_rad_lines = 0;
+  double *d_rad = nullptr;  // r(xx0), dxx0/dr
   double *d_wavespeed = nullptr, *d_finf = nullptr;
   double *d_red = nullptr;  // volume-integral partial sums (VI_MAX_BLOCKS x VI_SUMS) and totals
   int *d_gf_parity = nullptr;
@@ -268,170 +270,98 @@ bc_radiation_kernel(const int16_t *__restrict__ pts, int npts, int ngfs, const d
             invdxx0);
 }
 
-// All ghost layers of the radiation condition in one launch, for grids whose pure outer
-// points are radial lines (i1, i2 fixed, i0 = Nx0-NG .. Nx0-1; spherical-like coordinates):
-// one thread per (line, gridfunction) walks the layers innermost first; the right-hand side
-// at a layer's interior neighbour is the value the thread formed one layer earlier (the
-// first layer's is loaded), kept in a register.  Same arithmetic as rad_point.
-__global__ void __launch_bounds__(256)
-bc_radiation_lines_kernel(const int *__restrict__ lines, int nlines, int ngfs, int NG, const double *__restrict__ gfs,
-                          double *__restrict__ rhs, const double *__restrict__ xx0,
-                          const double *__restrict__ wavespeed, const double *__restrict__ finf, RadStencil st,
-                          int R, int coord, double AMPL, double SINHW, int Nx0, long s1, long s2, long Ntot,
-                          double invdxx0) {
+// All ghost layers of the radiation condition on one radial line (i1, i2 fixed, i0 = Nx0-NG ..
+// Nx0-1; the form of the pure outer points of spherical-like grids) of one gridfunction: f and rr
+// point at the line, r and dxr at r(xx0) and dxx0/dr.  The layers are walked innermost first; the
+// right-hand side at a layer's interior neighbour is the value formed one layer earlier.  Same
+// arithmetic as rad_point.
+//
+// The launch is bound by the cache lines its strided accesses touch, and on small grids by the
+// chain of dependent loads, so the number of ghost layers and the stencil radius are compile-time
+// constants: the line's NG + R + 2 values are loaded at once and each radial derivative is formed
+// once (a layer's interior neighbour is the layer before).  In whole steps, against staging 16 values
+// of each line in LDS (large grids) or loading per layer: 25.7 -> 20.0 us at 192x96x96, 14.3 -> 5.8
+// at 96x48x48, 8.8 -> 4.6 at 72x12x2; one launch of 12.2 us for a 64-member ensemble, which took one
+// of 16.0 per layer.
+struct RadLine {
+  double w[3][7];  // weights of the derivative on 2R+1 points shifted by -1, -2, -3
+};
+template <int NG, int R>
+__device__ __forceinline__ void rad_line(const RadLine &W, const double *__restrict__ f, double *__restrict__ rr,
+                                         const double *__restrict__ r, const double *__restrict__ dxr, double c,
+                                         double f_inf, int Nx0, double invdxx0) {
 #pragma clang fp contract(off)
+  constexpr int L = NG + R + 2;
+  double v[L], d[NG + 1];
+  const int lo = Nx0 - L, first = Nx0 - NG - 1;
+#pragma unroll
+  for (int e = 0; e < L; e++) v[e] = f[lo + e];
+  double dtf_int = rr[first];
+#pragma unroll
+  for (int m = 0; m <= NG; m++) {  // derivative at i0 = first + m, as partial_r_f with FACE0 = -1
+    const int off = (m > NG - R) ? NG - R - m : -1;
+    double acc = 0.0;
+#pragma unroll
+    for (int q = 0; q <= 2 * R; q++) acc += W.w[-off - 1][q] * v[1 + m + off + q];
+    d[m] = dxr[first + m] * (acc * invdxx0);
+  }
+#pragma unroll
+  for (int m = 1; m <= NG; m++) {
+    const double r_int = r[first + m - 1];
+    const double dtf_int_out = -c * (d[m - 1] + (v[R + m] - f_inf) / r_int);
+    const double k = r_int * r_int * r_int * (dtf_int - dtf_int_out);
+    const double rinv = 1.0 / r[first + m];
+    const double dtf_out = -c * (d[m] + (v[R + 1 + m] - f_inf) * rinv);
+    dtf_int = dtf_out + k * rinv * rinv * rinv;
+    rr[first + m] = dtf_int;
+  }
+}
+
+template <int NG, int R>
+__global__ void __launch_bounds__(256)
+bc_radiation_lines_kernel(const int *__restrict__ lines, int nlines, int ngfs, const double *__restrict__ gfs,
+                          double *__restrict__ rhs, const double *__restrict__ rad,
+                          const double *__restrict__ wavespeed, const double *__restrict__ finf, RadLine W, int Nx0,
+                          long s1, long s2, long Ntot, double invdxx0) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)nlines * ngfs) return;
   const int l = (int)(t % nlines), gf = (int)(t / nlines);
-  const long base = s1 * lines[2 * l] + s2 * lines[2 * l + 1];
-  const double *f = &gfs[gf * Ntot];
-  double *rr = &rhs[gf * Ntot];
-  const double c = wavespeed[gf], f_inf = finf[gf];
-  double dtf_int = rr[base + Nx0 - NG - 1];
-  double r_int, dxr_int;
-  r_and_dx0dr(coord, AMPL, SINHW, xx0[Nx0 - NG - 1], r_int, dxr_int);
-  for (int gz = 0; gz < NG; gz++) {
-    const int i0 = Nx0 - NG + gz, j0 = i0 - 1;
-    const long idx = base + i0, idx_int = base + j0;
-    double r, dxr;
-    r_and_dx0dr(coord, AMPL, SINHW, xx0[i0], r, dxr);
-    const double dfr = partial_r_f(st, R, f, Nx0, idx, i0, -1, dxr, invdxx0);
-    const double dfr_int = partial_r_f(st, R, f, Nx0, idx_int, j0, -1, dxr_int, invdxx0);
-    const double dtf_int_out = -c * (dfr_int + (f[idx_int] - f_inf) / r_int);
-    const double k = r_int * r_int * r_int * (dtf_int - dtf_int_out);
-    const double rinv = 1.0 / r;
-    const double dtf_out = -c * (dfr + (f[idx] - f_inf) * rinv);
-    const double v = dtf_out + k * rinv * rinv * rinv;
-    rr[idx] = v;
-    dtf_int = v;
-    r_int = r;
-    dxr_int = dxr;
-  }
+  const long base = gf * Ntot + s1 * lines[2 * l] + s2 * lines[2 * l + 1];
+  rad_line<NG, R>(W, gfs + base, rhs + base, rad, rad + Nx0, wavespeed[gf], finf[gf], Nx0, invdxx0);
 }
 
-// The same walk with each line's last RAD_SEG values of the gridfunction staged in LDS by
-// coalesced loads (lanes of a wave read consecutive values of four lines), instead of every
-// lane reading its own line with a separate cache line per load; the layers' results are
-// written back the same way.  Needs Nx0 >= RAD_SEG and every stencil point of the walk
-// within the segment (NG + R + 2 <= RAD_SEG, checked by the host).  Same arithmetic as
-// bc_radiation_lines_kernel.
-constexpr int RAD_SEG = 16, RAD_PITCH = RAD_SEG + 1;
-constexpr long RAD_STAGED_MIN_ITEMS = 8192;
-
-__device__ __forceinline__ double partial_r_seg(const RadStencil &st, int R, const double *seg, int Nx0, int i0,
-                                                double dx0dr, double invdxx0) {
-#pragma clang fp contract(off)
-  // one-sided towards the interior at the outer face (FACE0 = -1), as partial_r_f
-  const int off = (i0 > Nx0 - R - 1) ? (Nx0 - R - 1) - i0 : -1;
-  const int k = off + R;
-  const int c = i0 - (Nx0 - RAD_SEG);
-  double acc = 0.0;
-  for (int j = 0; j < st.n[k]; j++) acc += st.w[k][j] * seg[c + st.off[k][j]];
-  return dx0dr * (acc * invdxx0);
-}
-
+// The same over the concatenated lines of an ensemble's members.
+struct ens_rad_line {
+  int m, base;  // member; s1 * i1 + s2 * i2
+};
+template <int NG, int R>
 __global__ void __launch_bounds__(256)
-bc_radiation_lines_lds_kernel(const int *__restrict__ lines, int nlines, int ngfs, int NG,
-                              const double *__restrict__ gfs, double *__restrict__ rhs, const double *__restrict__ xx0,
-                              const double *__restrict__ wavespeed, const double *__restrict__ finf, RadStencil st,
-                              int R, int coord, double AMPL, double SINHW, int Nx0, long s1, long s2, long Ntot,
-                              double invdxx0) {
-#pragma clang fp contract(off)
-  __shared__ double seg[256 * RAD_PITCH];
-  __shared__ long row[256];  // gf * Ntot + line base of each item of the block
-  const int tid = (int)threadIdx.x;
-  const long nitems = (long)nlines * ngfs, t0 = (long)blockIdx.x * 256, t = t0 + tid;
-  const bool active = t < nitems;
-  if (active) {
-    const int l = (int)(t % nlines), gf = (int)(t / nlines);
-    row[tid] = gf * Ntot + s1 * lines[2 * l] + s2 * lines[2 * l + 1];
-  }
-  __syncthreads();
-  for (int j = 0; j < RAD_SEG; j++) {
-    const int e = tid + 256 * j, it = e / RAD_SEG, x = e % RAD_SEG;
-    if (t0 + it < nitems) seg[it * RAD_PITCH + x] = gfs[row[it] + (Nx0 - RAD_SEG) + x];
-  }
-  __syncthreads();
-  if (active) {
-    const double *f = &seg[tid * RAD_PITCH];
-    const long base = row[tid];
-    const int gf = (int)(t / nlines);
-    const double c = wavespeed[gf], f_inf = finf[gf];
-    double dtf_int = rhs[base + Nx0 - NG - 1];
-    double r_int, dxr_int;
-    r_and_dx0dr(coord, AMPL, SINHW, xx0[Nx0 - NG - 1], r_int, dxr_int);
-    double v[8];
-    for (int gz = 0; gz < NG; gz++) {
-      const int i0 = Nx0 - NG + gz, j0 = i0 - 1;
-      double r, dxr;
-      r_and_dx0dr(coord, AMPL, SINHW, xx0[i0], r, dxr);
-      const double dfr = partial_r_seg(st, R, f, Nx0, i0, dxr, invdxx0);
-      const double dfr_int = partial_r_seg(st, R, f, Nx0, j0, dxr_int, invdxx0);
-      const double dtf_int_out = -c * (dfr_int + (f[j0 - (Nx0 - RAD_SEG)] - f_inf) / r_int);
-      const double k = r_int * r_int * r_int * (dtf_int - dtf_int_out);
-      const double rinv = 1.0 / r;
-      const double dtf_out = -c * (dfr + (f[i0 - (Nx0 - RAD_SEG)] - f_inf) * rinv);
-      v[gz] = dtf_out + k * rinv * rinv * rinv;
-      dtf_int = v[gz];
-      r_int = r;
-      dxr_int = dxr;
-    }
-    // this thread alone read its segment: its results take the segment's first NG slots
-    for (int gz = 0; gz < NG; gz++) seg[tid * RAD_PITCH + gz] = v[gz];
-  }
-  __syncthreads();
-  for (int j = 0; j < NG; j++) {
-    const int e = tid + 256 * j, it = e / NG, gz = e % NG;
-    if (t0 + it < nitems) rhs[row[it] + (Nx0 - NG) + gz] = seg[it * RAD_PITCH + gz];
-  }
+ens_bc_radiation_lines_kernel(const bhah_member *__restrict__ mem, const ens_rad_line *__restrict__ lines, int nlines,
+                              int ngfs, int in_sel, int rhs_sel, const double *__restrict__ wavespeed,
+                              const double *__restrict__ finf, RadLine W) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (long)nlines * ngfs) return;
+  const int gf = (int)(t / nlines);
+  const ens_rad_line e = lines[t % nlines];
+  const bhah_member *M = &mem[e.m];
+  const int Nx0 = M->kp.Nx0;
+  const long base = gf * M->kp.Ntot + e.base;
+  rad_line<NG, R>(W, M->arr[in_sel] + base, M->arr[rhs_sel] + base, M->rad, M->rad + Nx0, wavespeed[gf], finf[gf],
+                  Nx0, M->kp.invdxx0);
+}
+
+// r(xx0) and dxx0/dr of every xx0 point, as rad_point forms them.
+__global__ void __launch_bounds__(256)
+rad_arrays_kernel(double *__restrict__ rad, const double *__restrict__ xx0, int Nx0, int coord, double AMPL, double SINHW) {
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i >= Nx0) return;
+  double r, dxr;
+  r_and_dx0dr(coord, AMPL, SINHW, xx0[i], r, dxr);
+  rad[i] = r;
+  rad[Nx0 + i] = dxr;
 }
 
 constexpr int BC_INNER_BATCH = 12;  // gridfunctions in flight per thread in the inner-parity copy
-
-// Batched forms over an ensemble: one record per (member, boundary point), one
-// thread per (record, gridfunction); member arrays are picked by index.
-struct ens_outer_pt {
-  int m;
-  int16_t q[6];  // i0, i1, i2, face normal
-};
-struct ens_inner_pt {
-  int m, dst, src;
-  unsigned mask;
-};
-
-__global__ void __launch_bounds__(256)
-ens_bc_radiation_kernel(const bhah_member *__restrict__ mem, const ens_outer_pt *__restrict__ pts, int npts,
-                        int ngfs, int in_sel, int rhs_sel, const double *__restrict__ wavespeed,
-                        const double *__restrict__ finf, RadStencil st, int R) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)npts * ngfs) return;
-  const int p = (int)(t % npts), gf = (int)(t / npts);
-  const ens_outer_pt e = pts[p];
-  const bhah_member *M = &mem[e.m];
-  rad_point(e.q, gf, M->arr[in_sel], M->arr[rhs_sel], M->xx0, wavespeed[gf], finf[gf], st, R, M->coord, M->AMPL,
-            M->SINHW, M->kp.Nx0, M->kp.s1, M->kp.s2, M->kp.Ntot, M->kp.invdxx0);
-}
-
-__global__ void __launch_bounds__(256)
-ens_bc_inner_kernel(const bhah_member *__restrict__ mem, const ens_inner_pt *__restrict__ pts, int npts, int ngfs,
-                    const int *__restrict__ gf_parity, int sel) {
-  // one thread per boundary point, all gridfunctions: the record is read once
-  const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (p >= npts) return;
-  const ens_inner_pt e = pts[p];
-  const bhah_member *M = &mem[e.m];
-  double *f = M->arr[sel];
-  const long Ntot = M->kp.Ntot;
-  for (int g0 = 0; g0 < ngfs; g0 += BC_INNER_BATCH) {  // loads of a batch before its stores
-    double v[BC_INNER_BATCH];
-#pragma unroll
-    for (int j = 0; j < BC_INNER_BATCH; j++)
-      if (g0 + j < ngfs) v[j] = f[(g0 + j) * Ntot + e.src];
-#pragma unroll
-    for (int j = 0; j < BC_INNER_BATCH; j++)
-      if (g0 + j < ngfs) f[(g0 + j) * Ntot + e.dst] = ((e.mask >> gf_parity[g0 + j]) & 1u) ? -v[j] : v[j];
-  }
-}
 
 // Quadratic extrapolation f0 = 3 f1 - 3 f2 + f3 along the face normal
 // (…/apply_bcs_outerextrap_and_inner__openmp.c:8-34).
@@ -470,6 +400,27 @@ bc_inner_kernel(const int *__restrict__ dst, const int *__restrict__ src, const 
     for (int j = 0; j < BC_INNER_BATCH; j++)
       if (g0 + j < ngfs) gfs[(g0 + j) * Ntot + d] = ((m >> gf_parity[g0 + j]) & 1u) ? -v[j] : v[j];
   }
+}
+
+// (source, parity mask) of every point for the RK pass: itself, then the inner ghost points' sources.
+__global__ void __launch_bounds__(256) point_map_self_kernel(int2 *__restrict__ map, long n) {
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < n) map[p] = int2{(int)p, 0};
+}
+__global__ void __launch_bounds__(256)
+point_map_inner_kernel(int2 *__restrict__ map, const int *__restrict__ dst, const int *__restrict__ src,
+                       const unsigned short *__restrict__ mask, int n) {
+  const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (t < n) map[dst[t]] = int2{src[t], (int)mask[t]};
+}
+
+__global__ void __launch_bounds__(256)
+pair_map_kernel(int2 *__restrict__ pairs, const int2 *__restrict__ map, long npairs) {
+  const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= npairs) return;
+  const int2 a = map[2 * q], b = map[2 * q + 1];
+  const bool one = (a.x >> 1) == (b.x >> 1);
+  pairs[q] = int2{a.x >> 1, one ? ((a.x & 1) | ((b.x & 1) << 1) | (a.y << 4) | (b.y << 16)) : -1};
 }
 
 // ---- Adjoints of the boundary conditions (reverse mode; linear maps).
@@ -1196,6 +1147,22 @@ int enqueue_volume_integrals(bhah_patch *P, const double *diag, double *partial,
   return BHAH_OK;
 }
 
+// The line form of the radiation condition takes three or four ghost layers (every build's) and
+// lines that hold all the values it reads.
+bool rad_lines_fit(int Nx0, int NG, int R) { return (NG == 3 || NG == 4) && Nx0 >= NG + R + 2; }
+
+// Workgroups of one wave until each CU has several: a launch over few items is then spread over
+// more CUs (3,456 items at 72x12x2).
+unsigned rad_threads(long items) { return items < (1L << 17) ? 64u : 256u; }
+
+RadLine rad_line_weights(const RadStencil &st, int R) {
+  RadLine W;
+  memset(&W, 0, sizeof(W));
+  for (int o = 1; o <= R; o++)  // no weight of a shifted stencil vanishes: entry q is offset q - o - R
+    for (int q = 0; q < 2 * R + 1; q++) W.w[o - 1][q] = st.w[R - o][q];
+  return W;
+}
+
 // Device address of `scratch` on the current GPU, looked up once per GPU with that GPU current
 // (each GPU holds its own copy of the array at its own address).
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -1582,6 +1549,26 @@ static int setup_on_device(bhah_patch &P, std::vector<double> &rfm0, std::vector
 }
 
 // Upload the set-up to the device and finish the patch (both set-up paths).
+// d_inner_map and d_inner_pairs, from the inner points on the device.
+static int inner_maps(bhah_patch *P, int n_inner) {
+  HIP_TRY(hipMalloc((void **)&P->d_inner_map, sizeof(int2) * (size_t)P->Ntot));
+  dim3 g, b;
+  launch_1d(P->Ntot, g, b);
+  hipLaunchKernelGGL(point_map_self_kernel, g, b, 0, nullptr, (int2 *)P->d_inner_map, P->Ntot);
+  launch_1d((long)n_inner, g, b);
+  hipLaunchKernelGGL(point_map_inner_kernel, g, b, 0, nullptr, (int2 *)P->d_inner_map, P->d_inner_dst, P->d_inner_src,
+                     P->d_inner_mask, n_inner);
+  if (!(P->Ntot & 1)) {
+    HIP_TRY(hipMalloc((void **)&P->d_inner_pairs, sizeof(int) * (size_t)P->Ntot));
+    launch_1d(P->Ntot / 2, g, b);
+    hipLaunchKernelGGL(pair_map_kernel, g, b, 0, nullptr, (int2 *)P->d_inner_pairs, (const int2 *)P->d_inner_map,
+                       P->Ntot / 2);
+  }
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(nullptr));
+  return BHAH_OK;
+}
+
 static int patch_upload(bhah_patch *P, const std::vector<double> &rfm0, const std::vector<double> &rfm1,
                         bhah_patch **out) {
   const bhah_patch_desc &d = P->d;
@@ -1624,25 +1611,8 @@ static int patch_upload(bhah_patch *P, const std::vector<double> &rfm0, const st
     bhah_hip_patch_destroy(P);
     return rc;
   }
-  if (d.system == BHAH_SYSTEM_BSSN && !(P->Ntot & 1) && !dst.empty()) {
-    std::vector<int> imap((size_t)P->Ntot, -1);
-    for (size_t p = 0; p < dst.size(); p++) imap[(size_t)dst[p]] = (int)p;
-    std::vector<int> pairs((size_t)P->Ntot);  // (source pair, code) per pair
-    bool ok = true;
-    for (long q = 0; q < P->Ntot / 2 && ok; q++) {
-      long sr[2];
-      unsigned m[2];
-      for (int e = 0; e < 2; e++) {
-        const int ip = imap[(size_t)(2 * q + e)];
-        sr[e] = ip >= 0 ? (long)src[(size_t)ip] : 2 * q + e;
-        m[e] = ip >= 0 ? mask[(size_t)ip] : 0u;
-        if (m[e] >> 12) ok = false;
-      }
-      if ((sr[0] >> 1) != (sr[1] >> 1)) ok = false;
-      pairs[(size_t)(2 * q)] = (int)(sr[0] >> 1);
-      pairs[(size_t)(2 * q + 1)] = (int)((sr[0] & 1) | ((sr[1] & 1) << 1) | (m[0] << 4) | (m[1] << 16));
-    }
-    if (ok && (rc = upload(pairs, &P->d_inner_pairs))) {
+  if (d.system == BHAH_SYSTEM_BSSN && !dst.empty()) {
+    if ((rc = inner_maps(P, (int)dst.size()))) {
       bhah_hip_patch_destroy(P);
       return rc;
     }
@@ -1677,6 +1647,16 @@ static int patch_upload(bhah_patch *P, const std::vector<double> &rfm0, const st
         return rc;
       }
       P->n_rad_lines = (int)(L0.size() / 6);
+      if (hipMalloc((void **)&P->d_rad, sizeof(double) * 2 * (size_t)P->Nx[0]) != hipSuccess) {
+        bhah_hip_patch_destroy(P);
+        return fail(BHAH_ERR_HIP, "hipMalloc failed");
+      }
+      hipLaunchKernelGGL(rad_arrays_kernel, dim3((P->Nx[0] + 255) / 256), dim3(256), 0, nullptr, P->d_rad, P->d_xx0,
+                         P->Nx[0], d.coord, d.grid_physical_size, d.SINHW);
+      if (hipGetLastError() != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
+        bhah_hip_patch_destroy(P);
+        return fail(BHAH_ERR_HIP, "radiation set-up failed");
+      }
     }
   }
   if (hipMalloc((void **)&P->d_red, (VI_MAX_BLOCKS + 1) * VI_SUMS * sizeof(double)) != hipSuccess) {
@@ -1709,7 +1689,9 @@ int bhah_hip_patch_destroy(bhah_patch *P) {
   hipFree(P->d_inner_src_list);
   hipFree(P->d_inner_src);
   hipFree(P->d_inner_mask);
+  hipFree(P->d_inner_map);
   hipFree(P->d_inner_pairs);
+  hipFree(P->d_rad);
   hipFree(P->d_wavespeed);
   hipFree(P->d_finf);
   hipFree(P->d_red);
@@ -1861,23 +1843,23 @@ static int apply_bcs_outerradiation(bhah_patch *P, const double *gfs, double *rh
   if (R < 1 || R > 3) return fail(BHAH_ERR_ARG, "radiation_bc_fd_order must be 2, 4 or 6");
   RadStencil st;
   rad_stencil(R, st);
-  if (P->n_rad_lines) {
-    dim3 g, b;
-    launch_1d((long)P->n_rad_lines * P->ngfs, g, b);
-    // Staged form from a few thousand (line, gridfunction) items up (259,584 items at
-    // 192x96x96: 71 -> 26 us per launch). Small patches keep the one-pass form, whose launch
-    // has no block-wide steps: at 3,456 items (72x12x2) the staged one took ~3 us longer.
+  if (P->n_rad_lines && rad_lines_fit(P->Nx[0], P->NG, R)) {
     const long items = (long)P->n_rad_lines * P->ngfs;
-    if (items >= RAD_STAGED_MIN_ITEMS && P->Nx[0] >= RAD_SEG && P->NG + R + 2 <= RAD_SEG && P->NG <= 8)
-      hipLaunchKernelGGL(bc_radiation_lines_lds_kernel, dim3((unsigned)(((long)P->n_rad_lines * P->ngfs + 255) / 256)),
-                         dim3(256), 0, P->stream, P->d_rad_lines, P->n_rad_lines, P->ngfs, P->NG, gfs, rhs, P->d_xx0,
-                         P->d_wavespeed, P->d_finf, st, R, P->d.coord, P->d.grid_physical_size, P->d.SINHW, P->Nx[0],
-                         (long)P->Nx[0], (long)P->Nx[0] * P->Nx[1], P->Ntot, P->invdxx[0]);
-    else
-      hipLaunchKernelGGL(bc_radiation_lines_kernel, g, b, 0, P->stream, P->d_rad_lines, P->n_rad_lines, P->ngfs,
-                         P->NG, gfs, rhs, P->d_xx0, P->d_wavespeed, P->d_finf, st, R, P->d.coord,
-                         P->d.grid_physical_size, P->d.SINHW, P->Nx[0], (long)P->Nx[0], (long)P->Nx[0] * P->Nx[1],
-                         P->Ntot, P->invdxx[0]);
+    const unsigned nt = rad_threads(items);
+    const dim3 g((unsigned)((items + nt - 1) / nt));
+    const RadLine W = rad_line_weights(st, R);
+#define RAD_LAUNCH(NG_, R_)                                                                                          \
+  if (P->NG == NG_ && R == R_)                                                                                       \
+    hipLaunchKernelGGL((bc_radiation_lines_kernel<NG_, R_>), g, dim3(nt), 0, P->stream, P->d_rad_lines,              \
+                       P->n_rad_lines, P->ngfs, gfs, rhs, P->d_rad, P->d_wavespeed, P->d_finf, W, P->Nx[0],          \
+                       (long)P->Nx[0], (long)P->Nx[0] * P->Nx[1], P->Ntot, P->invdxx[0])
+    RAD_LAUNCH(3, 1);
+    RAD_LAUNCH(3, 2);
+    RAD_LAUNCH(3, 3);
+    RAD_LAUNCH(4, 1);
+    RAD_LAUNCH(4, 2);
+    RAD_LAUNCH(4, 3);
+#undef RAD_LAUNCH
     HIP_TRY(hipGetLastError());
     return BHAH_OK;
   }
@@ -1949,11 +1931,7 @@ static int enqueue_step(bhah_patch *P, bhah_MoL_gridfunctions *gf, double dt) {
   }
   // BSSN: Ricci -> RHS -> radiation/extrapolation + inner BCs on RHS -> RK update + det(gammabar)
   // enforcement in one pass (two_blackholes_collide.py:290-313).
-  const uintptr_t al = reinterpret_cast<uintptr_t>(gf->y_n_gfs) | reinterpret_cast<uintptr_t>(gf->k_odd_gfs) |
-                       reinterpret_cast<uintptr_t>(gf->k_even_gfs) |
-                       reinterpret_cast<uintptr_t>(gf->y_nplus1_running_total_gfs);
-  if (P->d.outer_bc == BHAH_OUTER_BC_RADIATION && P->fold_inner && P->k->rk_det_inner && P->d_inner_pairs &&
-      !(P->Ntot & 1) && !(al & 15)) {
+  if (P->d.outer_bc == BHAH_OUTER_BC_RADIATION && P->fold_inner && P->d_inner_map) {
     // The inner copy of k rides in the RK pass, which gathers k at each inner ghost point from
     // its source: k stays in k_even and every stage goes to k_odd, so the pass never writes
     // the array it gathers from.  The same values reach every array as with the separate copy.
@@ -1964,7 +1942,7 @@ static int enqueue_step(bhah_patch *P, bhah_MoL_gridfunctions *gf, double dt) {
       if ((rc = bhah_hip_rhs_eval(P, gf->auxevol_gfs, in, k))) return rc;
       if ((rc = apply_bcs_outerradiation(P, in, k))) return rc;
       HIP_TRY(P->k->rk_det_inner(P->stream, k, gf->y_n_gfs, gf->y_nplus1_running_total_gfs, next, P->d_rfm0,
-                                 P->d_rfm1, P->kp(dt, s), P->d_inner_pairs, P->d_gf_parity));
+                                 P->d_rfm1, P->kp(dt, s), P->d_inner_map, P->d_inner_pairs));
     }
     return BHAH_OK;
   }
@@ -1975,10 +1953,8 @@ static int enqueue_step(bhah_patch *P, bhah_MoL_gridfunctions *gf, double dt) {
     if (P->d.outer_bc == BHAH_OUTER_BC_RADIATION) {
       if ((rc = bhah_hip_apply_bcs_outerradiation_and_inner(P, in, k))) return rc;
     }
-    dim3 g, b;
-    P->all_dims(g, b);
     double *next = (s == 4) ? gf->y_n_gfs : k;
-    HIP_TRY(P->k->rk_det(g, b, P->stream, k, gf->y_n_gfs, gf->y_nplus1_running_total_gfs, next, P->d_rfm0, P->d_rfm1,
+    HIP_TRY(P->k->rk_det(P->stream, k, gf->y_n_gfs, gf->y_nplus1_running_total_gfs, next, P->d_rfm0, P->d_rfm1,
                          P->kp(dt, s)));
     if (P->d.outer_bc == BHAH_OUTER_BC_EXTRAPOLATION) {
       // post-RHS extrapolation BCs then det enforcement (two_blackholes_collide.py:304-307)
@@ -2360,8 +2336,6 @@ static long tape_doubles(const bhah_patch *P) { return (8L * P->ngfs + 4L * 6) *
 // writes y_{n+1} there, as the MoL step writes it into y_n.
 static int enqueue_stages(bhah_patch *P, const StepTape &T, double *yrun, double dt, double *y_next) {
   const long N = P->Ntot, nv = N * P->ngfs;
-  dim3 ga, ba;
-  P->all_dims(ga, ba);
   int rc;
   for (int s = 1; s <= 4; s++) {
     double *in = T.Y[s - 1], *k = T.K + (s - 1) * nv, *aux = T.AUX + (s - 1) * 6 * N;
@@ -2369,9 +2343,9 @@ static int enqueue_stages(bhah_patch *P, const StepTape &T, double *yrun, double
     if ((rc = bhah_hip_rhs_eval(P, aux, in, k))) return rc;
     if ((rc = bhah_hip_apply_bcs_outerradiation_and_inner(P, in, k))) return rc;
     if (s < 4)
-      HIP_TRY(P->k->rk_det(ga, ba, P->stream, k, T.Y[0], yrun, T.Y[s], P->d_rfm0, P->d_rfm1, P->kp(dt, s)));
+      HIP_TRY(P->k->rk_det(P->stream, k, T.Y[0], yrun, T.Y[s], P->d_rfm0, P->d_rfm1, P->kp(dt, s)));
     else if (y_next)
-      HIP_TRY(P->k->rk_det(ga, ba, P->stream, k, T.Y[0], yrun, y_next, P->d_rfm0, P->d_rfm1, P->kp(dt, s)));
+      HIP_TRY(P->k->rk_det(P->stream, k, T.Y[0], yrun, y_next, P->d_rfm0, P->d_rfm1, P->kp(dt, s)));
   }
   return BHAH_OK;
 }
@@ -2543,13 +2517,10 @@ struct bhah_ensemble {
   bhah_item *d_lds[2] = {};
   int n_lds[2] = {};
   bool aligned16 = true;  // every bound stage array 16-byte aligned (schedules with pair loads need it)
-  ens_outer_pt *d_outer[8] = {};
-  int n_outer[8] = {};
-  ens_inner_pt *d_inner = nullptr;
-  int n_inner = 0;
+  ens_rad_line *d_lines = nullptr;  // radial lines of the outer boundary points, all members
+  int n_lines = 0;
   double *d_wavespeed = nullptr, *d_finf = nullptr;
-  int *d_gf_parity = nullptr;
-  RadStencil st;
+  RadLine W;
   int R = 2;
   int rhs_choice = 0, ricci_choice = 0;
   int tile_x = 64, tile_y = 4, max_wg = 0;
@@ -2563,6 +2534,12 @@ struct bhah_ensemble {
       graph_exec = nullptr;
     }
   }
+  // points per thread of the RK pass: 2 where every member's arrays allow 16-byte accesses
+  int np() const {
+    for (const bhah_patch *q : P)
+      if (q->Ntot & 1) return 1;
+    return aligned16 ? 2 : 1;
+  }
   dim3 grid_for(int nitems) const {
     const int g = (max_wg > 0 && max_wg < nitems) ? max_wg : nitems;
     return dim3(g > 0 ? g : 1);
@@ -2572,8 +2549,8 @@ struct bhah_ensemble {
 namespace {
 
 // Tile lists: interior tiles (tile_x x tile_y threads over (i0, i1), one xx2 plane each)
-// and, for the RK pass, chunks of 256 consecutive points of each member's arrays, all members
-// concatenated.
+// and, for the RK pass, chunks of 256 consecutive points (pairs of points where the pass takes
+// pairs) of each member's arrays, all members concatenated.
 int ensemble_build_items(bhah_ensemble *E) {
   std::vector<bhah_item> in, all;
   for (int m = 0; m < (int)E->P.size(); m++) {
@@ -2582,7 +2559,8 @@ int ensemble_build_items(bhah_ensemble *E) {
     for (int bz = 0; bz < n2; bz++)
       for (int by = 0; by < (n1 + E->tile_y - 1) / E->tile_y; by++)
         for (int bx = 0; bx < (n0 + E->tile_x - 1) / E->tile_x; bx++) in.push_back({m, bx, by, bz});
-    for (long c = 0; c < (P->Ntot + 255) / 256; c++) all.push_back({m, (int)c, 0, 0});
+    const long units = P->Ntot / E->np();
+    for (long c = 0; c < (units + 255) / 256; c++) all.push_back({m, (int)c, 0, 0});
   }
   hipFree(E->d_int);
   hipFree(E->d_all);
@@ -2623,7 +2601,6 @@ int ensemble_build_lds_items(bhah_ensemble *E, int kind) {
 }
 
 int ensemble_enqueue_step(bhah_ensemble *E) {
-  const int in_s[4] = {0, 2, 3, 2}, k_s[4] = {2, 3, 2, 3};
   const BssnCandidate &ric = E->k->ricci[E->ricci_choice], &rhs = E->k->rhs[E->rhs_choice];
   const dim3 tb(E->tile_x, E->tile_y, 1);
   if (!E->aligned16 && (pair_loads(ric.name) || pair_loads(rhs.name)))
@@ -2632,25 +2609,27 @@ int ensemble_enqueue_step(bhah_ensemble *E) {
   const bhah_item *ric_items = ric.lds[0] ? E->d_lds[1] : E->d_int, *rhs_items = rhs.lds[0] ? E->d_lds[0] : E->d_int;
   const int ric_n = ric.lds[0] ? E->n_lds[1] : E->n_int, rhs_n = rhs.lds[0] ? E->n_lds[0] : E->n_int;
   for (int s = 1; s <= 4; s++) {
-    const int in = in_s[s - 1], k = k_s[s - 1], out = (s == 4) ? 0 : k;
+    const int in = (s == 1) ? 0 : 2, k = 3, out = (s == 4) ? 0 : 2;
     HIP_TRY(ric.ens(E->grid_for(ric_n), tb, E->stream, E->d_mem, ric_items, ric_n, in, 4, 4));
     HIP_TRY(rhs.ens(E->grid_for(rhs_n), tb, E->stream, E->d_mem, rhs_items, rhs_n, in, 4, k));
-    for (int gz = 0; gz < E->NG; gz++) {
-      if (!E->n_outer[gz]) continue;
-      dim3 g, b;
-      launch_1d((long)E->n_outer[gz] * BHAH_NUM_EVOL_GFS_BSSN, g, b);
-      hipLaunchKernelGGL(ens_bc_radiation_kernel, g, b, 0, E->stream, E->d_mem, E->d_outer[gz], E->n_outer[gz],
-                         BHAH_NUM_EVOL_GFS_BSSN, in, k, E->d_wavespeed, E->d_finf, E->st, E->R);
-      HIP_TRY(hipGetLastError());
-    }
-    if (E->n_inner) {
-      dim3 g, b;
-      launch_1d((long)E->n_inner, g, b);
-      hipLaunchKernelGGL(ens_bc_inner_kernel, g, b, 0, E->stream, E->d_mem, E->d_inner, E->n_inner,
-                         BHAH_NUM_EVOL_GFS_BSSN, E->d_gf_parity, k);
-      HIP_TRY(hipGetLastError());
-    }
-    HIP_TRY(E->k->ens_rk_det(E->grid_for(E->n_all), dim3(256, 1, 1), E->stream, E->d_mem, E->d_all, E->n_all, k, out, s));
+    const long items = (long)E->n_lines * BHAH_NUM_EVOL_GFS_BSSN;
+    const unsigned nt = rad_threads(items);
+    const dim3 rg((unsigned)((items + nt - 1) / nt));
+#define RAD_LAUNCH(NG_, R_)                                                                                          \
+  if (E->NG == NG_ && E->R == R_)                                                                                    \
+    hipLaunchKernelGGL((ens_bc_radiation_lines_kernel<NG_, R_>), rg, dim3(nt), 0, E->stream, E->d_mem, E->d_lines,   \
+                       E->n_lines, BHAH_NUM_EVOL_GFS_BSSN, in, k, E->d_wavespeed, E->d_finf, E->W)
+    RAD_LAUNCH(3, 1);
+    RAD_LAUNCH(3, 2);
+    RAD_LAUNCH(3, 3);
+    RAD_LAUNCH(4, 1);
+    RAD_LAUNCH(4, 2);
+    RAD_LAUNCH(4, 3);
+#undef RAD_LAUNCH
+    HIP_TRY(hipGetLastError());
+    // the RK pass takes the inner-parity condition of k with it, as the single-patch step does
+    HIP_TRY(E->k->ens_rk_det(E->grid_for(4 * E->n_all), E->stream, E->d_mem, E->d_all, E->n_all, k, out, s,
+                               E->np()));
   }
   return BHAH_OK;
 }
@@ -2683,6 +2662,10 @@ int bhah_hip_ensemble_create(const bhah_patch_desc *descs, int n, bhah_ensemble 
       bhah_hip_ensemble_destroy(E);
       return fail(BHAH_ERR_ARG, "member %d uses a different kernel build than member 0", m);
     }
+    if (!P->d_inner_map) {  // the batched RK pass takes the inner condition through it
+      bhah_hip_ensemble_destroy(E);
+      return fail(BHAH_ERR_UNSUPPORTED, "member %d has no inner boundary points", m);
+    }
   }
   if (!E->k->ens_rk_det || !E->k->rhs[0].ens) {
     bhah_hip_ensemble_destroy(E);
@@ -2693,45 +2676,35 @@ int bhah_hip_ensemble_create(const bhah_patch_desc *descs, int n, bhah_ensemble 
     bhah_hip_ensemble_destroy(E);
     return fail(BHAH_ERR_ARG, "radiation_bc_fd_order must be 2, 4 or 6");
   }
-  rad_stencil(E->R, E->st);
-  // concatenated boundary records
-  std::vector<ens_inner_pt> inner;
-  std::vector<ens_outer_pt> outer[8];
+  RadStencil st;
+  rad_stencil(E->R, st);
+  E->W = rad_line_weights(st, E->R);
+  std::vector<ens_rad_line> lines;  // of all members
   for (int m = 0; m < n; m++) {
     const bhah_patch *P = E->P[m];
-    for (size_t p = 0; p < P->inner_dst.size(); p++) {
-      unsigned mk = 0;
-      for (int t = 0; t < 10; t++)
-        if (P->inner_parity[10 * p + t] < 0) mk |= 1u << t;
-      inner.push_back({m, (int)P->inner_dst[p], (int)P->inner_src[p], mk});
+    if (!P->n_rad_lines || !rad_lines_fit(P->Nx[0], P->NG, E->R)) {
+      bhah_hip_ensemble_destroy(E);
+      return fail(BHAH_ERR_UNSUPPORTED, "member %d: its outer points are not radial lines of %d points", m,
+                  P->NG + E->R + 2);
     }
-    for (int gz = 0; gz < E->NG; gz++)
-      for (int d = 0; d < 3; d++)
-        for (size_t q = 0; q < P->outer[gz][d].size(); q += 6) {
-          ens_outer_pt e;
-          e.m = m;
-          for (int j = 0; j < 6; j++) e.q[j] = P->outer[gz][d][q + j];
-          outer[gz].push_back(e);
-        }
+    for (size_t q = 0; q < P->outer[0][0].size(); q += 6) {
+      const int16_t *o = &P->outer[0][0][q];
+      lines.push_back({m, P->Nx[0] * (o[1] + P->Nx[1] * o[2])});
+    }
   }
   std::vector<double> ws(24, 1.0), fi(24, 0.0);
   ws[6] = sqrt(2.0);
   fi[6] = 1.0;
   fi[10] = 1.0;
-  std::vector<int> par(kBssnParity, kBssnParity + 24);
-  if ((rc = upload(inner, &E->d_inner)) || (rc = upload(ws, &E->d_wavespeed)) || (rc = upload(fi, &E->d_finf)) ||
-      (rc = upload(par, &E->d_gf_parity))) {
+  if ((rc = upload(ws, &E->d_wavespeed)) || (rc = upload(fi, &E->d_finf))) {
     bhah_hip_ensemble_destroy(E);
     return rc;
   }
-  E->n_inner = (int)inner.size();
-  for (int gz = 0; gz < E->NG; gz++) {
-    if ((rc = upload(outer[gz], &E->d_outer[gz]))) {
-      bhah_hip_ensemble_destroy(E);
-      return rc;
-    }
-    E->n_outer[gz] = (int)outer[gz].size();
+  if ((rc = upload(lines, &E->d_lines))) {
+    bhah_hip_ensemble_destroy(E);
+    return rc;
   }
+  E->n_lines = (int)lines.size();
   if ((rc = ensemble_build_items(E))) {
     bhah_hip_ensemble_destroy(E);
     return rc;
@@ -2754,11 +2727,9 @@ int bhah_hip_ensemble_destroy(bhah_ensemble *E) {
   hipFree(E->d_all);
   hipFree(E->d_lds[0]);
   hipFree(E->d_lds[1]);
-  for (int gz = 0; gz < 8; gz++) hipFree(E->d_outer[gz]);
-  hipFree(E->d_inner);
+  hipFree(E->d_lines);
   hipFree(E->d_wavespeed);
   hipFree(E->d_finf);
-  hipFree(E->d_gf_parity);
   delete E;
   return BHAH_OK;
 }
@@ -2787,6 +2758,9 @@ int bhah_hip_ensemble_bind(bhah_ensemble *E, const bhah_MoL_gridfunctions *gfs, 
     M.rfm0 = P->d_rfm0;
     M.rfm1 = P->d_rfm1;
     M.xx0 = P->d_xx0;
+    M.rad = P->d_rad;
+    M.inner_map = P->d_inner_map;
+    M.inner_pairs = P->d_inner_pairs;
     M.arr[0] = g.y_n_gfs;
     M.arr[1] = g.y_nplus1_running_total_gfs;
     M.arr[2] = g.k_odd_gfs;
@@ -2801,7 +2775,7 @@ int bhah_hip_ensemble_bind(bhah_ensemble *E, const bhah_MoL_gridfunctions *gfs, 
   HIP_TRY(hipMemcpy(E->d_mem, E->hmem.data(), sizeof(bhah_member) * E->hmem.size(), hipMemcpyHostToDevice));
   E->bound = true;
   E->invalidate_graph();
-  return BHAH_OK;
+  return ensemble_build_items(E);  // the RK pass's units depend on the arrays' alignment
 }
 
 int bhah_hip_ensemble_set_stream(bhah_ensemble *E, void *s) {

@@ -7,233 +7,175 @@
 #define Rational_1_2 (1.0 / 2.0)
 #define Rational_2_3 (2.0 / 3.0)
 
-extern "C" __global__ void __launch_bounds__(256)
-bssn_rk_det_SinhSpherical_symnone_KO1_fd4(const double *__restrict__ kin, const double *y_n, double *__restrict__ y_run, double *out,
-                  const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p) {
-  const long Ntot = p.Ntot;
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= Ntot) return;
-  const int i0 = (int)(idx % p.Nx0), i1 = (int)((idx / p.Nx0) % p.Nx1);
-  constexpr int NGF = 24;
-  double kk[NGF], ctr[NGF];
-#pragma unroll
-  for (int g = 0; g < NGF; g++) {
-    kk[g] = __builtin_nontemporal_load(&kin[g * Ntot + idx]);
-    ctr[g] = (p.substep == 1) ? __builtin_nontemporal_load(&y_n[g * Ntot + idx]) : 0.0;
-  }
-
-  // RK4 substep update (register_all_MoL_step_forward_in_time.c:4-103), in registers.
-  const double dt = p.dt;
-  double nxt[NGF];
-  if (p.substep == 1) {
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {
-      const double k = kk[g];
-      __builtin_nontemporal_store((1.0 / 6.0) * dt * k, &y_run[g * Ntot + idx]);
-      nxt[g] = (1.0 / 2.0) * dt * k + ctr[g];
-    }
-  } else if (p.substep == 4) {
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {
-      const double k = kk[g];
-      nxt[g] = (1.0 / 6.0) * dt * k + __builtin_nontemporal_load(&y_n[g * Ntot + idx]) + __builtin_nontemporal_load(&y_run[g * Ntot + idx]);
-    }
-  } else {
-    const double a = (p.substep == 2) ? (1.0 / 2.0) : 1.0;
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {
-      const double k = kk[g];
-      __builtin_nontemporal_store((1.0 / 3.0) * dt * k + __builtin_nontemporal_load(&y_run[g * Ntot + idx]), &y_run[g * Ntot + idx]);
-      nxt[g] = a * dt * k + __builtin_nontemporal_load(&y_n[g * Ntot + idx]);
-    }
-  }
-
-  {
-    const double hDD00 = nxt[11];
-    const double hDD01 = nxt[12];
-    const double hDD02 = nxt[13];
-    const double hDD11 = nxt[14];
-    const double hDD12 = nxt[15];
-    const double hDD22 = nxt[16];
-    const double f0_of_xx0 = rfm0[i0];
-    const double f0_of_xx0__D0 = rfm0[p.Nx0 + i0];
-    const double f1_of_xx1 = rfm1[i1];
-    const double dg0 = (f0_of_xx0*f0_of_xx0);
-    const double dg1 = dg0*hDD11 + dg0;
-    const double dg2 = (f0_of_xx0__D0*f0_of_xx0__D0);
-    const double dg3 = dg2*hDD00 + dg2;
-    const double dg4 = (f1_of_xx1*f1_of_xx1);
-    const double dg5 = dg0*dg4;
-    const double dg6 = dg5*hDD22 + dg5;
-    const double dg7 = (f0_of_xx0*f0_of_xx0*f0_of_xx0*f0_of_xx0);
-    const double dg8 = dg4*dg7;
-    const double dg9 = cbrt(fabs(dg2*dg8)/(-dg0*dg2*dg6*(hDD01*hDD01) - dg1*dg2*dg5*(hDD02*hDD02) + dg1*dg3*dg6 + 2.0*dg2*dg4*dg7*hDD01*hDD02*hDD12 - dg3*dg8*(hDD12*hDD12)));
-    const double new_hDD00 = dg9*(hDD00 + 1.0) - 1.0;
-    const double new_hDD01 = dg9*hDD01;
-    const double new_hDD02 = dg9*hDD02;
-    const double new_hDD11 = dg9*(hDD11 + 1.0) - 1.0;
-    const double new_hDD12 = dg9*hDD12;
-    const double new_hDD22 = dg9*(hDD22 + 1.0) - 1.0;
-    nxt[11] = new_hDD00;
-    nxt[12] = new_hDD01;
-    nxt[13] = new_hDD02;
-    nxt[14] = new_hDD11;
-    nxt[15] = new_hDD12;
-    nxt[16] = new_hDD22;
-  }
-#pragma unroll
-  for (int g = 0; g < NGF; g++) __builtin_nontemporal_store(nxt[g], &out[g * Ntot + idx]);
-}
-
 typedef double bhah_d2 __attribute__((ext_vector_type(2)));
-extern "C" __global__ void __launch_bounds__(256)
-bssn_rk_det2_SinhSpherical_symnone_KO1_fd4(const double *__restrict__ kin, const double *y_n, double *__restrict__ y_run, double *out,
-                   const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p) {
-  const long Ntot = p.Ntot;
-  const long idx2 = ((long)blockIdx.x * 256 + threadIdx.x) * 2;
-  if (idx2 >= Ntot) return;
-  constexpr int NGF = 24;
-  const bhah_d2 *K2 = (const bhah_d2 *)(kin + idx2), *YN2 = (const bhah_d2 *)(y_n + idx2);
-  bhah_d2 *YR2 = (bhah_d2 *)(y_run + idx2), *OUT2 = (bhah_d2 *)(out + idx2);
-  const long S2 = Ntot / 2;  // gridfunction stride in pairs
-  // RK4 substep update (register_all_MoL_step_forward_in_time.c:4-103), in registers.
-  const double dt = p.dt;
-  bhah_d2 nx2[NGF];
-  if (p.substep == 1) {
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {
-      const bhah_d2 k = __builtin_nontemporal_load(&K2[g * S2]);
-      __builtin_nontemporal_store((1.0 / 6.0) * dt * k, &YR2[g * S2]);
-      nx2[g] = (1.0 / 2.0) * dt * k + __builtin_nontemporal_load(&YN2[g * S2]);
-    }
-  } else if (p.substep == 4) {
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {
-      const bhah_d2 k = __builtin_nontemporal_load(&K2[g * S2]);
-      nx2[g] = (1.0 / 6.0) * dt * k + __builtin_nontemporal_load(&YN2[g * S2]) + __builtin_nontemporal_load(&YR2[g * S2]);
-    }
-  } else {
-    const double a = (p.substep == 2) ? (1.0 / 2.0) : 1.0;
-#pragma unroll
-    for (int g = 0; g < NGF; g++) {
-      const bhah_d2 k = __builtin_nontemporal_load(&K2[g * S2]);
-      __builtin_nontemporal_store((1.0 / 3.0) * dt * k + __builtin_nontemporal_load(&YR2[g * S2]), &YR2[g * S2]);
-      nx2[g] = a * dt * k + __builtin_nontemporal_load(&YN2[g * S2]);
-    }
-  }
-#pragma unroll
-  for (int h = 0; h < 2; h++) {
-    const long idx = idx2 + h;
-    const int i0 = (int)(idx % p.Nx0), i1 = (int)((idx / p.Nx0) % p.Nx1);
-    double nxt[NGF];
-#pragma unroll
-    for (int g = 0; g < NGF; g++) nxt[g] = nx2[g][h];
-  {
-    const double hDD00 = nxt[11];
-    const double hDD01 = nxt[12];
-    const double hDD02 = nxt[13];
-    const double hDD11 = nxt[14];
-    const double hDD12 = nxt[15];
-    const double hDD22 = nxt[16];
-    const double f0_of_xx0 = rfm0[i0];
-    const double f0_of_xx0__D0 = rfm0[p.Nx0 + i0];
-    const double f1_of_xx1 = rfm1[i1];
-    const double dg0 = (f0_of_xx0*f0_of_xx0);
-    const double dg1 = dg0*hDD11 + dg0;
-    const double dg2 = (f0_of_xx0__D0*f0_of_xx0__D0);
-    const double dg3 = dg2*hDD00 + dg2;
-    const double dg4 = (f1_of_xx1*f1_of_xx1);
-    const double dg5 = dg0*dg4;
-    const double dg6 = dg5*hDD22 + dg5;
-    const double dg7 = (f0_of_xx0*f0_of_xx0*f0_of_xx0*f0_of_xx0);
-    const double dg8 = dg4*dg7;
-    const double dg9 = cbrt(fabs(dg2*dg8)/(-dg0*dg2*dg6*(hDD01*hDD01) - dg1*dg2*dg5*(hDD02*hDD02) + dg1*dg3*dg6 + 2.0*dg2*dg4*dg7*hDD01*hDD02*hDD12 - dg3*dg8*(hDD12*hDD12)));
-    const double new_hDD00 = dg9*(hDD00 + 1.0) - 1.0;
-    const double new_hDD01 = dg9*hDD01;
-    const double new_hDD02 = dg9*hDD02;
-    const double new_hDD11 = dg9*(hDD11 + 1.0) - 1.0;
-    const double new_hDD12 = dg9*hDD12;
-    const double new_hDD22 = dg9*(hDD22 + 1.0) - 1.0;
-    nxt[11] = new_hDD00;
-    nxt[12] = new_hDD01;
-    nxt[13] = new_hDD02;
-    nxt[14] = new_hDD11;
-    nxt[15] = new_hDD12;
-    nxt[16] = new_hDD22;
-  }
-#pragma unroll
-    for (int g = 0; g < NGF; g++) nx2[g][h] = nxt[g];
-  }
-#pragma unroll
-  for (int g = 0; g < NGF; g++) __builtin_nontemporal_store(nx2[g], &OUT2[g * S2]);
+namespace rk_SinhSpherical_symnone_KO1_fd4 {
+constexpr int PAR[24] = {4, 5, 6, 7, 8, 9, 0, 1, 2, 3, 0, 4, 5, 6, 7, 8, 9, 1, 2, 3, 0, 1, 2, 3};
+// gridfunction j of group G
+constexpr __host__ __device__ int gf(int G, int j) {
+  return G == 0 ? 11 + j : G == 1 ? j : G == 2 ? (j < 5 ? 6 + j : 17) : 18 + j;
 }
-
-extern "C" __global__ void __launch_bounds__(256)
-bssn_rk_deti2_SinhSpherical_symnone_KO1_fd4(const double *__restrict__ kin, const double *y_n, double *__restrict__ y_run, double *out,
-                    const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p,
-                    const int2 *__restrict__ pmap, const int *__restrict__ gfpar) {
-  const long Ntot = p.Ntot;
-  const long q = (long)blockIdx.x * 256 + threadIdx.x;  // pair index
-  const long idx2 = q * 2;
-  if (idx2 >= Ntot) return;
-  constexpr int NGF = 24;
-  const bhah_d2 *K2 = (const bhah_d2 *)kin, *YN2 = (const bhah_d2 *)(y_n + idx2);
-  bhah_d2 *YR2 = (bhah_d2 *)(y_run + idx2), *OUT2 = (bhah_d2 *)(out + idx2);
-  const long S2 = Ntot / 2;  // gridfunction stride in pairs
-  // source pair; code bit 0 / bit 1: point 0 / point 1 takes the source pair's second value;
-  // bits 4-15 / 16-27: the parity-type masks of points 0 / 1 (bit t set: type t flips sign)
-  const int2 pm = pmap[q];
-  const long sp = pm.x;
-  const unsigned code = (unsigned)pm.y;
-#define BHAH_KPAIR(g)                                                                               \
-  ({                                                                                               \
-    const bhah_d2 v_ = __builtin_nontemporal_load(&K2[(g) * S2 + sp]);                              \
-    const unsigned par_ = (unsigned)gfpar[g];                                                       \
-    const double a_ = (code & 1u) ? v_.y : v_.x, b_ = (code & 2u) ? v_.y : v_.x;                    \
-    bhah_d2 k_;                                                                                     \
-    k_.x = ((code >> (4 + par_)) & 1u) ? -a_ : a_;                                                  \
-    k_.y = ((code >> (16 + par_)) & 1u) ? -b_ : b_;                                                 \
-    k_;                                                                                             \
-  })
-  const double dt = p.dt;
-  bhah_d2 nx2[NGF];
-  if (p.substep == 1) {
+// NP consecutive values; NT: with the non-temporal hint
+template <int NP>
+struct Vec;
+template <>
+struct Vec<1> {
+  double v[1];
+  template <bool NT>
+  static __device__ __forceinline__ Vec ld(const double *q) {
+    return {{NT ? __builtin_nontemporal_load(q) : *q}};
+  }
+  template <bool NT>
+  __device__ __forceinline__ void st(double *q) const {
+    if (NT) __builtin_nontemporal_store(v[0], q);
+    else *q = v[0];
+  }
+};
+template <>
+struct Vec<2> {
+  double v[2];
+  template <bool NT>
+  static __device__ __forceinline__ Vec ld(const double *q) {
+    const bhah_d2 t = NT ? __builtin_nontemporal_load((const bhah_d2 *)q) : *(const bhah_d2 *)q;
+    return {{t.x, t.y}};
+  }
+  template <bool NT>
+  __device__ __forceinline__ void st(double *q) const {
+    bhah_d2 t;
+    t.x = v[0];
+    t.y = v[1];
+    if (NT) __builtin_nontemporal_store(t, (bhah_d2 *)q);
+    else *(bhah_d2 *)q = t;
+  }
+};
+// Where this thread's points find the right-hand side: a point or an aligned pair (from, code), or,
+// for a pair whose sources are apart, two points with their parity masks.
+struct Source {
+  long from, s0, s1;
+  unsigned code, m0, m1;
+  bool split, ghost;  // ghost: every point of this thread is an inner ghost point
+};
+template <int NP>
+__device__ __forceinline__ Source find_source(const int2 *map, const int2 *pairs, long q) {
+  Source S;
+  const int2 m = (NP == 2) ? pairs[q] : map[q];
+  S.split = NP == 2 && m.y < 0;
+  S.code = (unsigned)m.y;
+  S.from = (long)m.x * NP;
+  S.s0 = S.s1 = 0;
+  S.m0 = S.m1 = 0;
+  S.ghost = S.from != q * NP;
+  if (S.split) {
+    const int4 t = ((const int4 *)map)[q];
+    S.s0 = t.x;
+    S.m0 = (unsigned)t.y;
+    S.s1 = t.z;
+    S.m1 = (unsigned)t.w;
+    S.ghost = S.s0 != 2 * q && S.s1 != 2 * q + 1;
+  }
+  return S;
+}
+// The six gridfunctions of group G of f at this thread's sources, with their parity signs.
+template <int G, int NP, bool NT>
+__device__ __forceinline__ void at_source(Vec<NP> (&r)[6], const double *f, const long Ntot, const Source &S) {
+  if (NP == 2 && S.split) {
 #pragma unroll
-    for (int g = 0; g < NGF; g++) {
-      const bhah_d2 k = BHAH_KPAIR(g);
-      __builtin_nontemporal_store((1.0 / 6.0) * dt * k, &YR2[g * S2]);
-      nx2[g] = (1.0 / 2.0) * dt * k + __builtin_nontemporal_load(&YN2[g * S2]);
+    for (int j = 0; j < 6; j++) {
+      r[j].v[0] = f[gf(G, j) * Ntot + S.s0];
+      r[j].v[NP - 1] = f[gf(G, j) * Ntot + S.s1];
     }
-  } else if (p.substep == 4) {
 #pragma unroll
-    for (int g = 0; g < NGF; g++) {
-      const bhah_d2 k = BHAH_KPAIR(g);
-      nx2[g] = (1.0 / 6.0) * dt * k + __builtin_nontemporal_load(&YN2[g * S2]) + __builtin_nontemporal_load(&YR2[g * S2]);
+    for (int j = 0; j < 6; j++) {
+      r[j].v[0] = ((S.m0 >> PAR[gf(G, j)]) & 1u) ? -r[j].v[0] : r[j].v[0];
+      r[j].v[NP - 1] = ((S.m1 >> PAR[gf(G, j)]) & 1u) ? -r[j].v[NP - 1] : r[j].v[NP - 1];
     }
-  } else {
-    const double a = (p.substep == 2) ? (1.0 / 2.0) : 1.0;
+    return;
+  }
 #pragma unroll
-    for (int g = 0; g < NGF; g++) {
-      const bhah_d2 k = BHAH_KPAIR(g);
-      __builtin_nontemporal_store((1.0 / 3.0) * dt * k + __builtin_nontemporal_load(&YR2[g * S2]), &YR2[g * S2]);
-      nx2[g] = a * dt * k + __builtin_nontemporal_load(&YN2[g * S2]);
+  for (int j = 0; j < 6; j++) r[j] = Vec<NP>::template ld<NT>(f + gf(G, j) * Ntot + S.from);
+#pragma unroll
+  for (int j = 0; j < 6; j++) {
+    const int t = PAR[gf(G, j)];
+    if (NP == 1) {
+      r[j].v[0] = ((S.code >> t) & 1u) ? -r[j].v[0] : r[j].v[0];
+    } else {
+      const double a = (S.code & 1u) ? r[j].v[NP - 1] : r[j].v[0], b = (S.code & 2u) ? r[j].v[NP - 1] : r[j].v[0];
+      r[j].v[0] = ((S.code >> (4 + t)) & 1u) ? -a : a;
+      r[j].v[NP - 1] = ((S.code >> (16 + t)) & 1u) ? -b : b;
     }
   }
-#undef BHAH_KPAIR
+}
+template <int G, int NP, bool INNER, bool NT>
+__device__ __forceinline__ void group(const double *__restrict__ kin, const double *y_n, double *y_run, double *out,
+                                      const double *__restrict__ rfm0, const double *__restrict__ rfm1,
+                                      const bhah_kparams &p, const int2 *__restrict__ map,
+                                      const int2 *__restrict__ pairs, const long q) {
+  const long Ntot = p.Ntot, idx = q * NP;
+  constexpr int N = 6;
+  const double dt = p.dt;
+  Vec<NP> k[N], y[N], r[N];
+  Source S;
+  S.ghost = false;
+  if (INNER) {
+    S = find_source<NP>(map, pairs, q);
+    at_source<G, NP, NT>(k, kin, Ntot, S);
+  } else {
 #pragma unroll
-  for (int h = 0; h < 2; h++) {
-    const long idx = idx2 + h;
-    const int i0 = (int)(idx % p.Nx0), i1 = (int)((idx / p.Nx0) % p.Nx1);
-    double nxt[NGF];
+    for (int j = 0; j < N; j++) k[j] = Vec<NP>::template ld<NT>(kin + gf(G, j) * Ntot + idx);
+  }
+  const bool ghost = S.ghost;
 #pragma unroll
-    for (int g = 0; g < NGF; g++) nxt[g] = nx2[g][h];
+  for (int j = 0; j < N; j++) y[j] = Vec<NP>::template ld<NT>(y_n + gf(G, j) * Ntot + idx);
+  // RK4 substep update (register_all_MoL_step_forward_in_time.c:4-103), in registers.
+  if (p.substep == 4) {
+    if (INNER && ghost) {
+      at_source<G, NP, true>(r, y_run, Ntot, S);
+    } else {
+#pragma unroll
+      for (int j = 0; j < N; j++) r[j] = Vec<NP>::template ld<true>(y_run + gf(G, j) * Ntot + idx);
+    }
+#pragma unroll
+    for (int j = 0; j < N; j++)
+#pragma unroll
+      for (int e = 0; e < NP; e++) y[j].v[e] = (1.0 / 6.0) * dt * k[j].v[e] + y[j].v[e] + r[j].v[e];
+  } else {
+    if (!ghost) {
+      if (p.substep == 1) {
+#pragma unroll
+        for (int j = 0; j < N; j++)
+#pragma unroll
+          for (int e = 0; e < NP; e++) r[j].v[e] = (1.0 / 6.0) * dt * k[j].v[e];
+      } else {
+#pragma unroll
+        for (int j = 0; j < N; j++) r[j] = Vec<NP>::template ld<true>(y_run + gf(G, j) * Ntot + idx);
+#pragma unroll
+        for (int j = 0; j < N; j++)
+#pragma unroll
+          for (int e = 0; e < NP; e++) r[j].v[e] = (1.0 / 3.0) * dt * k[j].v[e] + r[j].v[e];
+      }
+#pragma unroll
+      for (int j = 0; j < N; j++) r[j].template st<true>(y_run + gf(G, j) * Ntot + idx);
+    }
+    const double a = (p.substep == 3) ? 1.0 : (1.0 / 2.0);
+#pragma unroll
+    for (int j = 0; j < N; j++)
+#pragma unroll
+      for (int e = 0; e < NP; e++) y[j].v[e] = a * dt * k[j].v[e] + y[j].v[e];
+  }
+  if (G == 0) {
+#pragma unroll
+    for (int e = 0; e < NP; e++) {
+      const unsigned long u = (unsigned long)(idx + e), row = u / (unsigned)p.Nx0;
+      const int i0 = (int)(u - row * (unsigned)p.Nx0), i1 = (int)(row % (unsigned)p.Nx1);
+      double nxt[N];
+#pragma unroll
+      for (int j = 0; j < N; j++) nxt[j] = y[j].v[e];
   {
-    const double hDD00 = nxt[11];
-    const double hDD01 = nxt[12];
-    const double hDD02 = nxt[13];
-    const double hDD11 = nxt[14];
-    const double hDD12 = nxt[15];
-    const double hDD22 = nxt[16];
+    const double hDD00 = nxt[0];
+    const double hDD01 = nxt[1];
+    const double hDD02 = nxt[2];
+    const double hDD11 = nxt[3];
+    const double hDD12 = nxt[4];
+    const double hDD22 = nxt[5];
     const double f0_of_xx0 = rfm0[i0];
     const double f0_of_xx0__D0 = rfm0[p.Nx0 + i0];
     const double f1_of_xx1 = rfm1[i1];
@@ -253,18 +195,40 @@ bssn_rk_deti2_SinhSpherical_symnone_KO1_fd4(const double *__restrict__ kin, cons
     const double new_hDD11 = dg9*(hDD11 + 1.0) - 1.0;
     const double new_hDD12 = dg9*hDD12;
     const double new_hDD22 = dg9*(hDD22 + 1.0) - 1.0;
-    nxt[11] = new_hDD00;
-    nxt[12] = new_hDD01;
-    nxt[13] = new_hDD02;
-    nxt[14] = new_hDD11;
-    nxt[15] = new_hDD12;
-    nxt[16] = new_hDD22;
+    nxt[0] = new_hDD00;
+    nxt[1] = new_hDD01;
+    nxt[2] = new_hDD02;
+    nxt[3] = new_hDD11;
+    nxt[4] = new_hDD12;
+    nxt[5] = new_hDD22;
   }
 #pragma unroll
-    for (int g = 0; g < NGF; g++) nx2[g][h] = nxt[g];
+      for (int j = 0; j < N; j++) y[j].v[e] = nxt[j];
+    }
   }
 #pragma unroll
-  for (int g = 0; g < NGF; g++) __builtin_nontemporal_store(nx2[g], &OUT2[g * S2]);
+  for (int j = 0; j < N; j++) y[j].template st<NT>(out + gf(G, j) * Ntot + idx);
+}
+template <int NP, bool INNER, bool NT>
+__device__ __forceinline__ void any_group(int G, const double *__restrict__ kin, const double *y_n, double *y_run,
+                                          double *out, const double *__restrict__ rfm0,
+                                          const double *__restrict__ rfm1, const bhah_kparams &p,
+                                          const int2 *__restrict__ map, const int2 *__restrict__ pairs,
+                                          const long q) {
+  if (q * NP >= p.Ntot) return;
+  if (G == 0) group<0, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+  else if (G == 1) group<1, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+  else if (G == 2) group<2, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+  else group<3, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+}
+}  // namespace rk_SinhSpherical_symnone_KO1_fd4
+template <int NP, bool INNER, bool NT>
+__global__ void __launch_bounds__(256)
+bssn_rk_det_SinhSpherical_symnone_KO1_fd4(const double *__restrict__ kin, const double *y_n, double *y_run, double *out,
+                  const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p,
+                  const int2 *__restrict__ map, const int2 *__restrict__ pairs) {
+  rk_SinhSpherical_symnone_KO1_fd4::any_group<NP, INNER, NT>((int)(blockIdx.x & 3u), kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs,
+                                 (long)(blockIdx.x >> 2) * blockDim.x + threadIdx.x);
 }
 
 extern "C" __global__ void __launch_bounds__(256)
@@ -898,34 +862,50 @@ bssn_initial_lambda_SinhSpherical_symnone_KO1_fd4(double *gfs, const double *__r
 #undef Rational_1_2
 #undef Rational_2_3
 
-// Host-side launchers (one translation unit per variant; no relocatable device code needed).
-extern "C" hipError_t launch_bssn_rk_det_SinhSpherical_symnone_KO1_fd4(dim3 g, dim3 b, hipStream_t s, const double *kin, const double *y_n,
-    double *y_run, double *out, const double *rfm0, const double *rfm1, bhah_kparams p) {
-  (void)g;
-  (void)b;
-  const bool pairs = !(p.Ntot & 1) && !((reinterpret_cast<uintptr_t>(kin) | reinterpret_cast<uintptr_t>(y_n) |
-                                         reinterpret_cast<uintptr_t>(y_run) | reinterpret_cast<uintptr_t>(out)) & 15);
-  if (pairs)
-    hipLaunchKernelGGL(bssn_rk_det2_SinhSpherical_symnone_KO1_fd4, dim3((unsigned)((p.Ntot / 2 + 255) / 256)), dim3(256), 0, s, kin, y_n, y_run,
-                       out, rfm0, rfm1, p);
-  else
-    hipLaunchKernelGGL(bssn_rk_det_SinhSpherical_symnone_KO1_fd4, dim3((unsigned)((p.Ntot + 255) / 256)), dim3(256), 0, s, kin, y_n, y_run,
-                       out, rfm0, rfm1, p);
+static hipError_t rk_det_launch_SinhSpherical_symnone_KO1_fd4(hipStream_t s, const double *kin, const double *y_n, double *y_run, double *out,
+    const double *rfm0, const double *rfm1, const bhah_kparams &p, const int2 *map, const int2 *pairs) {
+  const int np = (!(p.Ntot & 1) && !((reinterpret_cast<uintptr_t>(kin) | reinterpret_cast<uintptr_t>(y_n) |
+                                      reinterpret_cast<uintptr_t>(y_run) | reinterpret_cast<uintptr_t>(out)) & 15))
+                     ? 2
+                     : 1;
+  const long units = p.Ntot / np;
+  // 256 threads a workgroup where that gives every CU several; 64 on small grids
+  const unsigned nt = units >= (1L << 17) ? 256 : 64;
+  const dim3 g(4u * (unsigned)((units + nt - 1) / nt));
+  // The running sum is not read again before the next substep, so it always streams past the
+  // caches.  The other arrays (five stage arrays in all) are read by the next kernels: caching
+  // them gains where a good part of them stays in the 256 MB last-level cache (7229 -> 6947 us
+  // per four steps at 127x63x62 fd6, 0.64 GB; 2297 -> 2003 at 256x64x16, 0.39 GB; 6958 -> 6925
+  // for an ensemble of 1.5 GB) and loses where none does (23493 -> 23839 at 192x96x96, 2.1 GB).
+  const bool nt_all = p.Ntot * (5 * 24 * 8L) > 1800000000L;
+#define RK_LAUNCH(NP_, IN_, NT_)                                                                                     \
+  if (np == NP_ && (map != nullptr) == IN_ && nt_all == NT_)                                                         \
+    hipLaunchKernelGGL((bssn_rk_det_SinhSpherical_symnone_KO1_fd4<NP_, IN_, NT_>), g, dim3(nt), 0, s, kin, y_n, y_run, out, rfm0, rfm1, p,   \
+                       map, pairs)
+  RK_LAUNCH(1, false, false);
+  RK_LAUNCH(1, false, true);
+  RK_LAUNCH(1, true, false);
+  RK_LAUNCH(1, true, true);
+  RK_LAUNCH(2, false, false);
+  RK_LAUNCH(2, false, true);
+  RK_LAUNCH(2, true, false);
+  RK_LAUNCH(2, true, true);
+#undef RK_LAUNCH
   return hipGetLastError();
 }
-// The RK pass with the inner boundary condition folded in: pairs only (even Ntot, 16-byte aligned
-// arrays); a call that does not meet that returns hipErrorInvalidValue and launches nothing.
+extern "C" hipError_t launch_bssn_rk_det_SinhSpherical_symnone_KO1_fd4(hipStream_t s, const double *kin, const double *y_n, double *y_run,
+    double *out, const double *rfm0, const double *rfm1, bhah_kparams p) {
+  return rk_det_launch_SinhSpherical_symnone_KO1_fd4(s, kin, y_n, y_run, out, rfm0, rfm1, p, nullptr, nullptr);
+}
+// The RK pass with the inner boundary condition folded in.
 extern "C" hipError_t launch_bssn_rk_det_inner_SinhSpherical_symnone_KO1_fd4(hipStream_t s, const double *kin, const double *y_n,
-    double *y_run, double *out, const double *rfm0, const double *rfm1, bhah_kparams p, const int *pmap,
-    const int *gfpar) {
-  if ((p.Ntot & 1) || ((reinterpret_cast<uintptr_t>(kin) | reinterpret_cast<uintptr_t>(y_n) |
-                        reinterpret_cast<uintptr_t>(y_run) | reinterpret_cast<uintptr_t>(out) |
-                        reinterpret_cast<uintptr_t>(pmap)) & 15))
-    return hipErrorInvalidValue;
-  hipLaunchKernelGGL(bssn_rk_deti2_SinhSpherical_symnone_KO1_fd4, dim3((unsigned)((p.Ntot / 2 + 255) / 256)), dim3(256), 0, s, kin, y_n, y_run,
-                     out, rfm0, rfm1, p, reinterpret_cast<const int2 *>(pmap), gfpar);
-  return hipGetLastError();
+    double *y_run, double *out, const double *rfm0, const double *rfm1, bhah_kparams p, const int *map,
+    const int *pairs) {
+  return rk_det_launch_SinhSpherical_symnone_KO1_fd4(s, kin, y_n, y_run, out, rfm0, rfm1, p, reinterpret_cast<const int2 *>(map),
+                             reinterpret_cast<const int2 *>(pairs));
 }
+
+// Host-side launchers (one translation unit per variant; no relocatable device code needed).
 extern "C" hipError_t launch_bssn_constraints_SinhSpherical_symnone_KO1_fd4(dim3 g, dim3 b, hipStream_t s, const double *in,
     const double *aux, double *diag, const double *rfm0, const double *rfm1, bhah_kparams p) {
   hipLaunchKernelGGL(bssn_constraints_SinhSpherical_symnone_KO1_fd4, g, b, 0, s, in, aux, diag, rfm0, rfm1, p);
