@@ -701,17 +701,15 @@ KPARAMS = """
 
 XCD_REMAP = """  // Workgroups are dispatched round-robin over the 8 XCDs (each with its own L2):
   // renumber them so XCD k sweeps the k-th contiguous eighth of the tiles and
-  // stencil neighbours share an L2.  Identity when the tile count is not a multiple of 8.
+  // stencil neighbours share an L2.
   unsigned bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
   {
     const unsigned gx = gridDim.x, gy = gridDim.y, n = gx * gy * gridDim.z;
-    if ((n & 7u) == 0u) {
-      const unsigned h = bx + gx * (by + gy * bz);
-      const unsigned l = (h & 7u) * (n >> 3) + (h >> 3);
-      bx = l % gx;
-      by = (l / gx) % gy;
-      bz = l / (gx * gy);
-    }
+    const unsigned h = bx + gx * (by + gy * bz), x = h & 7u, r = n & 7u;
+    const unsigned l = x * (n >> 3) + (x < r ? x : r) + (h >> 3);
+    bx = l % gx;
+    by = (l / gx) % gy;
+    bz = l / (gx * gy);
   }
 """
 
@@ -2128,8 +2126,12 @@ def wave_kernels(fd_order: int) -> str:
     tag = f"fd{fd_order}"
     lv = [f"rhs[{spec.gfs.index(g)} * Ntot + idx]" for g, _ in spec.outputs]
     body = _ordered_body(spec, fd_order, lv, rats)
-    lvk = [f"kk[{spec.gfs.index(g)}]" for g, _ in spec.outputs]
-    bodyk = _ordered_body(spec, fd_order, lvk, rats)
+    w = dict(fd.weights_1d("dDD", fd_order))
+    assert fd_order == 4 and fd.ghost_zones(fd_order, False) == 2
+    lap = " + ".join(f"c2 * uu_dDD{d}{d}" for d in range(3))
+    lines = "".join(
+        f"  const double uu_dDD{d}{d} = p.invdxx{d} * p.invdxx{d} * line<GHOSTS>(in, idx, {st}, u, i{d} - 2, "
+        f"p.Nx{d} - 3 - i{d});\n" for d, st in enumerate(("1", "s1", "s2")))
     consts = "\n".join(f"#define {k} ({v})" for k, v in sorted(rats.items()))
     undefs = "\n".join(f"#undef {k}" for k in sorted(rats))
     return f"""// ---- scalar wave kernels, Cartesian, fd_order={fd_order}
@@ -2140,16 +2142,53 @@ wave_rhs_{tag}(const double *__restrict__ in, double *__restrict__ rhs, const bh
 {body}
 }}
 
-extern "C" __global__ void __launch_bounds__(256)
+// rhs_eval and the RK4 substep update in one pass at interior points.  Ghost values enter only
+// through the five-point lines of uu, and in a stage past the first they are the quadratic
+// extrapolation of the line's own interior points (the boundary condition of every stage), so
+// with GHOSTS false each thread forms them from the values it holds and the stage's ghost zones
+// need not be filled: one boundary launch a step instead of one a stage.  The arithmetic is
+// the boundary kernel's, so the state is the same bit for bit.
+namespace wave_{tag} {{
+// 3 f1 - 3 f2 + f3, as the boundary kernel forms it
+__device__ __forceinline__ double extrapolate(double f1, double f2, double f3) {{
+#pragma clang fp contract(off)
+  return +3.0 * f1 - 3.0 * f2 + 1.0 * f3;
+}}
+// The second-derivative sum along one direction; u: the centre value; lo, hi: interior points
+// below and above (at least three interior points in every direction, checked by the host).
+template <bool GHOSTS>
+__device__ __forceinline__ double line(const double *__restrict__ f, long idx, long s, double u, int lo, int hi) {{
+  double a1 = f[idx + s], a2 = f[idx + 2 * s], b1 = f[idx - s], b2 = f[idx - 2 * s];
+  if (!GHOSTS) {{
+    if (hi == 0) {{
+      a1 = extrapolate(u, b1, b2);
+      a2 = extrapolate(a1, u, b1);
+    }} else if (hi == 1) {{
+      a2 = extrapolate(a1, u, b1);
+    }}
+    if (lo == 0) {{
+      b1 = extrapolate(u, a1, a2);
+      b2 = extrapolate(b1, u, a1);
+    }} else if (lo == 1) {{
+      b2 = extrapolate(b1, u, a1);
+    }}
+  }}
+  return {_dbl(w[0])} * u + {_dbl(w[1])} * (a1 + b1) + {_dbl(w[2])} * (a2 + b2);
+}}
+}}  // namespace wave_{tag}
+template <bool GHOSTS>
+__global__ void __launch_bounds__(256)
 wave_rhs_rk_{tag}(const double *__restrict__ in, const double *y_n, double *__restrict__ y_run,
                   double *out, const bhah_kparams p) {{
-{_prologue(True)}
+  using namespace wave_{tag};
+{_prologue(True, xcd=True)}
   constexpr int NGF = 2;
-  double kk[NGF];
-{bodyk}
-  double ctr[NGF];
-#pragma unroll
-  for (int g = 0; g < NGF; g++) ctr[g] = (p.substep == 1) ? in[g * Ntot + idx] : 0.0;
+  double kk[NGF], ctr[NGF];
+  const double u = in[idx], c2 = p.wavespeed * p.wavespeed;
+  kk[0] = in[Ntot + idx];
+{lines}  kk[1] = {lap};
+  ctr[0] = u;
+  ctr[1] = kk[0];
 {RK_EPILOGUE}
 #pragma unroll
   for (int g = 0; g < NGF; g++) out[g * Ntot + idx] = nxt[g];
@@ -2161,8 +2200,9 @@ extern "C" hipError_t launch_wave_rhs_{tag}(dim3 g, dim3 b, hipStream_t s, const
   return hipGetLastError();
 }}
 extern "C" hipError_t launch_wave_rhs_rk_{tag}(dim3 g, dim3 b, hipStream_t s, const double *in, const double *y_n,
-    double *y_run, double *out, bhah_kparams p) {{
-  hipLaunchKernelGGL(wave_rhs_rk_{tag}, g, b, 0, s, in, y_n, y_run, out, p);
+    double *y_run, double *out, bhah_kparams p, int ghosts) {{
+  if (ghosts) hipLaunchKernelGGL(wave_rhs_rk_{tag}<true>, g, b, 0, s, in, y_n, y_run, out, p);
+  else hipLaunchKernelGGL(wave_rhs_rk_{tag}<false>, g, b, 0, s, in, y_n, y_run, out, p);
   return hipGetLastError();
 }}
 """

@@ -68,7 +68,7 @@ struct BssnKernels {
 
 extern "C" hipError_t launch_wave_rhs_fd4(dim3, dim3, hipStream_t, const double *, double *, bhah_kparams);
 extern "C" hipError_t launch_wave_rhs_rk_fd4(dim3, dim3, hipStream_t, const double *, const double *, double *,
-                                             double *, bhah_kparams);
+                                             double *, bhah_kparams, int);
 
 namespace {
 
@@ -377,6 +377,132 @@ bc_extrap_kernel(const int16_t *__restrict__ pts, int npts, int ngfs, double *__
   const long s = q[3] + s1 * q[4] + s2 * q[5];
   double *f = &gfs[gf * Ntot];
   f[i] = +3.0 * f[i + s] - 3.0 * f[i + 2 * s] + 1.0 * f[i + 3 * s];
+}
+
+// All layers of the extrapolation on one radial line of one gridfunction (spherical-like grids),
+// innermost first: one launch where the per-layer form takes NG dependent ones.
+__global__ void __launch_bounds__(256)
+bc_extrap_lines_kernel(const int *__restrict__ lines, int nlines, int ngfs, int NG, double *__restrict__ gfs, int Nx0,
+                       long s1, long s2, long Ntot) {
+#pragma clang fp contract(off)
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (long)nlines * ngfs) return;
+  const int l = (int)(t % nlines), gf = (int)(t / nlines);
+  double *f = gfs + gf * Ntot + s1 * lines[2 * l] + s2 * lines[2 * l + 1] + (Nx0 - NG);
+  double f1 = f[-1], f2 = f[-2], f3 = f[-3];
+  for (int gz = 0; gz < NG; gz++) {
+    const double v = +3.0 * f1 - 3.0 * f2 + 1.0 * f3;
+    f[gz] = v;
+    f3 = f2;
+    f2 = f1;
+    f1 = v;
+  }
+}
+
+// All ghost layers of a Cartesian box (every ghost point a pure outer point) in one launch.  The
+// per-list form fills layer by layer, in each layer the xx0, then the xx1, then the xx2 faces, each
+// widened by the ghost points before it: a point whose layer numbers are l0, l1, l2 (0 inside) is
+// extrapolated along the last direction of largest layer number.  Every ghost value is so a
+// function of the 3 x 3 x 3 interior points nearest to it, and each workgroup below forms what
+// it needs itself, with the same operations: faces by lines, edges and corners through a patch of
+// the box in LDS, filled in the lists' order.  Needs three interior points in each direction.
+constexpr int BOX_NG = 2;
+struct BoxBlocks {
+  int face[3], edge[3];  // workgroups per face pair normal to d; per set of four edges along d
+};
+__global__ void __launch_bounds__(256)
+bc_extrap_box_kernel(double *__restrict__ gfs, int ngfs, int Nx0, int Nx1, int Nx2, long Ntot, BoxBlocks nb) {
+#pragma clang fp contract(off)
+  constexpr int NG = BOX_NG, W = NG + 3;  // a corner patch: NG ghost and 3 interior points a side
+  const int N[3] = {Nx0, Nx1, Nx2};
+  const long S[3] = {1, Nx0, (long)Nx0 * Nx1};
+  const int tid = (int)threadIdx.x;
+  int b = (int)blockIdx.x;
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const int e0 = d == 0 ? 1 : 0, e1 = d == 2 ? 1 : 2;
+    if (b < nb.face[d]) {  // one thread per (gridfunction, side, line normal to the face)
+      const long n0 = N[e0] - 2 * NG, n1 = N[e1] - 2 * NG, per = n0 * n1;
+      const long t = (long)b * 256 + tid;
+      if (t >= 2 * per * ngfs) return;
+      const long q = t % per, r = t / per;
+      const int side = (int)(r & 1), g = (int)(r >> 1);
+      double *f = gfs + g * Ntot + (NG + q % n0) * S[e0] + (NG + q / n0) * S[e1] + (side ? N[d] - NG - 1 : NG) * S[d];
+      const long s = side ? S[d] : -S[d];  // outward
+      double f1 = f[0], f2 = f[-s], f3 = f[-2 * s];
+#pragma unroll
+      for (int l = 1; l <= NG; l++) {
+        const double v = +3.0 * f1 - 3.0 * f2 + 1.0 * f3;
+        f[l * s] = v;
+        f3 = f2;
+        f2 = f1;
+        f1 = v;
+      }
+      return;
+    }
+    b -= nb.face[d];
+  }
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const int e0 = d == 0 ? 1 : 0, e1 = d == 2 ? 1 : 2;  // e0 < e1: the directions of the edge's ghosts
+    if (b < nb.edge[d]) {  // one thread per (gridfunction, edge, point along it)
+      const long n = N[d] - 2 * NG;
+      const long t = (long)b * 256 + tid;
+      if (t >= 4 * n * ngfs) return;
+      const long q = t % n;
+      const int c = (int)((t / n) & 3), g = (int)(t / (4 * n));
+      const long o0 = (c & 1) ? S[e0] : -S[e0], o1 = (c & 2) ? S[e1] : -S[e1];
+      double *f = gfs + g * Ntot + (NG + q) * S[d] + ((c & 1) ? N[e0] - NG - 1 : NG) * S[e0] +
+                  ((c & 2) ? N[e1] - NG - 1 : NG) * S[e1];
+      double v[W][W];  // v[a + 2][b + 2]: layer a along e0, b along e1 (-2, -1, 0 interior)
+#pragma unroll
+      for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) v[i][j] = f[(i - 2) * o0 + (j - 2) * o1];
+#pragma unroll
+      for (int z = 3; z < W; z++) {
+#pragma unroll
+        for (int j = 0; j < z; j++) v[z][j] = +3.0 * v[z - 1][j] - 3.0 * v[z - 2][j] + 1.0 * v[z - 3][j];
+#pragma unroll
+        for (int i = 0; i <= z; i++) v[i][z] = +3.0 * v[i][z - 1] - 3.0 * v[i][z - 2] + 1.0 * v[i][z - 3];
+      }
+#pragma unroll
+      for (int i = 3; i < W; i++)
+#pragma unroll
+        for (int j = 3; j < W; j++) f[(i - 2) * o0 + (j - 2) * o1] = v[i][j];
+      return;
+    }
+    b -= nb.edge[d];
+  }
+  // one workgroup per (gridfunction, corner)
+  __shared__ double v[W][W][W];
+  const int c = b & 7, g = b >> 3;
+  long base = g * Ntot, o[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const bool hi = (c >> d) & 1;
+    o[d] = hi ? S[d] : -S[d];
+    base += (hi ? N[d] - NG - 1 : NG) * S[d];
+  }
+  const int i0 = tid % W, i1 = (tid / W) % W, i2 = tid / (W * W);
+  const bool mine = tid < W * W * W;
+  double *f = gfs + base + (i0 - 2) * o[0] + (i1 - 2) * o[1] + (i2 - 2) * o[2];
+  if (mine && i0 < 3 && i1 < 3 && i2 < 3) v[i2][i1][i0] = *f;
+  for (int z = 3; z < W; z++)
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      __syncthreads();
+      const bool now = mine && (d == 0   ? i0 == z && i1 < z && i2 < z
+                                : d == 1 ? i1 == z && i0 <= z && i2 < z
+                                         : i2 == z && i0 <= z && i1 <= z);
+      if (now) {
+        const double *w = &v[i2][i1][i0];
+        const int s = d == 0 ? 1 : d == 1 ? W : W * W;
+        v[i2][i1][i0] = +3.0 * w[-s] - 3.0 * w[-2 * s] + 1.0 * w[-3 * s];
+      }
+    }
+  __syncthreads();
+  if (mine && i0 >= 3 && i1 >= 3 && i2 >= 3) *f = v[i2][i1][i0];
 }
 
 // gf[dst] = +-gf[src] by a sign-bit flip (…/apply_bcs_inner_only__openmp.c:3-57).
@@ -1821,8 +1947,39 @@ int bhah_hip_apply_bcs_inner_only(bhah_patch *P, double *gfs) {
   return BHAH_OK;
 }
 
+// Whether the box form of the extrapolation runs: every ghost point outer, three points to
+// extrapolate from in each direction.
+static bool extrap_box(const bhah_patch *P) {
+  return P->d.coord == BHAH_CARTESIAN && P->NG == BOX_NG && P->inner_dst.empty() && P->d.Nxx[0] >= 3 &&
+         P->d.Nxx[1] >= 3 && P->d.Nxx[2] >= 3;
+}
+
 int bhah_hip_apply_bcs_outerextrap_and_inner(bhah_patch *P, double *gfs) {
   if (!P || !gfs) return fail(BHAH_ERR_ARG, "NULL argument");
+  if (extrap_box(P)) {
+    // One launch for the 3 NG lists' dependent ones: 2.8 us each at 64^3.
+    BoxBlocks nb;
+    long total = 8L * P->ngfs;
+    for (int d = 0; d < 3; d++) {
+      const long n = P->d.Nxx[d], face = (long)P->d.Nxx[(d + 1) % 3] * P->d.Nxx[(d + 2) % 3];
+      nb.face[d] = (int)((2 * face * P->ngfs + 255) / 256);
+      nb.edge[d] = (int)((4 * n * P->ngfs + 255) / 256);
+      total += nb.face[d] + nb.edge[d];
+    }
+    hipLaunchKernelGGL(bc_extrap_box_kernel, dim3((unsigned)total), dim3(256), 0, P->stream, gfs, P->ngfs, P->Nx[0],
+                       P->Nx[1], P->Nx[2], P->Ntot, nb);
+    HIP_TRY(hipGetLastError());
+    return BHAH_OK;
+  }
+  if (P->n_rad_lines && P->d.Nxx[0] + P->NG >= 3) {
+    const long items = (long)P->n_rad_lines * P->ngfs;
+    const unsigned nt = rad_threads(items);
+    hipLaunchKernelGGL(bc_extrap_lines_kernel, dim3((unsigned)((items + nt - 1) / nt)), dim3(nt), 0, P->stream,
+                       P->d_rad_lines, P->n_rad_lines, P->ngfs, P->NG, gfs, P->Nx[0], (long)P->Nx[0],
+                       (long)P->Nx[0] * P->Nx[1], P->Ntot);
+    HIP_TRY(hipGetLastError());
+    return bhah_hip_apply_bcs_inner_only(P, gfs);
+  }
   for (int gz = 0; gz < P->NG; gz++)
     for (int d = 0; d < 3; d++) {
       const int n = (int)(P->outer[gz][d].size() / 6);
@@ -1923,9 +2080,11 @@ static int enqueue_step(bhah_patch *P, bhah_MoL_gridfunctions *gf, double dt) {
       dim3 g, b;
       P->interior_dims(g, b);
       double *next = (s == 4) ? gf->y_n_gfs : out_s[s - 1];
+      // stages past the first form the ghost values they read themselves (the caller's y_n may hold
+      // any); only y_n's ghost zones are filled
       HIP_TRY(launch_wave_rhs_rk_fd4(g, b, P->stream, in_s[s - 1], gf->y_n_gfs, gf->y_nplus1_running_total_gfs, next,
-                                     P->kp(dt, s)));
-      if ((rc = bhah_hip_wave_apply_bcs(P, next))) return rc;
+                                     P->kp(dt, s), s == 1 || !extrap_box(P)));
+      if ((s == 4 || !extrap_box(P)) && (rc = bhah_hip_wave_apply_bcs(P, next))) return rc;
     }
     return BHAH_OK;
   }
