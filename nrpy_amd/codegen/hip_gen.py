@@ -952,6 +952,12 @@ SMALL_CANDIDATES = {"rhs": ["p1_lb1", "p1_lb1_sl_lf_pf16_u32_w2", "p1_lb1_sj_L16
                     "ricci": ["r1_lb1", "r1_lb1_pf16_u32", "r1_lb1_sj_L16x8x2x1_d3_dma_rb1",
                               "r1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_lr40_di_mi_xcd"]}
 
+# The staged constraints kernel of every build (the plain one in bssn_kernels takes what this one
+# does not: input that is not 16-byte aligned, 2^29 points and more).  27 first and second
+# derivatives' worth of LDS reads a point; the tile and ring are those of the fd6 Ricci kernel.  100 us
+# at 128x64x64 fd6 against 453 us for the plain kernel.
+CONSTRAINTS_STAGED = "k1_lb1_L16x2x2x1_d3_dmo_rb1_io_pg_lr40_di_mi_xcd"
+
 CAND_SIG = ("dim3 g, dim3 b, hipStream_t s, const double *in, const double *aux, double *out, "
             "const double *rfm0, const double *rfm1, bhah_kparams p")
 
@@ -1671,20 +1677,23 @@ def candidate_tu(v: specs.Variant, fd_order: int, kind: str, cand: str, ensemble
     ens_kernels, ens_calls = [], []
     if kind == "rhs":
         spec = specs.bssn_rhs_spec(v, staged=staged)
-        groups = RHS_PARTITIONS[part]
+        groups, all_outs = RHS_PARTITIONS[part], list(bssn.EVOL_GFS)
+    elif kind == "constraints":
+        spec = specs.constraints_spec(v)
+        all_outs = [g for g, _ in spec.outputs]
+        groups = [all_outs]
     else:
         spec = specs.ricci_spec(v, staged=staged)
-        groups = RICCI_PARTITIONS[part]
+        groups, all_outs = RICCI_PARTITIONS[part], list(bssn.AUXEVOL_GFS)
     for k, gfs in enumerate(groups):
         sub = spec if len(groups) == 1 else _subspec(spec, f"{spec.name}_{part}g{k}", gfs)
         if scope == "local":
             sub = _subspec(sub, f"{sub.name}_local", [g for g, _ in sub.outputs])
         kname = f"bssn_{kind}_{tag}_{cand}_g{k}"
         if lds:
-            outs = list(bssn.EVOL_GFS if kind == "rhs" else bssn.AUXEVOL_GFS)
             ename = f"bssn_ens_{kind}_{tag}_{cand}_g{k}" if ensemble else ""
             src, launch, fl = lds_kernel(sub, fd_order, kname, rats, lds, 2 if lb == "lb2" else 1, scope,
-                                         [f"out[{outs.index(g)} * Ntot + idx]" for g, _ in sub.outputs], xcd=xcd,
+                                         [f"out[{all_outs.index(g)} * Ntot + idx]" for g, _ in sub.outputs], xcd=xcd,
                                          depth=next((int(o[1:]) for o in opts if o[0] == "d" and o[1:].isdigit()), 1),
                                          zfirst="zf" in opts, blocked="blk" in opts,
                                          group=next((int(o[1:]) for o in opts if o[0] == "g" and o[1:].isdigit()), 1),
@@ -2264,12 +2273,20 @@ def generate(outdir: str) -> List[str]:
             arrays[kind] = f"kCand_{kind}_{tag}"
             ncand[kind] = len(kcands)
             table_decl.append(f"static const BssnCandidate {arrays[kind]}[] = {{{', '.join(rows)}}};")
+        cand = CONSTRAINTS_STAGED
+        src, fl = candidate_tu(v, order, "constraints", cand)
+        path = os.path.join(outdir, f"bssn_{tag}_constraints_{cand}.hip")
+        with open(path, "w", encoding="utf-8") as f:
+            f.write(hdr + src)
+        paths.append(path)
+        meta["candidates"][f"constraints_{tag}_{cand}"] = fl
+        table_decl.append(f'extern "C" hipError_t launch_bssn_constraints_{tag}_{cand}({CAND_SIG});')
         sym_mask = sum(1 << int(c) for c in v.symmetry_axes)
         table_rows.append(
             f"    {{{COORD_ENUM[v.coord]}, {sym_mask}, {int(v.enable_KO)}, {order}, \"{tag}\", "
             f"{arrays['rhs']}, {ncand['rhs']}, {arrays['ricci']}, {ncand['ricci']}, "
             f"launch_bssn_rk_det_{tag}, launch_bssn_rk_det_inner_{tag}, launch_bssn_detgamma_{tag}, "
-            f"launch_bssn_constraints_{tag}, "
+            f"launch_bssn_constraints_{tag}, launch_bssn_constraints_{tag}_{CONSTRAINTS_STAGED}, "
             f"launch_bssn_initial_lambda_{tag}, "
             f"{f'launch_bssn_ens_rk_det_{tag}' if ens else 'nullptr'}, "
             + (f"adj_nslots_{tag}, launch_adj_rhs_{tag}, launch_adj_ricci_{tag}, launch_adj_final_{tag}, "

@@ -8,7 +8,8 @@ import numpy as np
 import pytest
 
 from nrpy_amd import initial_data as ID
-from tests.test_kernels_on_cpu import _check, schedules
+from nrpy_amd.codegen.hip_gen import CONSTRAINTS_STAGED
+from tests.test_kernels_on_cpu import _check, build, interior, rel_err, run, schedules
 
 BUILDS = {
     "Spherical_sym2_KO0_fd4": dict(coord=1, fd_order=4, sym=4, KO=False, size=7.5, variant=0),
@@ -29,6 +30,23 @@ def test_odd_row_schedules_on_cpu(oracle_lib, tag, Nxx):
     cands = [kc for kc in schedules(tag) if "_dmo_" in kc[1]]
     assert {k for k, _ in cands} == {"rhs", "ricci"}
     _check(oracle_lib, tag, cands, [(64, 4)], Nxx=Nxx)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+@pytest.mark.parametrize("tag,Nxx", [(t, n) for t in BUILDS for n in SIZES[t][:2]])
+def test_staged_constraints_on_cpu(oracle_lib, tag, Nxx, tmp_path):
+    """Bounds of every access, and H, M^i, M^2 and |Lambda| against the oracle: each is a sum that
+    cancels to the constraint violation of the data (here of the order of its terms), so 1e-11 of
+    the largest value, the bound of the GPU parity test."""
+    b = BUILDS[tag]
+    O = oracle_lib.OracleGrid(b["coord"], Nxx, b["fd_order"], b["size"], 0.2, variant=b["variant"])
+    y = ID.smooth_perturbation(ID.brill_lindquist(b["coord"], O.xx, b["size"], 0.2), O.xx, 5)
+    y = np.ascontiguousarray(y)
+    O.apply_bcs_outerextrap_and_inner(y)
+    aux = O.ricci(y)
+    exe = build(tag, "constraints", CONSTRAINTS_STAGED, str(tmp_path))
+    out = run(exe, O, "rhs", y, aux, (64, 4), str(tmp_path))[:6]
+    assert rel_err(interior(out, O.NG), interior(O.constraints(y, aux), O.NG)).max() < 1e-11
 
 
 @pytest.mark.gpu
