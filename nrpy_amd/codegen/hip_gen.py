@@ -926,31 +926,33 @@ def _group_bounds(lb: str, k: int, ngroups: int) -> str:
 # is selected.  The plain one-thread-per-point schedule comes first (any size and alignment).
 # What decides between the forms, measured per launch on MI355X:
 #   * _dmo takes rows of any length; _dma needs even ones and has a box two values narrower
-#     where the stencils reach NGHOSTS: rhs fd6 752 against 820 us at 192x96x96, 208 against 207
-#     at 128x64x64 and 127x63x62 (the plain schedule: 1032 us there).
+#     where the stencils reach NGHOSTS: rhs fd6 691 against 791 us at 192x96x96, 185 against 188
+#     at 128x64x64 and 127x63x62 (the plain schedule: 1027 us there).
+#   * _tp forms mixed derivatives in two passes within a wave (``lds_kernel``): rhs fd6 691
+#     against 749 us at 192x96x96, Ricci fd6 269 against 336, Ricci fd4 132 against 151 at
+#     160x80x80; the fd4 right-hand side gains little (74.9 against 75.5 us at 96x48x48).
 #   * Small workgroups suit the kernels whose boxes are small: a wave then waits for its own
 #     box instead of three other waves', and several workgroups of a CU are at different
-#     points.  Ricci fd6, 64 threads against 256: 314 against 360 us at 192x96x96; fd4: 35.4
-#     against 41.0 at 96x48x48; phi-symmetric: 23.0 against 29.4 at 256x64x16.  rhs
-#     phi-symmetric (no xx2 halo): 42.9 against 59.3.  The 3D right-hand side's boxes reach
-#     three or four points every way; there a 64-thread tile stages nine boxes' worth of
-#     halo and loses (99 against 75 us, fd4 at 96x48x48).
+#     points.  Ricci fd6, 128 threads against 256: 269 against 286 us at 192x96x96;
+#     phi-symmetric, 64 threads: Ricci 23.0 against 29.4 at 256x64x16, rhs (no xx2 halo) 42.9
+#     against 59.3.  The 3D right-hand side's boxes reach three or four points every way;
+#     there a 128-thread tile stages two thirds more halo and loses (843 against 691 us).
 FULL_CANDIDATES = {
     "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_mi_xcd", "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk",
-            "p1_lb1_sj_L16x4x4x1_d4_dmo_rb1_io_pg_ub_sa_lr40_di_mi_blk_xcd",
-            "p1_lb1_sj_L16x4x4x1_d4_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk"],
+            "p1_lb1_sj_L16x4x4x1_d4_dmo_rb1_io_pg_ub_sa_lr48_di_tp_mi_blk_xcd",
+            "p1_lb1_sj_L16x4x4x1_d4_dma_rb1_io_pg_ub_sa_lr48_di_tp_mi_xcd_blk"],
     "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_lr40_mi_xcd",
-              "r1_lb1_sj_L16x2x2x1_d3_dmo_rb1_io_pg_lr40_di_mi_xcd", "r1_lb1_sj_L16x2x2x1_d3_dma_rb1_io_pg_lr40_di_mi_xcd"],
+              "r1_lb1_sj_L16x4x2x1_d3_dmo_rb1_io_pg_lr48_di_tp_mi_xcd", "r1_lb1_sj_L16x4x2x1_d3_dma_rb1_io_pg_lr48_di_tp_mi_xcd"],
 }
 FULL_FD4_CANDIDATES = {
-    "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d4_dmo_rb1_io_pg_ub_sa_lr40_di_mi_xcd"],
-    "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x1x1_d3_dmo_rb1_io_pg_lr40_di_mi_xcd"],
+    "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d5_dmo_rb1_io_pg_ub_sa_lr48_di_tp_mi_xcd"],
+    "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x2x1_d3_dmo_rb1_io_pg_lr48_di_tp_mi_blk_xcd"],
 }
 SMALL_CANDIDATES = {"rhs": ["p1_lb1", "p1_lb1_sl_lf_pf16_u32_w2", "p1_lb1_sj_L16x8x2x1_d3_dma_rb1",
                             "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8", "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8_ub",
-                            "p1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_ub_lr40_di_mi_xcd"],
+                            "p1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_ub_lr48_di_tp_mi_xcd"],
                     "ricci": ["r1_lb1", "r1_lb1_pf16_u32", "r1_lb1_sj_L16x8x2x1_d3_dma_rb1",
-                              "r1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_lr40_di_mi_xcd"]}
+                              "r1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_lr48_di_tp_mi_xcd"]}
 
 # The staged constraints kernel of every build (the plain one in bssn_kernels takes what this one
 # does not: input that is not 16-byte aligned, 2^29 points and more).  27 first and second
@@ -1037,6 +1039,11 @@ LDS_DMA_MACROS = """#ifndef BHAH_DMA16
 // the same before the LDS reads of DMA phase n; the comment marks it in the assembly listing
 // for the build's wait check (nrpy_amd/isa_check.py)
 #define BHAH_BARRIER_PHASE(n) asm volatile("s_waitcnt lgkmcnt(0)\\n\\ts_barrier ; bhah_read_phase " #n ::: "memory")
+#endif
+#ifndef BHAH_WAVE_SYNC
+// order of LDS accesses of one wave: the hardware runs them in program order, and the clobber keeps
+// the compiler from moving a lane's load above the stores other lanes make for it
+#define BHAH_WAVE_SYNC() asm volatile("" ::: "memory")
 #endif
 """
 
@@ -1161,7 +1168,7 @@ def _int_line_sum(W: Dict[int, int], pts: Dict[int, str], mirror: str) -> Tuple[
     return f"({' + '.join(parts)})", fl
 
 
-_SH_REF = re.compile(r"sh\[c\d+[yzw]?(?: [+-] \d+)?\]")
+_SH_REF = re.compile(r"sh\[c\w+(?: [+-] \d+)?\]")
 
 
 def _batch_lds_reads(stmts: List[Tuple[str, List[str]]], nmax: int, prefix: str) -> List[Tuple[str, List[str]]]:
@@ -1224,7 +1231,7 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
                one_barrier: bool = False, ensemble: str = "", interleave: bool = False,
                pin_group: int = -1, branchless_upwind: bool = False, blocked: bool = False,
                sym_lines: bool = False, read_batch: int = 0, dma_spread: bool = False,
-               odd_rows: bool = False) -> Tuple[str, str, int]:
+               odd_rows: bool = False, two_pass: bool = False) -> Tuple[str, str, int]:
     """One workgroup-tiled kernel.  Each gridfunction with derivatives is staged, one at a
     time, from global memory into a halo box in LDS: ``group`` gridfunctions per
     barrier-separated phase, with the loads of the next ``depth`` phases in flight while
@@ -1241,6 +1248,14 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
     instead, which any Nx0 allows: a row then starts in its box at its first point or one
     point before, and the reads go through four base indices, by the parity of the row's
     distance in xx1 and xx2 from the thread's own row.
+
+    With ``two_pass`` a mixed second derivative is formed as the stencil along one direction of the
+    first-derivative sums along the other, within one wave (16 points along xx0, 4 along xx1, one
+    xx2): every lane's own xx1 and xx2 sums, which the first derivatives need anyway, and those of
+    the 2h columns and rows around the wave go to a wave-private LDS patch, and each mixed derivative
+    is then 2h reads of the patch (h = fd_order / 2).  Per gridfunction at fd6 that is 48 LDS accesses
+    and 39 FP64 operations against 108 and 111, and two LDS round trips against four.  No barrier:
+    a wave's LDS accesses run in order.
 
     The box has a halo along xx2 only where the kernel differentiates along xx2 (a
     phi-symmetric build does not).
@@ -1313,8 +1328,16 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
     NJ = (NB // 2 + NT - 1) // NT  # 16-byte DMA loads per thread per box
     SLOT = 2 * NT * NJ if dma else NB  # doubles per box (DMA boxes padded so every lane loads)
     nslots = (max(1, min(depth, -(-len(staged) // group))) * group) if dma else min(group, len(staged))
-    if 8 * SLOT * nslots > 160 * 1024:
-        raise ValueError(f"{kname}: {8 * SLOT * nslots} bytes of LDS exceed the 160 KiB of a CU")
+    # two-pass patch of a wave: first-derivative sums along xx2 on a cross of 4 + 2h rows, then those
+    # along xx1 on 4 rows, rows of 16 + 2h values at a pitch of 24, and one unused place
+    HS, PP = fd_order // 2, 24
+    patch_y = PP * (4 + 2 * HS) if HZ else 0
+    patch = (patch_y + PP * 4 + 2) if two_pass else 0
+    if two_pass and (TX != 16 or TY % 4 or P != 1 or not dma):
+        raise ValueError("two-pass mixed derivatives take DMA-staged waves of 16 x 4 points")
+    lds_doubles = nslots * SLOT + patch * (NT // 64)
+    if 8 * lds_doubles > 160 * 1024:
+        raise ValueError(f"{kname}: {8 * lds_doubles} bytes of LDS exceed the 160 KiB of a CU")
     # algebra for a placeholder point; each point substitutes its own register names
     ovr: Dict[str, str] = {}
     for n in centre:
@@ -1353,6 +1376,40 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
   const int q{k} = (o0 - {H} + (int)s1 * (o1 + ly) + (int)s2 * (o2 + lz + {k * ZS})) & 1;
   const int c{k} = c{k}b + q{k}, c{k}y = c{k}b + (q{k} ^ ((int)s1 & 1)), c{k}z = c{k}b + (q{k} ^ ((int)s2 & 1)),
             c{k}w = c{k}b + (q{k} ^ ((int)(s1 + s2) & 1));""")
+    if two_pass:
+        # halo sums of this lane: rounds along xx2 (rows above and below the wave, then columns left
+        # and right), one round along xx1 (columns); cNh: their places in the box, cNd: in the patch
+        nyh, nxh = 2 * HS * 16, 2 * HS * 4
+        ztot = (nyh + nxh) if HZ else 0
+        zr = -(-ztot // 64)
+        a(f"""  const int lane = tid & 63, pb = {nslots * SLOT} + {patch} * (tid >> 6), wy = ly & ~3;
+  const int cz = pb + (lx + {HS}) + {PP} * ((ly - wy) + {HS}), cy = pb + {patch_y} + (lx + {HS}) + {PP} * (ly - wy);""")
+        for r in range(zr + 1):
+            if r < zr:
+                a(f"""  int hx{r}, hy{r}, c0d{r};
+  {{
+    const int e = lane + {64 * r}, q = (e - {nyh}) % {2 * HS}, w = e / 16;
+    const bool row = e < {nyh}, none = e >= {ztot};
+    hx{r} = none ? 0 : row ? e % 16 : (q < {HS} ? q - {HS} : {16 - HS} + q);
+    hy{r} = none ? 0 : row ? (w < {HS} ? w - {HS} : {4 - HS} + w) : (e - {nyh}) / {2 * HS};
+    c0d{r} = none ? pb + {patch - 2} : pb + (hx{r} + {HS}) + {PP} * (hy{r} + {HS});
+  }}""")
+            else:
+                a(f"""  int hx{r}, hy{r}, c0d{r};
+  {{
+    const int q = lane % {2 * HS};
+    const bool none = lane >= {nxh};
+    hx{r} = none ? 0 : q < {HS} ? q - {HS} : {16 - HS} + q;
+    hy{r} = none ? 0 : lane / {2 * HS};
+    c0d{r} = none ? pb + {patch - 2} : pb + {patch_y} + (hx{r} + {HS}) + {PP} * hy{r};
+  }}""")
+            box0 = f"(hx{r} + {H + (0 if odd_rows else SH)}) + BX * (wy + hy{r} + {H}) + BX * BY * (lz + {HZ})"
+            if odd_rows:
+                st = "s2" if r < zr else "s1"
+                a(f"""  const int q0h{r} = (o0 - {H} + (int)s1 * (o1 + wy + hy{r}) + (int)s2 * (o2 + lz)) & 1;
+  const int c0h{r} = {box0} + q0h{r}, c0h{r}o = {box0} + (q0h{r} ^ ((int){st} & 1));""")
+            else:
+                a(f"  const int c0h{r} = {box0};")
     # Upwind sums are formed with integer weights (their common denominator DU moved into
     # one uniform scale per direction): an FP64 multiply-add takes an integer weight as an
     # instruction literal, where a weight such as 1/30 needs a register pair loaded first.
@@ -1440,9 +1497,40 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
                 stmts: List[Tuple[str, List[str]]] = []  # (statement, values it forms)
                 if g in ovr and g in used:
                     stmts.append((f"  double V{k}_{g} = {st.load(g, (0, 0, 0))};", [f"V{k}_{g}"]))
+                mixed = [d for d in dused if d.gf == g and d.op == "dDD" and d.dirs[0] != d.dirs[1]] if two_pass else []
+                w1 = dict(fd.weights_1d("dD", fd_order))
+
+                def sum1(ref):
+                    """First-derivative sum (no 1/dx) over ref(offset), the terms of StencilEmitter.expr."""
+                    return " + ".join(f"{_dbl(w1[o])} * ({ref(o)} - {ref(-o)})" for o in sorted(w1) if o > 0)
+
+                def at(c, o):
+                    return f"sh[{c}{f' + {o}' if o > 0 else (f' - {-o}' if o < 0 else '')}]"
+
+                dirs2 = sorted({d.dirs[1] for d in mixed})  # mixed (0, 1), (0, 2), (1, 2): the sums stored
+                for q2 in dirs2:
+                    n = f"S{q2}_{g}"
+                    stmts.append((f"  double {n} = {sum1(lambda o: st.load(g, tuple(o if r == q2 else 0 for r in range(3))))};",
+                                  [n]))
                 for d in dused:
-                    if d.gf == g:
-                        stmts.append((f"  double V{k}_{d.symbol} = {st.expr(d)};", [f"V{k}_{d.symbol}"]))
+                    if d.gf != g or d in mixed:
+                        continue
+                    if d.op == "dD" and d.dirs[0] in dirs2:
+                        stmts.append((f"  double V{k}_{d.symbol} = p.invdxx{d.dirs[0]} * S{d.dirs[0]}_{g};",
+                                      [f"V{k}_{d.symbol}"]))
+                        continue
+                    stmts.append((f"  double V{k}_{d.symbol} = {st.expr(d)};", [f"V{k}_{d.symbol}"]))
+                halo = []
+                for r in range(zr + 1) if mixed else ():
+                    q2, stride = (2, BX * BY) if r < zr else (1, BX)
+                    if q2 not in dirs2:
+                        continue
+                    n = f"S{q2}h{r}_{g}"
+                    base = box(ph, q)
+                    stmts.append((f"  double {n} = "
+                                  f"{sum1(lambda o: at(f'c0h{r}' + ('o' if odd_rows and o & 1 else ''), base + o * stride))};",
+                                  [n]))
+                    halo.append((r, n))
                 for dirn in range(3):
                     key = (g, dirn)
                     if key not in line_out:
@@ -1484,6 +1572,23 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
                     stmts.append((f"  {acc} += {' + '.join(tc)};", [acc]))
                 if read_batch:
                     stmts = _batch_lds_reads(stmts, read_batch, f"R{k}_{g}")
+                if mixed:
+                    # the sums into the wave's patch, then each mixed derivative from it
+                    put = [f"  sh[{'cz' if q2 == 2 else 'cy'}] = S{q2}_{g};" for q2 in dirs2]
+                    put += [f"  sh[c0d{r}] = {n};" for r, n in halo]
+                    second = []
+                    for d in mixed:
+                        a0, a1 = d.dirs
+                        c, stride = ("cy", 1) if a1 == 1 else ("cz", 1 if a0 == 0 else PP)
+                        second.append((f"  double V{k}_{d.symbol} = p.invdxx{a0} * p.invdxx{a1} * "
+                                       f"({sum1(lambda o: at(c, o * stride))});", [f"V{k}_{d.symbol}"]))
+                    if read_batch:
+                        second = _batch_lds_reads(second, read_batch, f"T{k}_{g}")
+                    stmts = stmts + [("  BHAH_WAVE_SYNC();\n" + "\n".join(put) + "\n  BHAH_WAVE_SYNC();", [])] + second
+                    if k == 0:
+                        P1 = len(w1) // 2
+                        fl[0] += (len(dirs2) + len(halo) + len(mixed)) * (3 * P1 - 1) + 2 * len(mixed)
+                        fl[0] -= sum(stencil_flops(d, fd_order) for d in mixed) + len(dirs2) * (3 * P1 - 1)
                 for text, formed in stmts:
                     e(text)
                     for x in formed:
@@ -1615,7 +1720,7 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
 {dma_note}extern "C" __global__ void __launch_bounds__({bounds})
 {kname}(const double *__restrict__ in, const double *__restrict__ aux, double *__restrict__ out,
         const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p) {{
-  __shared__ double sh[{nslots * SLOT}];
+  __shared__ double sh[{lds_doubles}];
 {_lds_tile_order(xcd, zfirst, blocked)}
 {tile_body}
 }}
@@ -1633,7 +1738,7 @@ static __device__ __forceinline__ void {kname}_tile(const double *__restrict__ i
 extern "C" __global__ void __launch_bounds__({bounds})
 {ensemble}(const bhah_member *__restrict__ mem, const bhah_item *__restrict__ items, const int nitems,
         const int in_sel, const int aux_sel, const int out_sel) {{
-  __shared__ double sh[{nslots * SLOT}];
+  __shared__ double sh[{lds_doubles}];
   for (int it = blockIdx.x; it < nitems; it += gridDim.x) {{
     const bhah_item w = items[it];
     const bhah_member *M = &mem[w.m];
@@ -1701,7 +1806,7 @@ def candidate_tu(v: specs.Variant, fd_order: int, kind: str, cand: str, ensemble
                                          interleave="io" in opts,
                                          branchless_upwind="ub" in opts, sym_lines="sa" in opts,
                                          read_batch=next((int(o[2:]) for o in opts if o[:2] == "lr" and o[2:].isdigit()), 0),
-                                         dma_spread="di" in opts, odd_rows="dmo" in opts,
+                                         dma_spread="di" in opts, odd_rows="dmo" in opts, two_pass="tp" in opts,
                                          pin_group=next((int(o[2:] or 0) for o in opts if o[:2] == "pg" and o[2:].isdigit() or o == "pg"), -1))
             kernels.append(src)
             calls.append(launch)

@@ -23,6 +23,11 @@
 // for the build's wait check (nrpy_amd/isa_check.py)
 #define BHAH_BARRIER_PHASE(n) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier ; bhah_read_phase " #n ::: "memory")
 #endif
+#ifndef BHAH_WAVE_SYNC
+// order of LDS accesses of one wave: the hardware runs them in program order, and the clobber keeps
+// the compiler from moving a lane's load above the stores other lanes make for it
+#define BHAH_WAVE_SYNC() asm volatile("" ::: "memory")
+#endif
 #define Rational_1_2 (1.0 / 2.0)
 #define Rational_1_3 (1.0 / 3.0)
 #define Rational_1_4 (1.0 / 4.0)

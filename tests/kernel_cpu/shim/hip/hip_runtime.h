@@ -86,6 +86,8 @@ inline bhah_cpu_barrier_t bhah_cpu_bar;
 #define BHAH_BARRIER() bhah_cpu_bar.wait()
 #define BHAH_BARRIER_PHASE(n) bhah_cpu_bar.wait()
 #define BHAH_VMWAIT(n) ((void)0)
+// a wave's lanes run in step on the device; here the whole block waits
+#define BHAH_WAVE_SYNC() bhah_cpu_bar.wait()
 // every lane of a wave holds the same value where the kernels use it (the wave index)
 #define __builtin_amdgcn_readfirstlane(x) (x)
 // global-to-LDS load of 16 bytes per lane: lane l writes dst + 16 l (dst is the wave's base)
