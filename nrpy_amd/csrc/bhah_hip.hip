@@ -124,7 +124,7 @@ struct bhah_patch {
   // BHAH_HIP_SEPARATE_INNER_BC=1 at patch creation keeps the separate copy, for comparison)
   bool fold_inner = true;
   // inner points grouped by source: d_inner_by_src[d_inner_src_start[u] .. [u+1]) lists the
-  // points (indices into the inner arrays) copied from source d_inner_src_list[u]
+  // points (destination, parity mask) copied from source d_inner_src_list[u]
   int *d_inner_by_src = nullptr, *d_inner_src_start = nullptr, *d_inner_src_list = nullptr;
   int n_inner_src = 0;
   int16_t *d_outer[8][3] = {};
@@ -610,41 +610,50 @@ bc_radiation_adjoint_kernel(const int16_t *__restrict__ pts, int npts, int ngfs,
 // bc_radiation_lines_kernel): one thread per (line, gridfunction) walks the layers from the
 // outermost in, with the operations of bc_radiation_adjoint_kernel in the same order.  Only
 // this thread touches its line's values, so the additions need no atomics and the result is
-// the per-layer kernels' bit for bit.
+// the per-layer kernels' bit for bit.  The layer count and stencil radius are constants: the line's
+// values are loaded once, updated in registers and stored once, where every addition was a
+// load and a store of its own (@ADJRAD@).
+template <int NG, int R>
 __global__ void __launch_bounds__(256)
-bc_radiation_adjoint_lines_kernel(const int *__restrict__ lines, int nlines, int ngfs, int NG,
-                                  double *__restrict__ lam_rhs, double *__restrict__ lam_f,
-                                  const double *__restrict__ xx0, const double *__restrict__ wavespeed,
-                                  RadStencil st, int R, int coord, double AMPL, double SINHW, int Nx0, long s1,
-                                  long s2, long Ntot, double invdxx0) {
+bc_radiation_adjoint_lines_kernel(const int *__restrict__ lines, int nlines, int ngfs, double *__restrict__ lam_rhs,
+                                  double *__restrict__ lam_f, const double *__restrict__ rad,
+                                  const double *__restrict__ wavespeed, RadLine W, int Nx0, long s1, long s2, long Ntot,
+                                  double invdxx0) {
 #pragma clang fp contract(off)
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)nlines * ngfs) return;
   const int l = (int)(t % nlines), gf = (int)(t / nlines);
-  const long base = s1 * lines[2 * l] + s2 * lines[2 * l + 1];
-  double *lr = &lam_rhs[gf * Ntot];
-  double *lf = &lam_f[gf * Ntot];
+  constexpr int L = NG + R + 2;
+  const int first = Nx0 - NG - 1;
+  const long base = gf * Ntot + s1 * lines[2 * l] + s2 * lines[2 * l + 1];
+  double *lr = lam_rhs + base + first, *lf = lam_f + base + (Nx0 - L);
+  const double *r = rad + first, *dxr = rad + Nx0 + first;
   const double c = wavespeed[gf];
-  for (int gz = NG - 1; gz >= 0; gz--) {
-    const int i0 = Nx0 - NG + gz, j0 = i0 - 1;
-    const long idx = base + i0, idx_int = base + j0;
-    const double lam = lr[idx];
-    lr[idx] = 0.0;
+  double k[NG + 1], a[L];
+#pragma unroll
+  for (int m = 0; m <= NG; m++) k[m] = lr[m];
+#pragma unroll
+  for (int e = 0; e < L; e++) a[e] = lf[e];
+#pragma unroll
+  for (int m = NG; m >= 1; m--) {
+    const double lam = k[m];
+    k[m] = 0.0;
     if (lam == 0.0) continue;
-    double r, dxr, r_int, dxr_int;
-    r_and_dx0dr(coord, AMPL, SINHW, xx0[i0], r, dxr);
-    r_and_dx0dr(coord, AMPL, SINHW, xx0[j0], r_int, dxr_int);
-    const double ratio = (r_int * r_int * r_int) / (r * r * r);
-    lr[idx_int] += ratio * lam;
-    long at[8];
-    double w[8];
-    int n = partial_r_taps(st, R, Nx0, idx, i0, -1, at, w);
-    for (int j = 0; j < n; j++) lf[at[j]] += -c * dxr * invdxx0 * w[j] * lam;
-    lf[idx] += -c / r * lam;
-    n = partial_r_taps(st, R, Nx0, idx_int, j0, -1, at, w);
-    for (int j = 0; j < n; j++) lf[at[j]] += ratio * c * dxr_int * invdxx0 * w[j] * lam;
-    lf[idx_int] += ratio * c / r_int * lam;
+    const double rm = r[m], ri = r[m - 1];
+    const double ratio = (ri * ri * ri) / (rm * rm * rm);
+    k[m - 1] += ratio * lam;
+    const int off = (m > NG - R) ? NG - R - m : -1, offi = (m - 1 > NG - R) ? NG - R - (m - 1) : -1;
+#pragma unroll
+    for (int q = 0; q <= 2 * R; q++) a[1 + m + off + q] += -c * dxr[m] * invdxx0 * W.w[-off - 1][q] * lam;
+    a[R + 1 + m] += -c / rm * lam;
+#pragma unroll
+    for (int q = 0; q <= 2 * R; q++) a[m + offi + q] += ratio * c * dxr[m - 1] * invdxx0 * W.w[-offi - 1][q] * lam;
+    a[R + m] += ratio * c / ri * lam;
   }
+#pragma unroll
+  for (int m = 0; m <= NG; m++) lr[m] = k[m];
+#pragma unroll
+  for (int e = 0; e < L; e++) lf[e] = a[e];
 }
 
 // Reverse of gf[dst] = +-gf[src]: lam[src] += sum of +-lam[dst] over the points copied from
@@ -652,9 +661,8 @@ bc_radiation_adjoint_lines_kernel(const int *__restrict__ lines, int nlines, int
 // order, so the result does not depend on scheduling.  Sources are never destinations, and
 // every destination belongs to one source, so no two threads touch the same value.
 __global__ void __launch_bounds__(256)
-bc_inner_adjoint_kernel(const int *__restrict__ dst, const int *__restrict__ by_src,
-                        const int *__restrict__ src_start, const int *__restrict__ src_list, int nsrc,
-                        const unsigned short *__restrict__ mask, int ngfs, const int *__restrict__ gf_parity,
+bc_inner_adjoint_kernel(const int2 *__restrict__ by_src, const int *__restrict__ src_start,
+                        const int *__restrict__ src_list, int nsrc, int ngfs, const int *__restrict__ gf_parity,
                         double *__restrict__ lam, long Ntot) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)nsrc * ngfs) return;
@@ -663,10 +671,10 @@ bc_inner_adjoint_kernel(const int *__restrict__ dst, const int *__restrict__ by_
   const int par = gf_parity[gf];
   double acc = 0.0;
   for (int j = src_start[u]; j < src_start[u + 1]; j++) {
-    const int p = by_src[j];
-    const double v = l[dst[p]];
-    l[dst[p]] = 0.0;
-    acc += ((mask[p] >> par) & 1u) ? -v : v;
+    const int2 e = by_src[j];  // destination, parity mask
+    const double v = l[e.x];
+    l[e.x] = 0.0;
+    acc += (((unsigned)e.y >> par) & 1u) ? -v : v;
   }
   l[src_list[u]] += acc;
 }
@@ -1732,12 +1740,17 @@ static int patch_upload(bhah_patch *P, const std::vector<double> &rfm0, const st
       by_src_src.push_back(src[order[j]]);
     }
   by_src_start.push_back((int)order.size());
+  std::vector<int> by_src(2 * order.size());
+  for (size_t j = 0; j < order.size(); j++) {
+    by_src[2 * j] = dst[order[j]];
+    by_src[2 * j + 1] = mask[order[j]];
+  }
   P->n_inner_src = (int)by_src_src.size();
   if ((rc = upload(rfm0, &P->d_rfm0)) || (rc = upload(rfm1, &P->d_rfm1)) || (rc = upload(P->xx[0], &P->d_xx0)) ||
       (rc = upload(P->xx[1], &P->d_xx1)) || (rc = upload(P->xx[2], &P->d_xx2)) ||
       (rc = upload(dst, &P->d_inner_dst)) || (rc = upload(src, &P->d_inner_src)) ||
       (rc = upload(mask, &P->d_inner_mask)) || (rc = upload(ws, &P->d_wavespeed)) || (rc = upload(fi, &P->d_finf)) ||
-      (rc = upload(par, &P->d_gf_parity)) || (rc = upload(order, &P->d_inner_by_src)) ||
+      (rc = upload(par, &P->d_gf_parity)) || (rc = upload(by_src, &P->d_inner_by_src)) ||
       (rc = upload(by_src_start, &P->d_inner_src_start)) || (rc = upload(by_src_src, &P->d_inner_src_list))) {
     bhah_hip_patch_destroy(P);
     return rc;
@@ -2451,21 +2464,31 @@ static int adjoint_rhs_bcs(bhah_patch *P, double *lam_k, double *lam_f) {
   if (P->n_inner_src) {
     dim3 g, b;
     launch_1d((long)P->n_inner_src * P->ngfs, g, b);
-    hipLaunchKernelGGL(bc_inner_adjoint_kernel, g, b, 0, P->stream, P->d_inner_dst, P->d_inner_by_src,
-                       P->d_inner_src_start, P->d_inner_src_list, P->n_inner_src, P->d_inner_mask, P->ngfs,
-                       P->d_gf_parity, lam_k, P->Ntot);
+    hipLaunchKernelGGL(bc_inner_adjoint_kernel, g, b, 0, P->stream, (const int2 *)P->d_inner_by_src,
+                       P->d_inner_src_start, P->d_inner_src_list, P->n_inner_src, P->ngfs, P->d_gf_parity, lam_k,
+                       P->Ntot);
     HIP_TRY(hipGetLastError());
   }
   const int R = (P->d.radiation_bc_fd_order > 0 ? P->d.radiation_bc_fd_order : 4) / 2;
   RadStencil st;
   rad_stencil(R, st);
-  if (P->n_rad_lines) {  // outer points on radial lines: every layer in one launch
-    dim3 g, b;
-    launch_1d((long)P->n_rad_lines * P->ngfs, g, b);
-    hipLaunchKernelGGL(bc_radiation_adjoint_lines_kernel, g, b, 0, P->stream, P->d_rad_lines, P->n_rad_lines,
-                       P->ngfs, P->NG, lam_k, lam_f, P->d_xx0, P->d_wavespeed, st, R, P->d.coord,
-                       P->d.grid_physical_size, P->d.SINHW, P->Nx[0], (long)P->Nx[0], (long)P->Nx[0] * P->Nx[1],
-                       P->Ntot, P->invdxx[0]);
+  if (P->n_rad_lines && rad_lines_fit(P->Nx[0], P->NG, R)) {  // every layer in one launch
+    const long items = (long)P->n_rad_lines * P->ngfs;
+    const unsigned nt = rad_threads(items);
+    const dim3 g((unsigned)((items + nt - 1) / nt));
+    const RadLine W = rad_line_weights(st, R);
+#define RAD_LAUNCH(NG_, R_)                                                                                          \
+  if (P->NG == NG_ && R == R_)                                                                                       \
+    hipLaunchKernelGGL((bc_radiation_adjoint_lines_kernel<NG_, R_>), g, dim3(nt), 0, P->stream, P->d_rad_lines,      \
+                       P->n_rad_lines, P->ngfs, lam_k, lam_f, P->d_rad, P->d_wavespeed, W, P->Nx[0],                 \
+                       (long)P->Nx[0], (long)P->Nx[0] * P->Nx[1], P->Ntot, P->invdxx[0])
+    RAD_LAUNCH(3, 1);
+    RAD_LAUNCH(3, 2);
+    RAD_LAUNCH(3, 3);
+    RAD_LAUNCH(4, 1);
+    RAD_LAUNCH(4, 2);
+    RAD_LAUNCH(4, 3);
+#undef RAD_LAUNCH
     HIP_TRY(hipGetLastError());
     return BHAH_OK;
   }
