@@ -247,6 +247,23 @@ def split_linear(spec: specs.Spec):
     return cores, terms
 
 
+# Reciprocals of the reference-metric arrays the algebra divides by, formed once per point.
+INVERSE_RFM = {f"inv_{n}": f"(1.0 / {RFM_EXPR[specs.RFM_SYMBOLS.index(n)]})"
+               for n in ("f0_of_xx0", "f0_of_xx0__D0", "f1_of_xx1")}
+
+
+def _inverse_rfm(e):
+    """Negative powers of the reference-metric arrays as powers of their reciprocals: each
+    distinct power was a division of its own (about 11 FP64 instructions)."""
+    e = sp.sympify(e)
+    sub = {}
+    for q in e.atoms(sp.Pow):
+        b, n = q.args
+        if n.is_Integer and int(n) < 0 and f"inv_{b}" in INVERSE_RFM:
+            sub[q] = sp.Symbol(f"inv_{b}", real=True) ** (-int(n))
+    return e.xreplace(sub) if sub else e
+
+
 def _emit_defs(spec: specs.Spec, fd_order: int, u32: bool = False):
     centre, aux, derivs, rfm, params = spec.classify()
     st = StencilEmitter(spec, fd_order, u32=u32)
@@ -269,7 +286,7 @@ def _ordered_body(spec: specs.Spec, fd_order: int, out_lvalues: List[str], ratio
                   stream_linear: bool = True, order: str = "dfs", barriers: bool = True,
                   cse_scope: str = "joint", linear: str = "stream", prefetch: int = 0,
                   ahead: int = 12, u32: bool = False, chunk: int = 0, wide: bool = False,
-                  defs_override: Dict[str, str] | None = None) -> str:
+                  defs_override: Dict[str, str] | None = None, inverse_rfm: bool = False) -> str:
     """Stencils and CSE'd algebra for one pointwise spec.
 
     With ``stream_linear``, upwind and KO derivatives are consumed as soon as
@@ -294,6 +311,8 @@ def _ordered_body(spec: specs.Spec, fd_order: int, out_lvalues: List[str], ratio
     defs = _emit_defs(spec, fd_order, u32)
     if defs_override:
         defs.update(defs_override)
+    if inverse_rfm:
+        defs.update(INVERSE_RFM)
     derivs = {d.symbol: d for d in spec.classify()[2]}
     centre_names = set(spec.classify()[0]) | set(spec.classify()[1])
     pr = emit.DoublePrinter(rationals)
@@ -548,6 +567,9 @@ def _ordered_body(spec: specs.Spec, fd_order: int, out_lvalues: List[str], ratio
             code(f"  double lin_{g} = 0.0;")
 
     sdefs = spec.used_defs()
+    if inverse_rfm:
+        sdefs = [(sy, _inverse_rfm(e)) for sy, e in sdefs]
+        outs = [_inverse_rfm(e) for e in outs]
     if sdefs and cse_scope == "local":
         # CSE within each staged definition and each output separately: temporaries
         # then live only inside one stage, at the cost of recomputing cheap
@@ -939,20 +961,20 @@ def _group_bounds(lb: str, k: int, ngroups: int) -> str:
 #     there a 128-thread tile stages two thirds more halo and loses (843 against 691 us).
 FULL_CANDIDATES = {
     "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_mi_xcd", "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk",
-            "p1_lb1_sj_L16x4x4x1_d4_dmo_rb1_io_pg_ub_sa_lr48_di_tp_mi_blk_xcd",
+            "p1_lb1_sj_L16x4x4x1_d4_dmo_rb1_io_pg_ub_sa_lr48_di_tp_ir_eb_mi_blk_xcd",
             "p1_lb1_sj_L16x4x4x1_d4_dma_rb1_io_pg_ub_sa_lr48_di_tp_mi_xcd_blk"],
     "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_lr40_mi_xcd",
               "r1_lb1_sj_L16x4x2x1_d3_dmo_rb1_io_pg_lr48_di_tp_mi_xcd", "r1_lb1_sj_L16x4x2x1_d3_dma_rb1_io_pg_lr48_di_tp_mi_xcd"],
 }
 FULL_FD4_CANDIDATES = {
-    "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d5_dmo_rb1_io_pg_ub_sa_lr48_di_tp_mi_xcd"],
-    "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x2x1_d3_dmo_rb1_io_pg_lr48_di_tp_mi_blk_xcd"],
+    "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d5_dmo_rb1_io_pg_ub_sa_lr48_di_tp_ir_eb_mi_xcd"],
+    "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x2x1_d3_dmo_rb1_io_pg_lr48_di_tp_ir_mi_blk_xcd"],
 }
 SMALL_CANDIDATES = {"rhs": ["p1_lb1", "p1_lb1_sl_lf_pf16_u32_w2", "p1_lb1_sj_L16x8x2x1_d3_dma_rb1",
                             "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8", "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8_ub",
-                            "p1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_ub_lr48_di_tp_mi_xcd"],
+                            "p1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_ub_lr48_di_tp_ir_eb_mi_xcd"],
                     "ricci": ["r1_lb1", "r1_lb1_pf16_u32", "r1_lb1_sj_L16x8x2x1_d3_dma_rb1",
-                              "r1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_lr48_di_tp_mi_xcd"]}
+                              "r1_lb1_sj_L16x4x1x1_d4_dmo_rb1_io_pg_lr48_di_tp_ir_mi_xcd"]}
 
 # The staged constraints kernel of every build (the plain one in bssn_kernels takes what this one
 # does not: input that is not 16-byte aligned, 2^29 points and more).  27 first and second
@@ -1231,7 +1253,8 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
                one_barrier: bool = False, ensemble: str = "", interleave: bool = False,
                pin_group: int = -1, branchless_upwind: bool = False, blocked: bool = False,
                sym_lines: bool = False, read_batch: int = 0, dma_spread: bool = False,
-               odd_rows: bool = False, two_pass: bool = False) -> Tuple[str, str, int]:
+               odd_rows: bool = False, two_pass: bool = False, inverse_rfm: bool = False,
+               early_box: bool = False) -> Tuple[str, str, int]:
     """One workgroup-tiled kernel.  Each gridfunction with derivatives is staged, one at a
     time, from global memory into a halo box in LDS: ``group`` gridfunctions per
     barrier-separated phase, with the loads of the next ``depth`` phases in flight while
@@ -1346,7 +1369,7 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
     for d in dused:
         ovr[d.symbol] = f"VPT_{d.symbol}"
     body = _ordered_body(sub, fd_order, lv, rats, cse_scope=scope, linear="lds", prefetch=0, barriers=False,
-                         defs_override=ovr)
+                         defs_override=ovr, inverse_rfm=inverse_rfm)
     flops = FLOPS[f"{sub.name}_fd{fd_order}{_mode_suffix('lds', 0)}"]
     pr = emit.DoublePrinter(rats)
     w_up = dict(fd.weights_1d("dupD", fd_order))
@@ -1418,11 +1441,33 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
     for d in range(3):
         a(f"  const double ius{d} = p.invdxx{d} * (1.0 / {DU}.0), nius{d} = -ius{d}, "
           f"ikos{d} = p.invdxx{d} * (1.0 / {DK}.0);")
+    phases = [staged[i:i + group] for i in range(0, len(staged), group)]
+    depth = max(1, min(depth, len(phases)))
+
+    def box(ph, q):
+        """LDS offset (doubles) of box q of phase ph."""
+        return ((ph % depth) * group + q) * SLOT if dma else q * NB
+
+    issue: List[Tuple[int, int]] = []  # DMA loads: (phase, loads per lane) in issue order
+
+    def dma_phase(ph):
+        issue.append((ph, len(phases[ph]) * NJ))
+        for q, g in enumerate(phases[ph]):
+            a(f"""  {{
+    const char *src = (const char *)(in + {sub.gfs.index(g)} * Ntot);
+#pragma unroll
+    for (int j = 0; j < {NJ}; j++) BHAH_DMA16O(src, pofs[j], sh + {box(ph, q)} + 2 * (NT * j + 64 * wv));
+  }}""")
+
+    early_box = early_box and dma and one_barrier and bool(terms)
+    if early_box:
+        dma_phase(0)
     if terms:
         # coefficients of the linear terms and the upwind control vector at each point
-        crep, cred = sp.cse(coefs, symbols=sp.numbered_symbols("lc"), order="none")
+        inv = _inverse_rfm if inverse_rfm else sp.sympify
+        crep, cred = sp.cse([inv(c) for c in coefs], symbols=sp.numbered_symbols("lc"), order="none")
         flops += sum(emit._flops(e) for _, e in crep) + sum(emit._flops(e) for e in cred)
-        upw = [sp.sympify(sub.upwind[d]) for d in range(3)]
+        upw = [inv(sub.upwind[d]) for d in range(3)]
         names = set()
         for e in [e for _, e in crep] + list(cred) + upw:
             names |= {str(x) for x in e.free_symbols}
@@ -1438,6 +1483,8 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
                     a(f"    const double {n} = {RFM_EXPR[specs.RFM_SYMBOLS.index(n)]};")
                 elif n in PARAM_EXPR:
                     a(f"    const double {n} = {PARAM_EXPR[n]};")
+                elif n in INVERSE_RFM:
+                    a(f"    const double {n} = {INVERSE_RFM[n]};")
                 elif not n.startswith("lc"):
                     raise ValueError(f"linear coefficient depends on {n}")
             for sy, e in crep:
@@ -1459,13 +1506,7 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
                       f"L{k}_coef[{ck}] * (p.invdxx{d} * {_dbl(sym[3] / sym[2])});")
             for g_out in sorted(terms):
                 a(f"  double V{k}_lin_{g_out} = 0.0;")
-    phases = [staged[i:i + group] for i in range(0, len(staged), group)]
-    depth = max(1, min(depth, len(phases)))
     fl = [flops]
-
-    def box(ph, q):
-        """LDS offset (doubles) of box q of phase ph."""
-        return ((ph % depth) * group + q) * SLOT if dma else q * NB
 
     def emit_phase(ph, gfs, dma_lines=()):
         """Derivatives and linear-term contributions of the phase's gridfunctions; with
@@ -1618,17 +1659,6 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
         # loads issued after a phase's own is known at compile time: waiting until at most
         # that many are outstanding means this phase's boxes have landed (vmcnt counts in
         # order); the barrier then publishes all waves' boxes
-        issue: List[Tuple[int, int]] = []  # (phase, loads per lane) in issue order
-
-        def dma_phase(ph):
-            issue.append((ph, len(phases[ph]) * NJ))
-            for q, g in enumerate(phases[ph]):
-                a(f"""  {{
-    const char *src = (const char *)(in + {sub.gfs.index(g)} * Ntot);
-#pragma unroll
-    for (int j = 0; j < {NJ}; j++) BHAH_DMA16O(src, pofs[j], sh + {box(ph, q)} + 2 * (NT * j + 64 * wv));
-  }}""")
-
         def dma_lines(ph):
             """The loads of phase ph one statement each, in the order dma_phase issues them."""
             issue.append((ph, len(phases[ph]) * NJ))
@@ -1642,7 +1672,7 @@ def lds_kernel(sub: specs.Spec, fd_order: int, kname: str, rats: Dict[str, str],
             # per phase suffices; loads run depth - 1 phases ahead.
             if depth < 2:
                 raise ValueError("single-barrier DMA staging needs at least two ring slots")
-            for ph in range(depth - 1):
+            for ph in range(1 if early_box else 0, depth - 1):
                 dma_phase(ph)
             for ph, gfs in enumerate(phases):
                 later = sum(len(phases[x]) for x in range(ph + 1, min(ph + depth - 1, len(phases)))) * NJ
@@ -1806,7 +1836,7 @@ def candidate_tu(v: specs.Variant, fd_order: int, kind: str, cand: str, ensemble
                                          interleave="io" in opts,
                                          branchless_upwind="ub" in opts, sym_lines="sa" in opts,
                                          read_batch=next((int(o[2:]) for o in opts if o[:2] == "lr" and o[2:].isdigit()), 0),
-                                         dma_spread="di" in opts, odd_rows="dmo" in opts, two_pass="tp" in opts,
+                                         dma_spread="di" in opts, odd_rows="dmo" in opts, two_pass="tp" in opts, inverse_rfm="ir" in opts, early_box="eb" in opts,
                                          pin_group=next((int(o[2:] or 0) for o in opts if o[:2] == "pg" and o[2:].isdigit() or o == "pg"), -1))
             kernels.append(src)
             calls.append(launch)
@@ -1896,6 +1926,7 @@ constexpr __host__ __device__ int gf(int G, int j) {
   return G == 0 ? 11 + j : G == 1 ? j : G == 2 ? (j < 5 ? 6 + j : 17) : 18 + j;
 }
 // NP consecutive values; NT: with the non-temporal hint
+constexpr __host__ __device__ bool ricci_reads(int g) { return (g >= 11 && g <= 16) || (g >= 17 && g <= 19); }
 template <int NP>
 struct Vec;
 template <>
@@ -2056,7 +2087,11 @@ __device__ __forceinline__ void group(const double *__restrict__ kin, const doub
     }
   }
 #pragma unroll
-  for (int j = 0; j < N; j++) y[j].template st<NT>(out + gf(G, j) * Ntot + idx);
+  for (int j = 0; j < N; j++) {
+    double *o = out + gf(G, j) * Ntot + idx;
+    if (NT && !ricci_reads(gf(G, j))) y[j].template st<true>(o);
+    else y[j].template st<false>(o);
+  }
 }
 template <int NP, bool INNER, bool NT>
 __device__ __forceinline__ void any_group(int G, const double *__restrict__ kin, const double *y_n, double *y_run,

@@ -15,6 +15,7 @@ constexpr __host__ __device__ int gf(int G, int j) {
   return G == 0 ? 11 + j : G == 1 ? j : G == 2 ? (j < 5 ? 6 + j : 17) : 18 + j;
 }
 // NP consecutive values; NT: with the non-temporal hint
+constexpr __host__ __device__ bool ricci_reads(int g) { return (g >= 11 && g <= 16) || (g >= 17 && g <= 19); }
 template <int NP>
 struct Vec;
 template <>
@@ -205,7 +206,11 @@ __device__ __forceinline__ void group(const double *__restrict__ kin, const doub
     }
   }
 #pragma unroll
-  for (int j = 0; j < N; j++) y[j].template st<NT>(out + gf(G, j) * Ntot + idx);
+  for (int j = 0; j < N; j++) {
+    double *o = out + gf(G, j) * Ntot + idx;
+    if (NT && !ricci_reads(gf(G, j))) y[j].template st<true>(o);
+    else y[j].template st<false>(o);
+  }
 }
 template <int NP, bool INNER, bool NT>
 __device__ __forceinline__ void any_group(int G, const double *__restrict__ kin, const double *y_n, double *y_run,
