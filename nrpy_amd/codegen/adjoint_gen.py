@@ -318,7 +318,8 @@ def adjoint_tu(v: specs.Variant, fd_order: int) -> str:
     # input is Y = D(u), u = y_n + sum_j c_j K_j (D acts on hDD only), so the adjoint of Y goes
     # through the transposed Jacobian of D at u and is then scattered to y_n and the K_j.
     # adj_final: the last combination (y_{n+1}, weights b_j): lamYN = J_D^T lam, lamK_j = b_j lamYN.
-    # adj_stage: stage input Y_s (weight a on K_{s-1}): lamYN += J_D^T lamY, lamK_{s-1} += a (...).
+    # adj_stage: stage input Y_s (weight a on K_{s-1}): lamYN += J_D^T lamY, lamK_{s-1} += a (...),
+    # lamY = 0.
     # The operations are those of the separate combination, Jacobian and update kernels, in the
     # same order, so the results are theirs bit for bit.
     dspec = specs.detgamma_spec(v)
@@ -328,44 +329,59 @@ def adjoint_tu(v: specs.Variant, fd_order: int) -> str:
     det_out = {bssn.EVOL_GFS.index(g): g for g, _ in dspec.outputs}
     ngf = len(bssn.EVOL_GFS)
 
-    def det_body(u_expr, lam_src: str) -> List[str]:
-        lines = [f"  const double {n} = {u_expr(bssn.EVOL_GFS.index(n))};" for n in dcentre]
+    # Bound by latency on the grids that fit a tape: four workgroups share a block of points, one
+    # for hDD with its Jacobian and three for six other gridfunctions each (16.2 -> 8.8 us for
+    # adj_stage at 96x16x4 against one thread for all 24).
+    hdd = sorted(det_out)
+    rest = [k for k in range(ngf) if k not in det_out]
+    groups = [hdd] + [rest[6 * i:6 * i + 6] for i in range(3)]
+    assert sorted(sum(groups, [])) == list(range(ngf))
+
+    def body(u_expr, lam_src: str, update) -> str:
+        lines = [f"  if (grp == 0) {{"]
+        lines += [f"  const double {n} = {u_expr(bssn.EVOL_GFS.index(n))};" for n in dcentre]
         lines += [f"  const double {n} = {RFM_EXPR[specs.RFM_SYMBOLS.index(n)]};" for n in drfm]
         lines += [f"  const double l_{g} = {lam_src}[{bssn.EVOL_GFS.index(g)} * Ntot + idx];" for g, _ in dspec.outputs]
         lines += dfwd + drev
         # the adjoint of every gridfunction after the transposed Jacobian
-        lines += [f"  const double v{k} = " + (dinputs.get(det_out[k], "0.0") if k in det_out
-                                              else f"{lam_src}[{k} * Ntot + idx]") + ";" for k in range(ngf)]
-        return lines
+        lines += [f"  const double v{k} = {dinputs.get(det_out[k], '0.0')};" for k in hdd] + update(hdd)
+        for i, ks in enumerate(groups[1:], 1):
+            lines.append(f"  }} else if (grp == {i}) {{" if i < 3 else "  } else {")
+            lines += [f"  const double v{k} = {lam_src}[{k} * Ntot + idx];" for k in ks] + update(ks)
+        return "\n".join(lines + ["  }"])
 
-    point = """  const int i0 = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    point = """  const int grp = (int)(blockIdx.x & 3u);
+  const int i0 = (int)((blockIdx.x >> 2) * blockDim.x + threadIdx.x);
   const int i1 = (int)(blockIdx.y * blockDim.y + threadIdx.y);
   const int i2 = (int)blockIdx.z;
   if (i0 >= p.Nx0 || i1 >= p.Nx1) return;
   const long Ntot = p.Ntot, nv = """ + str(ngf) + """ * Ntot;
   const long idx = i0 + p.s1 * i1 + p.s2 * i2;"""
-    final_body = det_body(lambda k: (f"y[{k} * Ntot + idx] + b0 * K[{k} * Ntot + idx] + b1 * K[nv + {k} * Ntot + idx]"
-                                     f" + b2 * K[2 * nv + {k} * Ntot + idx] + b3 * K[3 * nv + {k} * Ntot + idx]"),
-                          "lam")
-    final_body += [f"  lamYN[{k} * Ntot + idx] = v{k};" for k in range(ngf)]
-    final_body += [f"  lamK[{j} * nv + {k} * Ntot + idx] = b{j} * v{k};" for j in range(4) for k in range(ngf)]
-    stage_body = det_body(lambda k: f"y[{k} * Ntot + idx] + a * K[{k} * Ntot + idx]", "lamY")
-    stage_body += [f"  lamYN[{k} * Ntot + idx] += v{k};\n  lamK[{k} * Ntot + idx] += a * v{k};" for k in range(ngf)]
+    final_body = body(lambda k: (f"y[{k} * Ntot + idx] + b0 * K[{k} * Ntot + idx] + b1 * K[nv + {k} * Ntot + idx]"
+                                 f" + b2 * K[2 * nv + {k} * Ntot + idx] + b3 * K[3 * nv + {k} * Ntot + idx]"),
+                      "lam", lambda ks: [f"  lamYN[{k} * Ntot + idx] = v{k};" for k in ks]
+                      + [f"  lamK[{j} * nv + {k} * Ntot + idx] = b{j} * v{k};" for j in range(4) for k in ks])
+    # the stage's adjoint is used up here: it is cleared for the stage before
+    stage_body = body(lambda k: f"y[{k} * Ntot + idx] + a * K[{k} * Ntot + idx]", "lamY",
+                      lambda ks: [f"  const double w{k} = lamYN[{k} * Ntot + idx], x{k} = lamK[{k} * Ntot + idx];"
+                                  for k in ks]
+                      + [f"  lamYN[{k} * Ntot + idx] = w{k} + v{k};\n  lamK[{k} * Ntot + idx] = x{k} + a * v{k};\n"
+                         f"  lamY[{k} * Ntot + idx] = 0.0;" for k in ks])
     adj_rk = f"""
 extern "C" __global__ void __launch_bounds__(256)
 adj_final_{tag}(const double *__restrict__ y, const double *__restrict__ K, double b0, double b1, double b2,
                 double b3, const double *__restrict__ lam, double *__restrict__ lamYN, double *__restrict__ lamK,
                 const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p) {{
 {point}
-{chr(10).join(final_body)}
+{final_body}
 }}
 
 extern "C" __global__ void __launch_bounds__(256)
 adj_stage_{tag}(const double *__restrict__ y, const double *__restrict__ K, double a,
-                const double *__restrict__ lamY, double *__restrict__ lamYN, double *__restrict__ lamK,
+                double *__restrict__ lamY, double *__restrict__ lamYN, double *__restrict__ lamK,
                 const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p) {{
 {point}
-{chr(10).join(stage_body)}
+{stage_body}
 }}
 """
     # ---- transposed stencils, unrolled per gridfunction: lam_y[g](q) += sum over the slots k
@@ -447,11 +463,13 @@ extern "C" hipError_t launch_adj_ricci_{tag}(dim3 g, dim3 b, hipStream_t s, cons
 extern "C" hipError_t launch_adj_final_{tag}(dim3 g, dim3 b, hipStream_t s, const double *y, const double *K,
     double b0, double b1, double b2, double b3, const double *lam, double *lamYN, double *lamK, const double *rfm0,
     const double *rfm1, bhah_kparams p) {{
+  g.x *= 4;
   hipLaunchKernelGGL(adj_final_{tag}, g, b, 0, s, y, K, b0, b1, b2, b3, lam, lamYN, lamK, rfm0, rfm1, p);
   return hipGetLastError();
 }}
 extern "C" hipError_t launch_adj_stage_{tag}(dim3 g, dim3 b, hipStream_t s, const double *y, const double *K, double a,
-    const double *lamY, double *lamYN, double *lamK, const double *rfm0, const double *rfm1, bhah_kparams p) {{
+    double *lamY, double *lamYN, double *lamK, const double *rfm0, const double *rfm1, bhah_kparams p) {{
+  g.x *= 4;
   hipLaunchKernelGGL(adj_stage_{tag}, g, b, 0, s, y, K, a, lamY, lamYN, lamK, rfm0, rfm1, p);
   return hipGetLastError();
 }}

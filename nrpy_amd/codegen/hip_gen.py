@@ -2450,7 +2450,7 @@ def generate(outdir: str) -> List[str]:
                 f"const double *, double, double, double, double, const double *, double *, double *, "
                 f"const double *, const double *, bhah_kparams);",
                 f'extern "C" hipError_t launch_adj_stage_{tag}(dim3, dim3, hipStream_t, const double *, '
-                f"const double *, double, const double *, double *, double *, const double *, const double *, "
+                f"const double *, double, double *, double *, double *, const double *, const double *, "
                 f"bhah_kparams);",
                 f'extern "C" hipError_t launch_adj_gather_{tag}(dim3, dim3, hipStream_t, const double *, double *, '
                 f"bhah_kparams);",

@@ -61,7 +61,7 @@ struct BssnKernels {
                           bhah_kparams);
   hipError_t (*adj_final)(dim3, dim3, hipStream_t, const double *, const double *, double, double, double, double,
                           const double *, double *, double *, const double *, const double *, bhah_kparams);
-  hipError_t (*adj_stage)(dim3, dim3, hipStream_t, const double *, const double *, double, const double *, double *,
+  hipError_t (*adj_stage)(dim3, dim3, hipStream_t, const double *, const double *, double, double *, double *,
                           double *, const double *, const double *, bhah_kparams);
   hipError_t (*adj_gather)(dim3, dim3, hipStream_t, const double *, double *, bhah_kparams);
 };
@@ -2588,11 +2588,11 @@ static int enqueue_reverse(bhah_patch *P, const StepTape &T, double dt, double *
   // y_{n+1} = D(y_n + sum b K): lamYN = J_D^T lam, then lamK_j = b_j lamYN
   HIP_TRY(P->k->adj_final(ga, ba, st, y_n, K, b_final[0], b_final[1], b_final[2], b_final[3], lam, W.lamYN, W.lamK,
                           P->d_rfm0, P->d_rfm1, P->kp(dt, 0)));
+  hipLaunchKernelGGL(fill_kernel, g1, b1, 0, st, W.lamY, 0.0, nv);  // adj_stage clears it for the next stage
+  HIP_TRY(hipGetLastError());
   for (int s = 4; s >= 1; s--) {
     const double *in = T.Y[s - 1], *aux = T.AUX + (s - 1) * 6 * N;
     double *lk = W.lamK + (s - 1) * nv;
-    hipLaunchKernelGGL(fill_kernel, g1, b1, 0, st, W.lamY, 0.0, nv);
-    HIP_TRY(hipGetLastError());
     if ((rc = adjoint_rhs_bcs(P, lk, W.lamY))) return rc;
     HIP_TRY(P->k->adj_rhs(gi, bi, st, in, aux, lk, W.S, P->d_rfm0, P->d_rfm1, P->kp(dt, 0)));
     HIP_TRY(P->k->adj_ricci(gi, bi, st, in, W.S, P->d_rfm0, P->d_rfm1, P->kp(dt, 0)));

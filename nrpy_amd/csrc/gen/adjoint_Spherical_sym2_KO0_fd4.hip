@@ -7207,12 +7207,14 @@ extern "C" __global__ void __launch_bounds__(256)
 adj_final_Spherical_sym2_KO0_fd4(const double *__restrict__ y, const double *__restrict__ K, double b0, double b1, double b2,
                 double b3, const double *__restrict__ lam, double *__restrict__ lamYN, double *__restrict__ lamK,
                 const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p) {
-  const int i0 = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  const int grp = (int)(blockIdx.x & 3u);
+  const int i0 = (int)((blockIdx.x >> 2) * blockDim.x + threadIdx.x);
   const int i1 = (int)(blockIdx.y * blockDim.y + threadIdx.y);
   const int i2 = (int)blockIdx.z;
   if (i0 >= p.Nx0 || i1 >= p.Nx1) return;
   const long Ntot = p.Ntot, nv = 24 * Ntot;
   const long idx = i0 + p.s1 * i1 + p.s2 * i2;
+  if (grp == 0) {
   const double hDD00 = y[11 * Ntot + idx] + b0 * K[11 * Ntot + idx] + b1 * K[nv + 11 * Ntot + idx] + b2 * K[2 * nv + 11 * Ntot + idx] + b3 * K[3 * nv + 11 * Ntot + idx];
   const double hDD01 = y[12 * Ntot + idx] + b0 * K[12 * Ntot + idx] + b1 * K[nv + 12 * Ntot + idx] + b2 * K[2 * nv + 12 * Ntot + idx] + b3 * K[3 * nv + 12 * Ntot + idx];
   const double hDD02 = y[13 * Ntot + idx] + b0 * K[13 * Ntot + idx] + b1 * K[nv + 13 * Ntot + idx] + b2 * K[2 * nv + 13 * Ntot + idx] + b3 * K[3 * nv + 13 * Ntot + idx];
@@ -7269,162 +7271,168 @@ adj_final_Spherical_sym2_KO0_fd4(const double *__restrict__ y, const double *__r
   a_f1_of_xx1 += a_w2 * (2.0*f1_of_xx1);
   a_f0_of_xx0 += a_w1 * (2.0*f0_of_xx0);
   double a_hDD00 = a_w0 * (1.0);
-  const double v0 = lam[0 * Ntot + idx];
-  const double v1 = lam[1 * Ntot + idx];
-  const double v2 = lam[2 * Ntot + idx];
-  const double v3 = lam[3 * Ntot + idx];
-  const double v4 = lam[4 * Ntot + idx];
-  const double v5 = lam[5 * Ntot + idx];
-  const double v6 = lam[6 * Ntot + idx];
-  const double v7 = lam[7 * Ntot + idx];
-  const double v8 = lam[8 * Ntot + idx];
-  const double v9 = lam[9 * Ntot + idx];
-  const double v10 = lam[10 * Ntot + idx];
   const double v11 = a_hDD00;
   const double v12 = a_hDD01;
   const double v13 = a_hDD02;
   const double v14 = a_hDD11;
   const double v15 = a_hDD12;
   const double v16 = a_hDD22;
-  const double v17 = lam[17 * Ntot + idx];
-  const double v18 = lam[18 * Ntot + idx];
-  const double v19 = lam[19 * Ntot + idx];
-  const double v20 = lam[20 * Ntot + idx];
-  const double v21 = lam[21 * Ntot + idx];
-  const double v22 = lam[22 * Ntot + idx];
-  const double v23 = lam[23 * Ntot + idx];
-  lamYN[0 * Ntot + idx] = v0;
-  lamYN[1 * Ntot + idx] = v1;
-  lamYN[2 * Ntot + idx] = v2;
-  lamYN[3 * Ntot + idx] = v3;
-  lamYN[4 * Ntot + idx] = v4;
-  lamYN[5 * Ntot + idx] = v5;
-  lamYN[6 * Ntot + idx] = v6;
-  lamYN[7 * Ntot + idx] = v7;
-  lamYN[8 * Ntot + idx] = v8;
-  lamYN[9 * Ntot + idx] = v9;
-  lamYN[10 * Ntot + idx] = v10;
   lamYN[11 * Ntot + idx] = v11;
   lamYN[12 * Ntot + idx] = v12;
   lamYN[13 * Ntot + idx] = v13;
   lamYN[14 * Ntot + idx] = v14;
   lamYN[15 * Ntot + idx] = v15;
   lamYN[16 * Ntot + idx] = v16;
-  lamYN[17 * Ntot + idx] = v17;
-  lamYN[18 * Ntot + idx] = v18;
-  lamYN[19 * Ntot + idx] = v19;
-  lamYN[20 * Ntot + idx] = v20;
-  lamYN[21 * Ntot + idx] = v21;
-  lamYN[22 * Ntot + idx] = v22;
-  lamYN[23 * Ntot + idx] = v23;
-  lamK[0 * nv + 0 * Ntot + idx] = b0 * v0;
-  lamK[0 * nv + 1 * Ntot + idx] = b0 * v1;
-  lamK[0 * nv + 2 * Ntot + idx] = b0 * v2;
-  lamK[0 * nv + 3 * Ntot + idx] = b0 * v3;
-  lamK[0 * nv + 4 * Ntot + idx] = b0 * v4;
-  lamK[0 * nv + 5 * Ntot + idx] = b0 * v5;
-  lamK[0 * nv + 6 * Ntot + idx] = b0 * v6;
-  lamK[0 * nv + 7 * Ntot + idx] = b0 * v7;
-  lamK[0 * nv + 8 * Ntot + idx] = b0 * v8;
-  lamK[0 * nv + 9 * Ntot + idx] = b0 * v9;
-  lamK[0 * nv + 10 * Ntot + idx] = b0 * v10;
   lamK[0 * nv + 11 * Ntot + idx] = b0 * v11;
   lamK[0 * nv + 12 * Ntot + idx] = b0 * v12;
   lamK[0 * nv + 13 * Ntot + idx] = b0 * v13;
   lamK[0 * nv + 14 * Ntot + idx] = b0 * v14;
   lamK[0 * nv + 15 * Ntot + idx] = b0 * v15;
   lamK[0 * nv + 16 * Ntot + idx] = b0 * v16;
-  lamK[0 * nv + 17 * Ntot + idx] = b0 * v17;
-  lamK[0 * nv + 18 * Ntot + idx] = b0 * v18;
-  lamK[0 * nv + 19 * Ntot + idx] = b0 * v19;
-  lamK[0 * nv + 20 * Ntot + idx] = b0 * v20;
-  lamK[0 * nv + 21 * Ntot + idx] = b0 * v21;
-  lamK[0 * nv + 22 * Ntot + idx] = b0 * v22;
-  lamK[0 * nv + 23 * Ntot + idx] = b0 * v23;
-  lamK[1 * nv + 0 * Ntot + idx] = b1 * v0;
-  lamK[1 * nv + 1 * Ntot + idx] = b1 * v1;
-  lamK[1 * nv + 2 * Ntot + idx] = b1 * v2;
-  lamK[1 * nv + 3 * Ntot + idx] = b1 * v3;
-  lamK[1 * nv + 4 * Ntot + idx] = b1 * v4;
-  lamK[1 * nv + 5 * Ntot + idx] = b1 * v5;
-  lamK[1 * nv + 6 * Ntot + idx] = b1 * v6;
-  lamK[1 * nv + 7 * Ntot + idx] = b1 * v7;
-  lamK[1 * nv + 8 * Ntot + idx] = b1 * v8;
-  lamK[1 * nv + 9 * Ntot + idx] = b1 * v9;
-  lamK[1 * nv + 10 * Ntot + idx] = b1 * v10;
   lamK[1 * nv + 11 * Ntot + idx] = b1 * v11;
   lamK[1 * nv + 12 * Ntot + idx] = b1 * v12;
   lamK[1 * nv + 13 * Ntot + idx] = b1 * v13;
   lamK[1 * nv + 14 * Ntot + idx] = b1 * v14;
   lamK[1 * nv + 15 * Ntot + idx] = b1 * v15;
   lamK[1 * nv + 16 * Ntot + idx] = b1 * v16;
-  lamK[1 * nv + 17 * Ntot + idx] = b1 * v17;
-  lamK[1 * nv + 18 * Ntot + idx] = b1 * v18;
-  lamK[1 * nv + 19 * Ntot + idx] = b1 * v19;
-  lamK[1 * nv + 20 * Ntot + idx] = b1 * v20;
-  lamK[1 * nv + 21 * Ntot + idx] = b1 * v21;
-  lamK[1 * nv + 22 * Ntot + idx] = b1 * v22;
-  lamK[1 * nv + 23 * Ntot + idx] = b1 * v23;
-  lamK[2 * nv + 0 * Ntot + idx] = b2 * v0;
-  lamK[2 * nv + 1 * Ntot + idx] = b2 * v1;
-  lamK[2 * nv + 2 * Ntot + idx] = b2 * v2;
-  lamK[2 * nv + 3 * Ntot + idx] = b2 * v3;
-  lamK[2 * nv + 4 * Ntot + idx] = b2 * v4;
-  lamK[2 * nv + 5 * Ntot + idx] = b2 * v5;
-  lamK[2 * nv + 6 * Ntot + idx] = b2 * v6;
-  lamK[2 * nv + 7 * Ntot + idx] = b2 * v7;
-  lamK[2 * nv + 8 * Ntot + idx] = b2 * v8;
-  lamK[2 * nv + 9 * Ntot + idx] = b2 * v9;
-  lamK[2 * nv + 10 * Ntot + idx] = b2 * v10;
   lamK[2 * nv + 11 * Ntot + idx] = b2 * v11;
   lamK[2 * nv + 12 * Ntot + idx] = b2 * v12;
   lamK[2 * nv + 13 * Ntot + idx] = b2 * v13;
   lamK[2 * nv + 14 * Ntot + idx] = b2 * v14;
   lamK[2 * nv + 15 * Ntot + idx] = b2 * v15;
   lamK[2 * nv + 16 * Ntot + idx] = b2 * v16;
-  lamK[2 * nv + 17 * Ntot + idx] = b2 * v17;
-  lamK[2 * nv + 18 * Ntot + idx] = b2 * v18;
-  lamK[2 * nv + 19 * Ntot + idx] = b2 * v19;
-  lamK[2 * nv + 20 * Ntot + idx] = b2 * v20;
-  lamK[2 * nv + 21 * Ntot + idx] = b2 * v21;
-  lamK[2 * nv + 22 * Ntot + idx] = b2 * v22;
-  lamK[2 * nv + 23 * Ntot + idx] = b2 * v23;
-  lamK[3 * nv + 0 * Ntot + idx] = b3 * v0;
-  lamK[3 * nv + 1 * Ntot + idx] = b3 * v1;
-  lamK[3 * nv + 2 * Ntot + idx] = b3 * v2;
-  lamK[3 * nv + 3 * Ntot + idx] = b3 * v3;
-  lamK[3 * nv + 4 * Ntot + idx] = b3 * v4;
-  lamK[3 * nv + 5 * Ntot + idx] = b3 * v5;
-  lamK[3 * nv + 6 * Ntot + idx] = b3 * v6;
-  lamK[3 * nv + 7 * Ntot + idx] = b3 * v7;
-  lamK[3 * nv + 8 * Ntot + idx] = b3 * v8;
-  lamK[3 * nv + 9 * Ntot + idx] = b3 * v9;
-  lamK[3 * nv + 10 * Ntot + idx] = b3 * v10;
   lamK[3 * nv + 11 * Ntot + idx] = b3 * v11;
   lamK[3 * nv + 12 * Ntot + idx] = b3 * v12;
   lamK[3 * nv + 13 * Ntot + idx] = b3 * v13;
   lamK[3 * nv + 14 * Ntot + idx] = b3 * v14;
   lamK[3 * nv + 15 * Ntot + idx] = b3 * v15;
   lamK[3 * nv + 16 * Ntot + idx] = b3 * v16;
+  } else if (grp == 1) {
+  const double v0 = lam[0 * Ntot + idx];
+  const double v1 = lam[1 * Ntot + idx];
+  const double v2 = lam[2 * Ntot + idx];
+  const double v3 = lam[3 * Ntot + idx];
+  const double v4 = lam[4 * Ntot + idx];
+  const double v5 = lam[5 * Ntot + idx];
+  lamYN[0 * Ntot + idx] = v0;
+  lamYN[1 * Ntot + idx] = v1;
+  lamYN[2 * Ntot + idx] = v2;
+  lamYN[3 * Ntot + idx] = v3;
+  lamYN[4 * Ntot + idx] = v4;
+  lamYN[5 * Ntot + idx] = v5;
+  lamK[0 * nv + 0 * Ntot + idx] = b0 * v0;
+  lamK[0 * nv + 1 * Ntot + idx] = b0 * v1;
+  lamK[0 * nv + 2 * Ntot + idx] = b0 * v2;
+  lamK[0 * nv + 3 * Ntot + idx] = b0 * v3;
+  lamK[0 * nv + 4 * Ntot + idx] = b0 * v4;
+  lamK[0 * nv + 5 * Ntot + idx] = b0 * v5;
+  lamK[1 * nv + 0 * Ntot + idx] = b1 * v0;
+  lamK[1 * nv + 1 * Ntot + idx] = b1 * v1;
+  lamK[1 * nv + 2 * Ntot + idx] = b1 * v2;
+  lamK[1 * nv + 3 * Ntot + idx] = b1 * v3;
+  lamK[1 * nv + 4 * Ntot + idx] = b1 * v4;
+  lamK[1 * nv + 5 * Ntot + idx] = b1 * v5;
+  lamK[2 * nv + 0 * Ntot + idx] = b2 * v0;
+  lamK[2 * nv + 1 * Ntot + idx] = b2 * v1;
+  lamK[2 * nv + 2 * Ntot + idx] = b2 * v2;
+  lamK[2 * nv + 3 * Ntot + idx] = b2 * v3;
+  lamK[2 * nv + 4 * Ntot + idx] = b2 * v4;
+  lamK[2 * nv + 5 * Ntot + idx] = b2 * v5;
+  lamK[3 * nv + 0 * Ntot + idx] = b3 * v0;
+  lamK[3 * nv + 1 * Ntot + idx] = b3 * v1;
+  lamK[3 * nv + 2 * Ntot + idx] = b3 * v2;
+  lamK[3 * nv + 3 * Ntot + idx] = b3 * v3;
+  lamK[3 * nv + 4 * Ntot + idx] = b3 * v4;
+  lamK[3 * nv + 5 * Ntot + idx] = b3 * v5;
+  } else if (grp == 2) {
+  const double v6 = lam[6 * Ntot + idx];
+  const double v7 = lam[7 * Ntot + idx];
+  const double v8 = lam[8 * Ntot + idx];
+  const double v9 = lam[9 * Ntot + idx];
+  const double v10 = lam[10 * Ntot + idx];
+  const double v17 = lam[17 * Ntot + idx];
+  lamYN[6 * Ntot + idx] = v6;
+  lamYN[7 * Ntot + idx] = v7;
+  lamYN[8 * Ntot + idx] = v8;
+  lamYN[9 * Ntot + idx] = v9;
+  lamYN[10 * Ntot + idx] = v10;
+  lamYN[17 * Ntot + idx] = v17;
+  lamK[0 * nv + 6 * Ntot + idx] = b0 * v6;
+  lamK[0 * nv + 7 * Ntot + idx] = b0 * v7;
+  lamK[0 * nv + 8 * Ntot + idx] = b0 * v8;
+  lamK[0 * nv + 9 * Ntot + idx] = b0 * v9;
+  lamK[0 * nv + 10 * Ntot + idx] = b0 * v10;
+  lamK[0 * nv + 17 * Ntot + idx] = b0 * v17;
+  lamK[1 * nv + 6 * Ntot + idx] = b1 * v6;
+  lamK[1 * nv + 7 * Ntot + idx] = b1 * v7;
+  lamK[1 * nv + 8 * Ntot + idx] = b1 * v8;
+  lamK[1 * nv + 9 * Ntot + idx] = b1 * v9;
+  lamK[1 * nv + 10 * Ntot + idx] = b1 * v10;
+  lamK[1 * nv + 17 * Ntot + idx] = b1 * v17;
+  lamK[2 * nv + 6 * Ntot + idx] = b2 * v6;
+  lamK[2 * nv + 7 * Ntot + idx] = b2 * v7;
+  lamK[2 * nv + 8 * Ntot + idx] = b2 * v8;
+  lamK[2 * nv + 9 * Ntot + idx] = b2 * v9;
+  lamK[2 * nv + 10 * Ntot + idx] = b2 * v10;
+  lamK[2 * nv + 17 * Ntot + idx] = b2 * v17;
+  lamK[3 * nv + 6 * Ntot + idx] = b3 * v6;
+  lamK[3 * nv + 7 * Ntot + idx] = b3 * v7;
+  lamK[3 * nv + 8 * Ntot + idx] = b3 * v8;
+  lamK[3 * nv + 9 * Ntot + idx] = b3 * v9;
+  lamK[3 * nv + 10 * Ntot + idx] = b3 * v10;
   lamK[3 * nv + 17 * Ntot + idx] = b3 * v17;
+  } else {
+  const double v18 = lam[18 * Ntot + idx];
+  const double v19 = lam[19 * Ntot + idx];
+  const double v20 = lam[20 * Ntot + idx];
+  const double v21 = lam[21 * Ntot + idx];
+  const double v22 = lam[22 * Ntot + idx];
+  const double v23 = lam[23 * Ntot + idx];
+  lamYN[18 * Ntot + idx] = v18;
+  lamYN[19 * Ntot + idx] = v19;
+  lamYN[20 * Ntot + idx] = v20;
+  lamYN[21 * Ntot + idx] = v21;
+  lamYN[22 * Ntot + idx] = v22;
+  lamYN[23 * Ntot + idx] = v23;
+  lamK[0 * nv + 18 * Ntot + idx] = b0 * v18;
+  lamK[0 * nv + 19 * Ntot + idx] = b0 * v19;
+  lamK[0 * nv + 20 * Ntot + idx] = b0 * v20;
+  lamK[0 * nv + 21 * Ntot + idx] = b0 * v21;
+  lamK[0 * nv + 22 * Ntot + idx] = b0 * v22;
+  lamK[0 * nv + 23 * Ntot + idx] = b0 * v23;
+  lamK[1 * nv + 18 * Ntot + idx] = b1 * v18;
+  lamK[1 * nv + 19 * Ntot + idx] = b1 * v19;
+  lamK[1 * nv + 20 * Ntot + idx] = b1 * v20;
+  lamK[1 * nv + 21 * Ntot + idx] = b1 * v21;
+  lamK[1 * nv + 22 * Ntot + idx] = b1 * v22;
+  lamK[1 * nv + 23 * Ntot + idx] = b1 * v23;
+  lamK[2 * nv + 18 * Ntot + idx] = b2 * v18;
+  lamK[2 * nv + 19 * Ntot + idx] = b2 * v19;
+  lamK[2 * nv + 20 * Ntot + idx] = b2 * v20;
+  lamK[2 * nv + 21 * Ntot + idx] = b2 * v21;
+  lamK[2 * nv + 22 * Ntot + idx] = b2 * v22;
+  lamK[2 * nv + 23 * Ntot + idx] = b2 * v23;
   lamK[3 * nv + 18 * Ntot + idx] = b3 * v18;
   lamK[3 * nv + 19 * Ntot + idx] = b3 * v19;
   lamK[3 * nv + 20 * Ntot + idx] = b3 * v20;
   lamK[3 * nv + 21 * Ntot + idx] = b3 * v21;
   lamK[3 * nv + 22 * Ntot + idx] = b3 * v22;
   lamK[3 * nv + 23 * Ntot + idx] = b3 * v23;
+  }
 }
 
 extern "C" __global__ void __launch_bounds__(256)
 adj_stage_Spherical_sym2_KO0_fd4(const double *__restrict__ y, const double *__restrict__ K, double a,
-                const double *__restrict__ lamY, double *__restrict__ lamYN, double *__restrict__ lamK,
+                double *__restrict__ lamY, double *__restrict__ lamYN, double *__restrict__ lamK,
                 const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p) {
-  const int i0 = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  const int grp = (int)(blockIdx.x & 3u);
+  const int i0 = (int)((blockIdx.x >> 2) * blockDim.x + threadIdx.x);
   const int i1 = (int)(blockIdx.y * blockDim.y + threadIdx.y);
   const int i2 = (int)blockIdx.z;
   if (i0 >= p.Nx0 || i1 >= p.Nx1) return;
   const long Ntot = p.Ntot, nv = 24 * Ntot;
   const long idx = i0 + p.s1 * i1 + p.s2 * i2;
+  if (grp == 0) {
   const double hDD00 = y[11 * Ntot + idx] + a * K[11 * Ntot + idx];
   const double hDD01 = y[12 * Ntot + idx] + a * K[12 * Ntot + idx];
   const double hDD02 = y[13 * Ntot + idx] + a * K[13 * Ntot + idx];
@@ -7481,78 +7489,130 @@ adj_stage_Spherical_sym2_KO0_fd4(const double *__restrict__ y, const double *__r
   a_f1_of_xx1 += a_w2 * (2.0*f1_of_xx1);
   a_f0_of_xx0 += a_w1 * (2.0*f0_of_xx0);
   double a_hDD00 = a_w0 * (1.0);
-  const double v0 = lamY[0 * Ntot + idx];
-  const double v1 = lamY[1 * Ntot + idx];
-  const double v2 = lamY[2 * Ntot + idx];
-  const double v3 = lamY[3 * Ntot + idx];
-  const double v4 = lamY[4 * Ntot + idx];
-  const double v5 = lamY[5 * Ntot + idx];
-  const double v6 = lamY[6 * Ntot + idx];
-  const double v7 = lamY[7 * Ntot + idx];
-  const double v8 = lamY[8 * Ntot + idx];
-  const double v9 = lamY[9 * Ntot + idx];
-  const double v10 = lamY[10 * Ntot + idx];
   const double v11 = a_hDD00;
   const double v12 = a_hDD01;
   const double v13 = a_hDD02;
   const double v14 = a_hDD11;
   const double v15 = a_hDD12;
   const double v16 = a_hDD22;
+  const double w11 = lamYN[11 * Ntot + idx], x11 = lamK[11 * Ntot + idx];
+  const double w12 = lamYN[12 * Ntot + idx], x12 = lamK[12 * Ntot + idx];
+  const double w13 = lamYN[13 * Ntot + idx], x13 = lamK[13 * Ntot + idx];
+  const double w14 = lamYN[14 * Ntot + idx], x14 = lamK[14 * Ntot + idx];
+  const double w15 = lamYN[15 * Ntot + idx], x15 = lamK[15 * Ntot + idx];
+  const double w16 = lamYN[16 * Ntot + idx], x16 = lamK[16 * Ntot + idx];
+  lamYN[11 * Ntot + idx] = w11 + v11;
+  lamK[11 * Ntot + idx] = x11 + a * v11;
+  lamY[11 * Ntot + idx] = 0.0;
+  lamYN[12 * Ntot + idx] = w12 + v12;
+  lamK[12 * Ntot + idx] = x12 + a * v12;
+  lamY[12 * Ntot + idx] = 0.0;
+  lamYN[13 * Ntot + idx] = w13 + v13;
+  lamK[13 * Ntot + idx] = x13 + a * v13;
+  lamY[13 * Ntot + idx] = 0.0;
+  lamYN[14 * Ntot + idx] = w14 + v14;
+  lamK[14 * Ntot + idx] = x14 + a * v14;
+  lamY[14 * Ntot + idx] = 0.0;
+  lamYN[15 * Ntot + idx] = w15 + v15;
+  lamK[15 * Ntot + idx] = x15 + a * v15;
+  lamY[15 * Ntot + idx] = 0.0;
+  lamYN[16 * Ntot + idx] = w16 + v16;
+  lamK[16 * Ntot + idx] = x16 + a * v16;
+  lamY[16 * Ntot + idx] = 0.0;
+  } else if (grp == 1) {
+  const double v0 = lamY[0 * Ntot + idx];
+  const double v1 = lamY[1 * Ntot + idx];
+  const double v2 = lamY[2 * Ntot + idx];
+  const double v3 = lamY[3 * Ntot + idx];
+  const double v4 = lamY[4 * Ntot + idx];
+  const double v5 = lamY[5 * Ntot + idx];
+  const double w0 = lamYN[0 * Ntot + idx], x0 = lamK[0 * Ntot + idx];
+  const double w1 = lamYN[1 * Ntot + idx], x1 = lamK[1 * Ntot + idx];
+  const double w2 = lamYN[2 * Ntot + idx], x2 = lamK[2 * Ntot + idx];
+  const double w3 = lamYN[3 * Ntot + idx], x3 = lamK[3 * Ntot + idx];
+  const double w4 = lamYN[4 * Ntot + idx], x4 = lamK[4 * Ntot + idx];
+  const double w5 = lamYN[5 * Ntot + idx], x5 = lamK[5 * Ntot + idx];
+  lamYN[0 * Ntot + idx] = w0 + v0;
+  lamK[0 * Ntot + idx] = x0 + a * v0;
+  lamY[0 * Ntot + idx] = 0.0;
+  lamYN[1 * Ntot + idx] = w1 + v1;
+  lamK[1 * Ntot + idx] = x1 + a * v1;
+  lamY[1 * Ntot + idx] = 0.0;
+  lamYN[2 * Ntot + idx] = w2 + v2;
+  lamK[2 * Ntot + idx] = x2 + a * v2;
+  lamY[2 * Ntot + idx] = 0.0;
+  lamYN[3 * Ntot + idx] = w3 + v3;
+  lamK[3 * Ntot + idx] = x3 + a * v3;
+  lamY[3 * Ntot + idx] = 0.0;
+  lamYN[4 * Ntot + idx] = w4 + v4;
+  lamK[4 * Ntot + idx] = x4 + a * v4;
+  lamY[4 * Ntot + idx] = 0.0;
+  lamYN[5 * Ntot + idx] = w5 + v5;
+  lamK[5 * Ntot + idx] = x5 + a * v5;
+  lamY[5 * Ntot + idx] = 0.0;
+  } else if (grp == 2) {
+  const double v6 = lamY[6 * Ntot + idx];
+  const double v7 = lamY[7 * Ntot + idx];
+  const double v8 = lamY[8 * Ntot + idx];
+  const double v9 = lamY[9 * Ntot + idx];
+  const double v10 = lamY[10 * Ntot + idx];
   const double v17 = lamY[17 * Ntot + idx];
+  const double w6 = lamYN[6 * Ntot + idx], x6 = lamK[6 * Ntot + idx];
+  const double w7 = lamYN[7 * Ntot + idx], x7 = lamK[7 * Ntot + idx];
+  const double w8 = lamYN[8 * Ntot + idx], x8 = lamK[8 * Ntot + idx];
+  const double w9 = lamYN[9 * Ntot + idx], x9 = lamK[9 * Ntot + idx];
+  const double w10 = lamYN[10 * Ntot + idx], x10 = lamK[10 * Ntot + idx];
+  const double w17 = lamYN[17 * Ntot + idx], x17 = lamK[17 * Ntot + idx];
+  lamYN[6 * Ntot + idx] = w6 + v6;
+  lamK[6 * Ntot + idx] = x6 + a * v6;
+  lamY[6 * Ntot + idx] = 0.0;
+  lamYN[7 * Ntot + idx] = w7 + v7;
+  lamK[7 * Ntot + idx] = x7 + a * v7;
+  lamY[7 * Ntot + idx] = 0.0;
+  lamYN[8 * Ntot + idx] = w8 + v8;
+  lamK[8 * Ntot + idx] = x8 + a * v8;
+  lamY[8 * Ntot + idx] = 0.0;
+  lamYN[9 * Ntot + idx] = w9 + v9;
+  lamK[9 * Ntot + idx] = x9 + a * v9;
+  lamY[9 * Ntot + idx] = 0.0;
+  lamYN[10 * Ntot + idx] = w10 + v10;
+  lamK[10 * Ntot + idx] = x10 + a * v10;
+  lamY[10 * Ntot + idx] = 0.0;
+  lamYN[17 * Ntot + idx] = w17 + v17;
+  lamK[17 * Ntot + idx] = x17 + a * v17;
+  lamY[17 * Ntot + idx] = 0.0;
+  } else {
   const double v18 = lamY[18 * Ntot + idx];
   const double v19 = lamY[19 * Ntot + idx];
   const double v20 = lamY[20 * Ntot + idx];
   const double v21 = lamY[21 * Ntot + idx];
   const double v22 = lamY[22 * Ntot + idx];
   const double v23 = lamY[23 * Ntot + idx];
-  lamYN[0 * Ntot + idx] += v0;
-  lamK[0 * Ntot + idx] += a * v0;
-  lamYN[1 * Ntot + idx] += v1;
-  lamK[1 * Ntot + idx] += a * v1;
-  lamYN[2 * Ntot + idx] += v2;
-  lamK[2 * Ntot + idx] += a * v2;
-  lamYN[3 * Ntot + idx] += v3;
-  lamK[3 * Ntot + idx] += a * v3;
-  lamYN[4 * Ntot + idx] += v4;
-  lamK[4 * Ntot + idx] += a * v4;
-  lamYN[5 * Ntot + idx] += v5;
-  lamK[5 * Ntot + idx] += a * v5;
-  lamYN[6 * Ntot + idx] += v6;
-  lamK[6 * Ntot + idx] += a * v6;
-  lamYN[7 * Ntot + idx] += v7;
-  lamK[7 * Ntot + idx] += a * v7;
-  lamYN[8 * Ntot + idx] += v8;
-  lamK[8 * Ntot + idx] += a * v8;
-  lamYN[9 * Ntot + idx] += v9;
-  lamK[9 * Ntot + idx] += a * v9;
-  lamYN[10 * Ntot + idx] += v10;
-  lamK[10 * Ntot + idx] += a * v10;
-  lamYN[11 * Ntot + idx] += v11;
-  lamK[11 * Ntot + idx] += a * v11;
-  lamYN[12 * Ntot + idx] += v12;
-  lamK[12 * Ntot + idx] += a * v12;
-  lamYN[13 * Ntot + idx] += v13;
-  lamK[13 * Ntot + idx] += a * v13;
-  lamYN[14 * Ntot + idx] += v14;
-  lamK[14 * Ntot + idx] += a * v14;
-  lamYN[15 * Ntot + idx] += v15;
-  lamK[15 * Ntot + idx] += a * v15;
-  lamYN[16 * Ntot + idx] += v16;
-  lamK[16 * Ntot + idx] += a * v16;
-  lamYN[17 * Ntot + idx] += v17;
-  lamK[17 * Ntot + idx] += a * v17;
-  lamYN[18 * Ntot + idx] += v18;
-  lamK[18 * Ntot + idx] += a * v18;
-  lamYN[19 * Ntot + idx] += v19;
-  lamK[19 * Ntot + idx] += a * v19;
-  lamYN[20 * Ntot + idx] += v20;
-  lamK[20 * Ntot + idx] += a * v20;
-  lamYN[21 * Ntot + idx] += v21;
-  lamK[21 * Ntot + idx] += a * v21;
-  lamYN[22 * Ntot + idx] += v22;
-  lamK[22 * Ntot + idx] += a * v22;
-  lamYN[23 * Ntot + idx] += v23;
-  lamK[23 * Ntot + idx] += a * v23;
+  const double w18 = lamYN[18 * Ntot + idx], x18 = lamK[18 * Ntot + idx];
+  const double w19 = lamYN[19 * Ntot + idx], x19 = lamK[19 * Ntot + idx];
+  const double w20 = lamYN[20 * Ntot + idx], x20 = lamK[20 * Ntot + idx];
+  const double w21 = lamYN[21 * Ntot + idx], x21 = lamK[21 * Ntot + idx];
+  const double w22 = lamYN[22 * Ntot + idx], x22 = lamK[22 * Ntot + idx];
+  const double w23 = lamYN[23 * Ntot + idx], x23 = lamK[23 * Ntot + idx];
+  lamYN[18 * Ntot + idx] = w18 + v18;
+  lamK[18 * Ntot + idx] = x18 + a * v18;
+  lamY[18 * Ntot + idx] = 0.0;
+  lamYN[19 * Ntot + idx] = w19 + v19;
+  lamK[19 * Ntot + idx] = x19 + a * v19;
+  lamY[19 * Ntot + idx] = 0.0;
+  lamYN[20 * Ntot + idx] = w20 + v20;
+  lamK[20 * Ntot + idx] = x20 + a * v20;
+  lamY[20 * Ntot + idx] = 0.0;
+  lamYN[21 * Ntot + idx] = w21 + v21;
+  lamK[21 * Ntot + idx] = x21 + a * v21;
+  lamY[21 * Ntot + idx] = 0.0;
+  lamYN[22 * Ntot + idx] = w22 + v22;
+  lamK[22 * Ntot + idx] = x22 + a * v22;
+  lamY[22 * Ntot + idx] = 0.0;
+  lamYN[23 * Ntot + idx] = w23 + v23;
+  lamK[23 * Ntot + idx] = x23 + a * v23;
+  lamY[23 * Ntot + idx] = 0.0;
+  }
 }
 
 __device__ __forceinline__ double adjg_tap(const double *__restrict__ Sk, long j, long Ntot, unsigned ok) {
@@ -8654,11 +8714,13 @@ extern "C" hipError_t launch_adj_ricci_Spherical_sym2_KO0_fd4(dim3 g, dim3 b, hi
 extern "C" hipError_t launch_adj_final_Spherical_sym2_KO0_fd4(dim3 g, dim3 b, hipStream_t s, const double *y, const double *K,
     double b0, double b1, double b2, double b3, const double *lam, double *lamYN, double *lamK, const double *rfm0,
     const double *rfm1, bhah_kparams p) {
+  g.x *= 4;
   hipLaunchKernelGGL(adj_final_Spherical_sym2_KO0_fd4, g, b, 0, s, y, K, b0, b1, b2, b3, lam, lamYN, lamK, rfm0, rfm1, p);
   return hipGetLastError();
 }
 extern "C" hipError_t launch_adj_stage_Spherical_sym2_KO0_fd4(dim3 g, dim3 b, hipStream_t s, const double *y, const double *K, double a,
-    const double *lamY, double *lamYN, double *lamK, const double *rfm0, const double *rfm1, bhah_kparams p) {
+    double *lamY, double *lamYN, double *lamK, const double *rfm0, const double *rfm1, bhah_kparams p) {
+  g.x *= 4;
   hipLaunchKernelGGL(adj_stage_Spherical_sym2_KO0_fd4, g, b, 0, s, y, K, a, lamY, lamYN, lamK, rfm0, rfm1, p);
   return hipGetLastError();
 }
