@@ -1686,7 +1686,6 @@ static int setup_on_device(bhah_patch &P, std::vector<double> &rfm0, std::vector
   return BHAH_OK;
 }
 
-// Upload the set-up to the device and finish the patch (both set-up paths).
 // d_inner_map and d_inner_pairs, from the inner points on the device.
 static int inner_maps(bhah_patch *P, int n_inner) {
   HIP_TRY(hipMalloc((void **)&P->d_inner_map, sizeof(int2) * (size_t)P->Ntot));
@@ -1707,6 +1706,7 @@ static int inner_maps(bhah_patch *P, int n_inner) {
   return BHAH_OK;
 }
 
+// Upload the set-up to the device and finish the patch (both set-up paths).
 static int patch_upload(bhah_patch *P, const std::vector<double> &rfm0, const std::vector<double> &rfm1,
                         bhah_patch **out) {
   const bhah_patch_desc &d = P->d;
