@@ -64,6 +64,9 @@ struct BssnKernels {
   hipError_t (*adj_stage)(dim3, dim3, hipStream_t, const double *, const double *, double, double *, double *,
                           double *, const double *, const double *, bhah_kparams);
   hipError_t (*adj_gather)(dim3, dim3, hipStream_t, const double *, double *, bhah_kparams);
+  // rk_det_inner that also writes k at the inner ghost points
+  hipError_t (*rk_det_taped)(hipStream_t, double *, const double *, double *, double *, const double *, const double *,
+                             bhah_kparams, const int *, const int *);
 };
 #include "gen/kernel_table.inc"
 
@@ -2534,11 +2537,15 @@ static int enqueue_stages(bhah_patch *P, const StepTape &T, double *yrun, double
     double *in = T.Y[s - 1], *k = T.K + (s - 1) * nv, *aux = T.AUX + (s - 1) * 6 * N;
     if ((rc = bhah_hip_Ricci_eval(P, in, aux))) return rc;
     if ((rc = bhah_hip_rhs_eval(P, aux, in, k))) return rc;
+    double *next = (s < 4) ? T.Y[s] : y_next;
+    if (next && P->fold_inner && P->d_inner_map) {
+      if ((rc = apply_bcs_outerradiation(P, in, k))) return rc;
+      HIP_TRY(P->k->rk_det_taped(P->stream, k, T.Y[0], yrun, next, P->d_rfm0, P->d_rfm1, P->kp(dt, s), P->d_inner_map,
+                                 P->d_inner_pairs));
+      continue;
+    }
     if ((rc = bhah_hip_apply_bcs_outerradiation_and_inner(P, in, k))) return rc;
-    if (s < 4)
-      HIP_TRY(P->k->rk_det(P->stream, k, T.Y[0], yrun, T.Y[s], P->d_rfm0, P->d_rfm1, P->kp(dt, s)));
-    else if (y_next)
-      HIP_TRY(P->k->rk_det(P->stream, k, T.Y[0], yrun, y_next, P->d_rfm0, P->d_rfm1, P->kp(dt, s)));
+    if (next) HIP_TRY(P->k->rk_det(P->stream, k, T.Y[0], yrun, next, P->d_rfm0, P->d_rfm1, P->kp(dt, s)));
   }
   return BHAH_OK;
 }

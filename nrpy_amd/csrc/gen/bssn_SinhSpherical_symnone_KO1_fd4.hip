@@ -105,8 +105,37 @@ __device__ __forceinline__ void at_source(Vec<NP> (&r)[6], const double *f, cons
     }
   }
 }
-template <int G, int NP, bool INNER, bool NT>
-__device__ __forceinline__ void group(const double *__restrict__ kin, const double *y_n, double *y_run, double *out,
+// KEEP: the pass also writes k at inner ghost points, which a taped step keeps.
+template <bool KEEP>
+struct KPtr {
+  typedef const double *__restrict__ type;
+};
+template <>
+struct KPtr<true> {
+  typedef double *type;
+};
+template <bool KEEP>
+using k_ptr = typename KPtr<KEEP>::type;
+// Write the inner ghost points' k among this thread's points: each point's own thread writes it, and
+// no thread takes a value from it (sources are never inner ghost points).
+template <int G, int NP>
+__device__ __forceinline__ void keep_ghosts(double *f, const Vec<NP> (&k)[6], const long Ntot, const Source &S,
+                                            const long idx) {
+  const bool g0 = (NP == 2 && S.split) ? S.s0 != idx : S.from != idx || (NP == 2 && (S.code & 1u));
+  const bool g1 = NP == 2 && (S.split ? S.s1 != idx + 1 : S.from != idx || !(S.code & 2u));
+#pragma unroll
+  for (int j = 0; j < 6; j++) {
+    double *o = f + gf(G, j) * Ntot + idx;
+    if (NP == 2 && g0 && g1) {
+      k[j].template st<false>(o);
+    } else {
+      if (g0) o[0] = k[j].v[0];
+      if (g1) o[1] = k[j].v[NP - 1];
+    }
+  }
+}
+template <int G, int NP, bool INNER, bool NT, bool KEEP>
+__device__ __forceinline__ void group(k_ptr<KEEP> kin, const double *y_n, double *y_run, double *out,
                                       const double *__restrict__ rfm0, const double *__restrict__ rfm1,
                                       const bhah_kparams &p, const int2 *__restrict__ map,
                                       const int2 *__restrict__ pairs, const long q) {
@@ -213,26 +242,27 @@ __device__ __forceinline__ void group(const double *__restrict__ kin, const doub
     if (NT && !ricci_reads(gf(G, j))) y[j].template st<true>(o);
     else y[j].template st<false>(o);
   }
+  if constexpr (KEEP) keep_ghosts<G, NP>(kin, k, Ntot, S, idx);
 }
-template <int NP, bool INNER, bool NT>
-__device__ __forceinline__ void any_group(int G, const double *__restrict__ kin, const double *y_n, double *y_run,
+template <int NP, bool INNER, bool NT, bool KEEP>
+__device__ __forceinline__ void any_group(int G, k_ptr<KEEP> kin, const double *y_n, double *y_run,
                                           double *out, const double *__restrict__ rfm0,
                                           const double *__restrict__ rfm1, const bhah_kparams &p,
                                           const int2 *__restrict__ map, const int2 *__restrict__ pairs,
                                           const long q) {
   if (q * NP >= p.Ntot) return;
-  if (G == 0) group<0, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
-  else if (G == 1) group<1, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
-  else if (G == 2) group<2, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
-  else group<3, NP, INNER, NT>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+  if (G == 0) group<0, NP, INNER, NT, KEEP>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+  else if (G == 1) group<1, NP, INNER, NT, KEEP>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+  else if (G == 2) group<2, NP, INNER, NT, KEEP>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
+  else group<3, NP, INNER, NT, KEEP>(kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs, q);
 }
 }  // namespace rk_SinhSpherical_symnone_KO1_fd4
-template <int NP, bool INNER, bool NT>
+template <int NP, bool INNER, bool NT, bool KEEP>
 __global__ void __launch_bounds__(256)
-bssn_rk_det_SinhSpherical_symnone_KO1_fd4(const double *__restrict__ kin, const double *y_n, double *y_run, double *out,
+bssn_rk_det_SinhSpherical_symnone_KO1_fd4(rk_SinhSpherical_symnone_KO1_fd4::k_ptr<KEEP> kin, const double *y_n, double *y_run, double *out,
                   const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p,
                   const int2 *__restrict__ map, const int2 *__restrict__ pairs) {
-  rk_SinhSpherical_symnone_KO1_fd4::any_group<NP, INNER, NT>((int)(blockIdx.x & 3u), kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs,
+  rk_SinhSpherical_symnone_KO1_fd4::any_group<NP, INNER, NT, KEEP>((int)(blockIdx.x & 3u), kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs,
                                  (long)(blockIdx.x >> 2) * blockDim.x + threadIdx.x);
 }
 
@@ -867,7 +897,8 @@ bssn_initial_lambda_SinhSpherical_symnone_KO1_fd4(double *gfs, const double *__r
 #undef Rational_1_2
 #undef Rational_2_3
 
-static hipError_t rk_det_launch_SinhSpherical_symnone_KO1_fd4(hipStream_t s, const double *kin, const double *y_n, double *y_run, double *out,
+template <bool KEEP>
+static hipError_t rk_det_launch_SinhSpherical_symnone_KO1_fd4(hipStream_t s, rk_SinhSpherical_symnone_KO1_fd4::k_ptr<KEEP> kin, const double *y_n, double *y_run, double *out,
     const double *rfm0, const double *rfm1, const bhah_kparams &p, const int2 *map, const int2 *pairs) {
   const int np = (!(p.Ntot & 1) && !((reinterpret_cast<uintptr_t>(kin) | reinterpret_cast<uintptr_t>(y_n) |
                                       reinterpret_cast<uintptr_t>(y_run) | reinterpret_cast<uintptr_t>(out)) & 15))
@@ -885,14 +916,16 @@ static hipError_t rk_det_launch_SinhSpherical_symnone_KO1_fd4(hipStream_t s, con
   const bool nt_all = p.Ntot * (5 * 24 * 8L) > 1800000000L;
 #define RK_LAUNCH(NP_, IN_, NT_)                                                                                     \
   if (np == NP_ && (map != nullptr) == IN_ && nt_all == NT_)                                                         \
-    hipLaunchKernelGGL((bssn_rk_det_SinhSpherical_symnone_KO1_fd4<NP_, IN_, NT_>), g, dim3(nt), 0, s, kin, y_n, y_run, out, rfm0, rfm1, p,   \
+    hipLaunchKernelGGL((bssn_rk_det_SinhSpherical_symnone_KO1_fd4<NP_, IN_, NT_, KEEP>), g, dim3(nt), 0, s, kin, y_n, y_run, out, rfm0, rfm1, p,   \
                        map, pairs)
-  RK_LAUNCH(1, false, false);
-  RK_LAUNCH(1, false, true);
+  if constexpr (!KEEP) {
+    RK_LAUNCH(1, false, false);
+    RK_LAUNCH(1, false, true);
+    RK_LAUNCH(2, false, false);
+    RK_LAUNCH(2, false, true);
+  }
   RK_LAUNCH(1, true, false);
   RK_LAUNCH(1, true, true);
-  RK_LAUNCH(2, false, false);
-  RK_LAUNCH(2, false, true);
   RK_LAUNCH(2, true, false);
   RK_LAUNCH(2, true, true);
 #undef RK_LAUNCH
@@ -900,14 +933,14 @@ static hipError_t rk_det_launch_SinhSpherical_symnone_KO1_fd4(hipStream_t s, con
 }
 extern "C" hipError_t launch_bssn_rk_det_SinhSpherical_symnone_KO1_fd4(hipStream_t s, const double *kin, const double *y_n, double *y_run,
     double *out, const double *rfm0, const double *rfm1, bhah_kparams p) {
-  return rk_det_launch_SinhSpherical_symnone_KO1_fd4(s, kin, y_n, y_run, out, rfm0, rfm1, p, nullptr, nullptr);
+  return rk_det_launch_SinhSpherical_symnone_KO1_fd4<false>(s, kin, y_n, y_run, out, rfm0, rfm1, p, nullptr, nullptr);
 }
 // The RK pass with the inner boundary condition folded in.
 extern "C" hipError_t launch_bssn_rk_det_inner_SinhSpherical_symnone_KO1_fd4(hipStream_t s, const double *kin, const double *y_n,
     double *y_run, double *out, const double *rfm0, const double *rfm1, bhah_kparams p, const int *map,
     const int *pairs) {
-  return rk_det_launch_SinhSpherical_symnone_KO1_fd4(s, kin, y_n, y_run, out, rfm0, rfm1, p, reinterpret_cast<const int2 *>(map),
-                             reinterpret_cast<const int2 *>(pairs));
+  return rk_det_launch_SinhSpherical_symnone_KO1_fd4<false>(s, kin, y_n, y_run, out, rfm0, rfm1, p, reinterpret_cast<const int2 *>(map),
+                                    reinterpret_cast<const int2 *>(pairs));
 }
 
 // Host-side launchers (one translation unit per variant; no relocatable device code needed).

@@ -80,6 +80,27 @@ def test_folded_pass_equals_the_separate_copy(hip, name):
     assert torch.equal(SF.y_n, SS.y_n)
 
 
+@pytest.mark.parametrize("Nxx", [(24, 6, 2), (17, 7, 2), (18, 5, 4)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_taped_step_keeps_inner_ghosts_of_k(hip, Nxx, off):
+    """The tape of a step whose RK pass takes the inner-parity condition with it equals, bit for
+    bit and inner ghost points of every k included, that of the separate copy."""
+    import torch
+
+    c = dict(coord=1, Nxx=Nxx, fd_order=4, sym=4, KO=False)
+    PF, PS = _patch(c, False), _patch(c, True)
+    y0 = _initial(PF)
+    tapes, ends = [], []
+    for P in (PF, PS):
+        flat = torch.zeros(P.tape_doubles + off, dtype=torch.float64, device="cuda")
+        y = y0.clone()
+        P.MoL_step_forward_taped(y, PF.dt, flat[off:])
+        torch.cuda.synchronize()
+        tapes.append(flat)
+        ends.append(y)
+    assert torch.isfinite(tapes[0]).all() and torch.equal(*tapes) and torch.equal(*ends)
+
+
 @pytest.mark.parametrize("name", ["fd6_odd", "fd4_odd_unaligned"])
 @pytest.mark.parametrize("order", [2, 4, 6])
 def test_radiation_lines_match_oracle(hip, oracle_lib, name, order):
