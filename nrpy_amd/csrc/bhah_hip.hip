@@ -2709,7 +2709,6 @@ struct bhah_ensemble {
   std::vector<bhah_patch *> P;
   const BssnKernels *k = nullptr;
   int NG = 0;
-  std::vector<bhah_member> hmem;
   bhah_member *d_mem = nullptr;
   bhah_item *d_int = nullptr, *d_all = nullptr;
   int n_int = 0, n_all = 0;
@@ -2717,6 +2716,7 @@ struct bhah_ensemble {
   bhah_item *d_lds[2] = {};
   int n_lds[2] = {};
   bool aligned16 = true;  // every bound stage array 16-byte aligned (schedules with pair loads need it)
+  int np = 2;             // points per thread of the RK pass that d_all is made for
   ens_rad_line *d_lines = nullptr;  // radial lines of the outer boundary points, all members
   int n_lines = 0;
   double *d_wavespeed = nullptr, *d_finf = nullptr;
@@ -2735,10 +2735,10 @@ struct bhah_ensemble {
     }
   }
   // points per thread of the RK pass: 2 where every member's arrays allow 16-byte accesses
-  int np() const {
+  int np_for(bool aligned) const {
     for (const bhah_patch *q : P)
       if (q->Ntot & 1) return 1;
-    return aligned16 ? 2 : 1;
+    return aligned ? 2 : 1;
   }
   dim3 grid_for(int nitems) const {
     const int g = (max_wg > 0 && max_wg < nitems) ? max_wg : nitems;
@@ -2748,40 +2748,47 @@ struct bhah_ensemble {
 
 namespace {
 
-// Tile lists: interior tiles (tile_x x tile_y threads over (i0, i1), one xx2 plane each)
-// and, for the RK pass, chunks of 256 consecutive points (pairs of points where the pass takes
-// pairs) of each member's arrays, all members concatenated.
-int ensemble_build_items(bhah_ensemble *E) {
-  std::vector<bhah_item> in, all;
+// Put a new work list in the place of *d (of *n records); on failure the old one stays.
+int replace_items(const std::vector<bhah_item> &v, bhah_item **d, int *n) {
+  bhah_item *fresh = nullptr;
+  const int rc = upload(v, &fresh);
+  if (rc) return rc;
+  hipFree(*d);
+  *d = fresh;
+  *n = (int)v.size();
+  return BHAH_OK;
+}
+
+// Interior tiles of all members: tile_x x tile_y threads over (i0, i1), one xx2 plane each.
+int ensemble_build_tiles(bhah_ensemble *E, int tile_x, int tile_y) {
+  std::vector<bhah_item> in;
   for (int m = 0; m < (int)E->P.size(); m++) {
     const bhah_patch *P = E->P[m];
     const int n0 = P->d.Nxx[0], n1 = P->d.Nxx[1], n2 = P->d.Nxx[2];
     for (int bz = 0; bz < n2; bz++)
-      for (int by = 0; by < (n1 + E->tile_y - 1) / E->tile_y; by++)
-        for (int bx = 0; bx < (n0 + E->tile_x - 1) / E->tile_x; bx++) in.push_back({m, bx, by, bz});
-    const long units = P->Ntot / E->np();
-    for (long c = 0; c < (units + 255) / 256; c++) all.push_back({m, (int)c, 0, 0});
+      for (int by = 0; by < (n1 + tile_y - 1) / tile_y; by++)
+        for (int bx = 0; bx < (n0 + tile_x - 1) / tile_x; bx++) in.push_back({m, bx, by, bz});
   }
-  hipFree(E->d_int);
-  hipFree(E->d_all);
-  E->d_int = E->d_all = nullptr;
-  int rc;
-  if ((rc = upload(in, &E->d_int)) || (rc = upload(all, &E->d_all))) return rc;
-  E->n_int = (int)in.size();
-  E->n_all = (int)all.size();
-  return BHAH_OK;
+  return replace_items(in, &E->d_int, &E->n_int);
+}
+
+// The RK pass's list: chunks of 256 units of np consecutive points of each member's arrays, all
+// members concatenated.
+int ensemble_build_units(bhah_ensemble *E, int np) {
+  std::vector<bhah_item> all;
+  for (int m = 0; m < (int)E->P.size(); m++)
+    for (long c = 0; c < (E->P[m]->Ntot / np + 255) / 256; c++) all.push_back({m, (int)c, 0, 0});
+  const int rc = replace_items(all, &E->d_all, &E->n_all);
+  if (!rc) E->np = np;
+  return rc;
 }
 
 // Tile list of a selected LDS-tiled schedule (kind 0: rhs, 1: Ricci): every member's interior
 // in the schedule's own TX x TY x TZ tiles.  Workgroups go round-robin over the 8 XCDs, so the
 // list is dealt out such that XCD k walks its k-th contiguous eighth: neighbouring tiles, whose
 // halos overlap, then share an L2.
-int ensemble_build_lds_items(bhah_ensemble *E, int kind) {
-  const BssnCandidate &c = kind == 0 ? E->k->rhs[E->rhs_choice] : E->k->ricci[E->ricci_choice];
-  hipFree(E->d_lds[kind]);
-  E->d_lds[kind] = nullptr;
-  E->n_lds[kind] = 0;
-  if (!c.lds[0]) return BHAH_OK;
+int ensemble_build_lds_items(bhah_ensemble *E, int kind, const BssnCandidate &c) {
+  if (!c.lds[0]) return BHAH_OK;  // walks the interior tiles
   std::vector<bhah_item> v;
   for (int m = 0; m < (int)E->P.size(); m++) {
     const bhah_patch *P = E->P[m];
@@ -2794,10 +2801,7 @@ int ensemble_build_lds_items(bhah_ensemble *E, int kind) {
   const size_t n = v.size();
   std::vector<bhah_item> order(n);
   for (size_t h = 0; h < n; h++) order[h] = v[(h & 7) * (n >> 3) + std::min(h & 7, n & 7) + (h >> 3)];
-  int rc;
-  if ((rc = upload(order, &E->d_lds[kind]))) return rc;
-  E->n_lds[kind] = (int)n;
-  return BHAH_OK;
+  return replace_items(order, &E->d_lds[kind], &E->n_lds[kind]);
 }
 
 int ensemble_enqueue_step(bhah_ensemble *E) {
@@ -2829,7 +2833,7 @@ int ensemble_enqueue_step(bhah_ensemble *E) {
     HIP_TRY(hipGetLastError());
     // the RK pass takes the inner-parity condition of k with it, as the single-patch step does
     HIP_TRY(E->k->ens_rk_det(E->grid_for(4 * E->n_all), E->stream, E->d_mem, E->d_all, E->n_all, k, out, s,
-                               E->np()));
+                             E->np));
   }
   return BHAH_OK;
 }
@@ -2905,7 +2909,7 @@ int bhah_hip_ensemble_create(const bhah_patch_desc *descs, int n, bhah_ensemble 
     return rc;
   }
   E->n_lines = (int)lines.size();
-  if ((rc = ensemble_build_items(E))) {
+  if ((rc = ensemble_build_tiles(E, E->tile_x, E->tile_y)) || (rc = ensemble_build_units(E, E->np_for(true)))) {
     bhah_hip_ensemble_destroy(E);
     return rc;
   }
@@ -2913,7 +2917,6 @@ int bhah_hip_ensemble_create(const bhah_patch_desc *descs, int n, bhah_ensemble 
     bhah_hip_ensemble_destroy(E);
     return fail(BHAH_ERR_HIP, "hipMalloc failed");
   }
-  E->hmem.resize(n);
   *out = E;
   return BHAH_OK;
 }
@@ -2947,13 +2950,16 @@ int bhah_hip_ensemble_member(bhah_ensemble *E, int m, bhah_patch **patch) {
 
 int bhah_hip_ensemble_bind(bhah_ensemble *E, const bhah_MoL_gridfunctions *gfs, const double *dt) {
   if (!E || !gfs) return fail(BHAH_ERR_ARG, "NULL argument");
-  E->aligned16 = true;
+  // Refused arguments leave the ensemble on the arrays it has: nothing of it changes before every
+  // member's are looked at.
+  std::vector<bhah_member> mem(E->P.size());
+  bool aligned = true;
   for (size_t m = 0; m < E->P.size(); m++) {
     const bhah_patch *P = E->P[m];
     const bhah_MoL_gridfunctions &g = gfs[m];
     if (!g.y_n_gfs || !g.y_nplus1_running_total_gfs || !g.k_odd_gfs || !g.k_even_gfs || !g.auxevol_gfs)
       return fail(BHAH_ERR_ARG, "member %d: MoL gridfunctions not allocated", (int)m);
-    bhah_member &M = E->hmem[m];
+    bhah_member &M = mem[m];
     M.kp = P->kp(dt ? dt[m] : P->dt, 0);
     M.rfm0 = P->d_rfm0;
     M.rfm1 = P->d_rfm1;
@@ -2967,15 +2973,20 @@ int bhah_hip_ensemble_bind(bhah_ensemble *E, const bhah_MoL_gridfunctions *gfs, 
     M.arr[3] = g.k_even_gfs;
     M.arr[4] = g.auxevol_gfs;
     for (int a = 0; a < 4; a++)
-      if ((uintptr_t)M.arr[a] & 15) E->aligned16 = false;
+      if ((uintptr_t)M.arr[a] & 15) aligned = false;
     M.coord = P->d.coord;
     M.AMPL = P->d.grid_physical_size;
     M.SINHW = P->d.SINHW;
   }
-  HIP_TRY(hipMemcpy(E->d_mem, E->hmem.data(), sizeof(bhah_member) * E->hmem.size(), hipMemcpyHostToDevice));
-  E->bound = true;
+  E->bound = false;  // until the device has the new arrays and the list that fits them
   E->invalidate_graph();
-  return ensemble_build_items(E);  // the RK pass's units depend on the arrays' alignment
+  const int np = E->np_for(aligned);
+  int rc;
+  if (np != E->np && (rc = ensemble_build_units(E, np))) return rc;
+  HIP_TRY(hipMemcpy(E->d_mem, mem.data(), sizeof(bhah_member) * mem.size(), hipMemcpyHostToDevice));
+  E->aligned16 = aligned;
+  E->bound = true;
+  return BHAH_OK;
 }
 
 int bhah_hip_ensemble_set_stream(bhah_ensemble *E, void *s) {
@@ -2996,21 +3007,25 @@ int bhah_hip_ensemble_select_schedule(bhah_ensemble *E, int kind, int index) {
     const int rc = schedule_fits(P, c.name);
     if (rc) return rc;
   }
+  const int rc = ensemble_build_lds_items(E, kind == BHAH_KERNEL_RHS ? 0 : 1, c);
+  if (rc) return rc;
   if (kind == BHAH_KERNEL_RHS) E->rhs_choice = index;
   else E->ricci_choice = index;
   E->invalidate_graph();
-  return ensemble_build_lds_items(E, kind == BHAH_KERNEL_RHS ? 0 : 1);
+  return BHAH_OK;
 }
 
 int bhah_hip_ensemble_set_launch(bhah_ensemble *E, int tile_x, int tile_y, int max_workgroups) {
   if (!E) return fail(BHAH_ERR_ARG, "NULL ensemble");
   if (tile_x * tile_y != 256 || tile_x < 16 || tile_x % 16) return fail(BHAH_ERR_ARG, "tile must be 256 threads, tile_x a multiple of 16");
   if (max_workgroups < 0) return fail(BHAH_ERR_ARG, "max_workgroups must be >= 0 (0: one per tile)");
+  const int rc = ensemble_build_tiles(E, tile_x, tile_y);
+  if (rc) return rc;
   E->tile_x = tile_x;
   E->tile_y = tile_y;
   E->max_wg = max_workgroups;
   E->invalidate_graph();
-  return ensemble_build_items(E);
+  return BHAH_OK;
 }
 
 int bhah_hip_ensemble_step_n(bhah_ensemble *E, int nsteps, int use_graph) {

@@ -93,3 +93,70 @@ def test_every_ensemble_schedule_and_launch_shape(hip):
                 for k in range(len(got)):
                     er = rel_err(got[k], ref[k])
                     assert er.max() < 1e-12, (ric, rhs, launch, k, er)
+
+
+def _moved(st, off):
+    """The member's arrays (aux apart) moved to start ``off`` doubles past a 16-byte boundary."""
+    import torch
+    from nrpy_amd.runtime import MoLGridfunctions
+
+    def moved(t):
+        flat = torch.zeros(t.numel() + 2, dtype=t.dtype, device=t.device)
+        new = flat[off:off + t.numel()].view(t.shape)
+        new.copy_(t)
+        return new
+
+    st.y_n, st.y_run, st.k_odd, st.k_even = (moved(t) for t in (st.y_n, st.y_run, st.k_odd, st.k_even))
+    assert st.y_n.data_ptr() % 16 == 8 * off
+    st.c = MoLGridfunctions(*(t.data_ptr() for t in (st.y_n, st.y_run, st.k_odd, st.k_even, st.aux)))
+
+
+def _started():
+    import torch
+    from nrpy_amd.runtime import Ensemble
+
+    E = Ensemble(_cfgs())
+    for k, (P, st) in enumerate(zip(E.members, E.states)):
+        st.y_n.copy_(torch.from_numpy(_initial(P, k)))
+        P.apply_bcs_outerextrap_and_inner(st.y_n)
+    return E
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_rebinding_arrays_of_another_alignment(hip, use_graph):
+    """The RK pass takes pairs of points, or single ones where a member's arrays are not 16-byte
+    aligned; binding other arrays changes the form both ways.  Same operations: the same bits."""
+    import torch
+
+    A, B = _started(), _started()
+    for off in (1, 0):
+        for st in B.states:
+            _moved(st, off)
+        B.bind()
+        A.steps(2, use_graph=use_graph)
+        B.steps(2, use_graph=use_graph)
+        torch.cuda.synchronize()
+        assert [bool(torch.isfinite(a.y_n).all()) and torch.equal(a.y_n, b.y_n)
+                for a, b in zip(A.states, B.states)] == [True] * len(GRIDS), off
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_refused_bind_keeps_the_bound_arrays(hip, use_graph):
+    """A bind that is refused (a later member has no arrays) leaves the ensemble on the arrays it
+    has, whatever the alignment of the ones offered."""
+    import torch
+    from nrpy_amd.runtime import BHaHError, MoLGridfunctions
+
+    A, B = _started(), _started()
+    A.steps(1, use_graph=use_graph)
+    B.steps(1, use_graph=use_graph)
+    kept = [st.c for st in B.states]
+    B.states[0].c = MoLGridfunctions(*(p + 8 for p in (kept[0].y_n_gfs, kept[0].y_nplus1_running_total_gfs,
+                                                       kept[0].k_odd_gfs, kept[0].k_even_gfs, kept[0].auxevol_gfs)))
+    B.states[-1].c = MoLGridfunctions()
+    with pytest.raises(BHaHError, match="not allocated"):
+        B.bind()
+    A.steps(2, use_graph=use_graph)
+    B.steps(2, use_graph=use_graph)
+    torch.cuda.synchronize()
+    assert [torch.equal(a.y_n, b.y_n) for a, b in zip(A.states, B.states)] == [True] * len(GRIDS)
