@@ -2886,14 +2886,19 @@ int bhah_hip_ensemble_create(const bhah_patch_desc *descs, int n, bhah_ensemble 
   std::vector<ens_rad_line> lines;  // of all members
   for (int m = 0; m < n; m++) {
     const bhah_patch *P = E->P[m];
-    if (!P->n_rad_lines || !rad_lines_fit(P->Nx[0], P->NG, E->R)) {
-      bhah_hip_ensemble_destroy(E);
-      return fail(BHAH_ERR_UNSUPPORTED, "member %d: its outer points are not radial lines of %d points", m,
-                  P->NG + E->R + 2);
-    }
+    // A line of one interior point holds NG + R + 1 values at R = NG.  The walk's first value is then
+    // the one before the line in memory, as it is for rad_point (no line starts the array: i1, i2
+    // are interior).  Only the reverse kernel, which updates what it reads, needs whole lines.
+    bool walk = P->n_rad_lines > 0 && (P->NG == 3 || P->NG == 4) && P->Nx[0] >= P->NG + E->R + 1;
     for (size_t q = 0; q < P->outer[0][0].size(); q += 6) {
       const int16_t *o = &P->outer[0][0][q];
       lines.push_back({m, P->Nx[0] * (o[1] + P->Nx[1] * o[2])});
+      walk = walk && lines.back().base > 0;
+    }
+    if (!walk) {
+      bhah_hip_ensemble_destroy(E);
+      return fail(BHAH_ERR_UNSUPPORTED, "member %d: its outer points are not radial lines of %d points", m,
+                  P->NG + E->R + 1);
     }
   }
   std::vector<double> ws(24, 1.0), fi(24, 0.0);

@@ -160,3 +160,33 @@ def test_refused_bind_keeps_the_bound_arrays(hip, use_graph):
     B.steps(2, use_graph=use_graph)
     torch.cuda.synchronize()
     assert [torch.equal(a.y_n, b.y_n) for a, b in zip(A.states, B.states)] == [True] * len(GRIDS)
+
+
+@pytest.mark.parametrize("order", [2, 4, 6])
+def test_members_of_one_radial_point(hip, order):
+    """The smallest grids the single patch takes, at every stencil of the radiation condition (one of
+    radius three reaches past a line of one interior point).  A step of the per-call functions, whose
+    radiation condition goes point by point there, against the batched step: same operations, within
+    the 1e-13 of the test above."""
+    import torch
+    from nrpy_amd.runtime import Ensemble, MoLState, Patch, PatchConfig
+
+    cfgs = [PatchConfig(Nxx=N, grid_physical_size=10.0, eta=2.0, radiation_bc_fd_order=order)
+            for N in [(1, 6, 2), (2, 4, 4), (1, 3, 2)]]
+    E = Ensemble(cfgs)
+    singles = []
+    for k, (cfg, P, st) in enumerate(zip(cfgs, E.members, E.states)):
+        y = torch.from_numpy(_initial(P, k)).cuda()
+        P.apply_bcs_outerextrap_and_inner(y)
+        st.y_n.copy_(y)
+        Q = Patch(cfg, tuned=False)
+        Q.select_schedule(0, 0)
+        Q.select_schedule(1, 0)
+        singles.append(MoLState(Q, y))
+    E.steps(1)
+    for S, dt in zip(singles, E.dts):
+        S.steps(1, dt)
+    torch.cuda.synchronize()
+    for S, st in zip(singles, E.states):
+        assert torch.isfinite(S.y_n).all()
+        assert rel_err(st.y_n.cpu().numpy(), S.y_n.cpu().numpy()).max() < 1e-13
