@@ -202,6 +202,9 @@ int bhah_hip_MoL_step_n(bhah_patch *patch, bhah_MoL_gridfunctions *gf, bhah_cloc
  * (nrpy/helpers/parallelization/utilities.py:108-196). */
 int bhah_hip_patch_num_schedules(const bhah_patch *patch, int kind);
 const char *bhah_hip_patch_schedule_name(const bhah_patch *patch, int kind, int index);
+/* Index of the schedule `name`, or a negative error where the build has none of that name.  A
+ * schedule of an earlier build that is no longer made gives the one that took its place. */
+int bhah_hip_patch_find_schedule(const bhah_patch *patch, int kind, const char *name);
 int bhah_hip_patch_select_schedule(bhah_patch *patch, int kind, int index);
 int bhah_hip_patch_get_schedule(const bhah_patch *patch, int kind);
 /* Interior thread-block shape (tile_x * tile_y = 256, tile_x along xx0); replaces the
@@ -326,6 +329,8 @@ int bhah_hip_ensemble_member(bhah_ensemble *ens, int m, bhah_patch **patch);
  * timestep (dt == NULL: each member's CFL timestep). */
 int bhah_hip_ensemble_bind(bhah_ensemble *ens, const bhah_MoL_gridfunctions *gfs, const double *dt);
 int bhah_hip_ensemble_set_stream(bhah_ensemble *ens, void *hip_stream);
+/* As bhah_hip_patch_find_schedule, for all members. */
+int bhah_hip_ensemble_find_schedule(const bhah_ensemble *ens, int kind, const char *name);
 int bhah_hip_ensemble_select_schedule(bhah_ensemble *ens, int kind, int index);
 /* Interior tile (tile_x * tile_y = 256) and the persistent grid size
  * (max_workgroups; 0 = one workgroup per tile). */

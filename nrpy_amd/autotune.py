@@ -16,6 +16,7 @@ from __future__ import annotations
 import argparse
 import json
 import os
+import warnings
 from typing import Dict, Optional
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -69,11 +70,12 @@ def apply_tuned(patch) -> Optional[Dict]:
     from .runtime import BHaHError
 
     for kind, key in ((KERNEL_RHS, "rhs"), (KERNEL_RICCI, "ricci")):
-        if d[key] in patch.schedules(kind):
-            try:
-                patch.select_schedule(kind, d[key])
-            except BHaHError:
-                pass  # schedule not usable at this grid size: keep the default
+        try:
+            patch.select_schedule(kind, d[key])
+        except BHaHError:
+            pass  # schedule not usable at this grid size: keep the default
+        except ValueError as e:
+            warnings.warn(f"stored table: {e}; the default stays")
     patch.set_tile(*d["tile"])
     return d
 
@@ -175,10 +177,11 @@ def apply_tuned_ensemble(E) -> Optional[Dict]:
                 d = json.load(f)
     if not d:
         return None
-    if d["rhs"] in E.schedules(KERNEL_RHS):
-        E.select_schedule(KERNEL_RHS, d["rhs"])
-    if d["ricci"] in E.schedules(KERNEL_RICCI):
-        E.select_schedule(KERNEL_RICCI, d["ricci"])
+    for kind, key in ((KERNEL_RHS, "rhs"), (KERNEL_RICCI, "ricci")):
+        try:
+            E.select_schedule(kind, d[key])
+        except ValueError as e:
+            warnings.warn(f"stored table: {e}; the schedule in use stays")
     E.set_launch(*d["launch"])
     return d
 

@@ -1353,6 +1353,51 @@ int default_schedule(const bhah_patch *P, const BssnCandidate *c, int n) {
   return i;
 }
 
+// Schedules of earlier builds, whose names programs and tuned tables may still hold.  Asking for one
+// gets the schedule that took its place, the preferred one of the build, wherever the retired one
+// could run.
+const struct {
+  const char *tag;
+  int kind;
+  const char *name;
+} kRetired[] = {
+    {"Spherical_sym2_KO0_fd4", BHAH_KERNEL_RHS, "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8_ub_mi"},
+    {"Spherical_sym2_KO0_fd4", BHAH_KERNEL_RICCI, "r1_lb1_sj_L16x4x4x1_d2_dma_xcd"},
+    {"Spherical_sym2_KO0_fd4", BHAH_KERNEL_RICCI, "r1_lb1_sj_L16x8x2x1_d3_dma_rb1_mi"},
+    {"SinhSpherical_symnone_KO1_fd6", BHAH_KERNEL_RHS, "p1_lb1_sj_L16x4x4x1_d4_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk"},
+    {"SinhSpherical_symnone_KO1_fd6", BHAH_KERNEL_RICCI, "r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg2_mi_xcd"},
+    {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RHS, "p1_lb1_sl_lf_pf16_u32_w2"},
+    {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RHS, "p1_lb1_sj_L16x8x2x1_d3_dma_rb1"},
+    {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RHS, "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8"},
+    {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RHS, "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8_ub"},
+    {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RHS, "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8_ub_mi"},
+    {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RICCI, "r1_lb1_pf16_u32"},
+    {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RICCI, "r1_lb1_sj_L16x4x4x1_d2_dma_xcd"},
+    {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RICCI, "r1_lb1_sj_L16x8x2x1_d3_dma_rb1"},
+    {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RICCI, "r1_lb1_sj_L16x8x2x1_d3_dma_rb1_mi"},
+};
+
+// Index of the schedule that `name` asks for on all n patches (of one build), or a negative error.
+int find_schedule(const bhah_patch *const *P, int n, int kind, const char *name) {
+  const BssnKernels *k = P[0]->k;
+  const BssnCandidate *c = kind == BHAH_KERNEL_RHS ? k->rhs : k->ricci;
+  const int nc = kind == BHAH_KERNEL_RHS ? k->n_rhs : kind == BHAH_KERNEL_RICCI ? k->n_ricci : -1;
+  if (nc < 0) return fail(BHAH_ERR_ARG, "unknown kernel kind %d", kind);
+  for (int i = 0; i < nc; i++)
+    if (!strcmp(c[i].name, name)) return i;
+  for (const auto &r : kRetired) {
+    if (r.kind != kind || strcmp(r.name, name) || strcmp(r.tag, k->tag)) continue;
+    int best = nc - 1;
+    for (int m = 0; m < n; m++) {
+      const int rc = schedule_fits(P[m], name);
+      if (rc) return rc;
+      best = std::min(best, default_schedule(P[m], c, nc));
+    }
+    return best;
+  }
+  return fail(BHAH_ERR_ARG, "build %s has no schedule %s", k->tag, name);
+}
+
 // Whether schedule `nm` fills its boxes with 16-byte loads (its input must be 16-byte aligned).
 bool pair_loads(const char *nm) { return strstr(nm, "_dma") || strstr(nm, "_dmo"); }
 
@@ -2227,6 +2272,12 @@ const char *bhah_hip_patch_schedule_name(const bhah_patch *P, int kind, int inde
   return nullptr;
 }
 
+int bhah_hip_patch_find_schedule(const bhah_patch *P, int kind, const char *name) {
+  if (!P || !P->k) return fail(BHAH_ERR_ARG, "patch is not a BSSN patch");
+  if (!name) return fail(BHAH_ERR_ARG, "NULL argument");
+  return find_schedule(&P, 1, kind, name);
+}
+
 int bhah_hip_patch_select_schedule(bhah_patch *P, int kind, int index) {
   const int n = bhah_hip_patch_num_schedules(P, kind);
   if (n < 0) return n;
@@ -2999,6 +3050,11 @@ int bhah_hip_ensemble_set_stream(bhah_ensemble *E, void *s) {
   E->stream = (hipStream_t)s;
   E->invalidate_graph();
   return BHAH_OK;
+}
+
+int bhah_hip_ensemble_find_schedule(const bhah_ensemble *E, int kind, const char *name) {
+  if (!E || !name) return fail(BHAH_ERR_ARG, "NULL argument");
+  return find_schedule(E->P.data(), (int)E->P.size(), kind, name);
 }
 
 int bhah_hip_ensemble_select_schedule(bhah_ensemble *E, int kind, int index) {

@@ -148,6 +148,7 @@ SIGNATURES: Dict[str, tuple] = {
     "bhah_hip_MoL_step_n": (_I, [_P, ctypes.POINTER(MoLGridfunctions), ctypes.POINTER(Clock), _I, _I]),
     "bhah_hip_patch_num_schedules": (_I, [_P, _I]),
     "bhah_hip_patch_schedule_name": (ctypes.c_char_p, [_P, _I, _I]),
+    "bhah_hip_patch_find_schedule": (_I, [_P, _I, ctypes.c_char_p]),
     "bhah_hip_patch_select_schedule": (_I, [_P, _I, _I]),
     "bhah_hip_patch_get_schedule": (_I, [_P, _I]),
     "bhah_hip_patch_set_tile": (_I, [_P, _I, _I]),
@@ -174,6 +175,7 @@ SIGNATURES: Dict[str, tuple] = {
     "bhah_hip_ensemble_member": (_I, [_P, _I, ctypes.POINTER(_P)]),
     "bhah_hip_ensemble_bind": (_I, [_P, ctypes.POINTER(MoLGridfunctions), ctypes.POINTER(_D)]),
     "bhah_hip_ensemble_set_stream": (_I, [_P, _P]),
+    "bhah_hip_ensemble_find_schedule": (_I, [_P, _I, ctypes.c_char_p]),
     "bhah_hip_ensemble_select_schedule": (_I, [_P, _I, _I]),
     "bhah_hip_ensemble_set_launch": (_I, [_P, _I, _I, _I]),
     "bhah_hip_ensemble_step_n": (_I, [_P, _I, _I]),
@@ -203,10 +205,26 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     return lib
 
 
+BHAH_ERR_ARG = -1
+
+
 def _check(rc: int) -> None:
     if rc != 0:
         msg = load_library().bhah_hip_last_error().decode()
         raise BHaHError(f"bhah_hip error {rc}: {msg}")
+
+
+def _schedule_index(find, handle, kind: int, name_or_index) -> int:
+    """Index of a schedule given by index or name (names of schedules that earlier builds had and
+    this one replaces included); ValueError for a name the build never had."""
+    if not isinstance(name_or_index, str):
+        return int(name_or_index)
+    idx = find(handle, kind, name_or_index.encode())
+    if idx == BHAH_ERR_ARG:
+        raise ValueError(load_library().bhah_hip_last_error().decode())
+    if idx < 0:
+        _check(idx)
+    return idx
 
 
 @dataclass
@@ -350,8 +368,7 @@ class Patch:
         return [self.lib.bhah_hip_patch_schedule_name(self.handle, kind, i).decode() for i in range(n)]
 
     def select_schedule(self, kind: int, name_or_index):
-        names = self.schedules(kind)
-        idx = names.index(name_or_index) if isinstance(name_or_index, str) else int(name_or_index)
+        idx = _schedule_index(self.lib.bhah_hip_patch_find_schedule, self.handle, kind, name_or_index)
         _check(self.lib.bhah_hip_patch_select_schedule(self.handle, kind, idx))
 
     def schedule(self, kind: int) -> str:
@@ -562,8 +579,7 @@ class Ensemble:
         return self.members[0].schedules(kind)
 
     def select_schedule(self, kind: int, name_or_index):
-        names = self.schedules(kind)
-        idx = names.index(name_or_index) if isinstance(name_or_index, str) else int(name_or_index)
+        idx = _schedule_index(self.lib.bhah_hip_ensemble_find_schedule, self.handle, kind, name_or_index)
         _check(self.lib.bhah_hip_ensemble_select_schedule(self.handle, kind, idx))
         self.choice[kind] = idx
 
