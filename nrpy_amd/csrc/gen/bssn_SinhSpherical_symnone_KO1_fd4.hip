@@ -105,17 +105,23 @@ __device__ __forceinline__ void at_source(Vec<NP> (&r)[6], const double *f, cons
     }
   }
 }
-// KEEP: the pass also writes k at inner ghost points, which a taped step keeps.
-template <bool KEEP>
+// KEEP: the pass also writes k at inner ghost points, which a taped step keeps.  Only the pass that
+// folds the inner condition and leaves k alone has k in an array of its own: without the fold the
+// stage is written over k.
+template <bool INNER, bool KEEP>
 struct KPtr {
+  typedef const double *type;
+};
+template <>
+struct KPtr<true, false> {
   typedef const double *__restrict__ type;
 };
 template <>
-struct KPtr<true> {
+struct KPtr<true, true> {
   typedef double *type;
 };
-template <bool KEEP>
-using k_ptr = typename KPtr<KEEP>::type;
+template <bool INNER, bool KEEP>
+using k_ptr = typename KPtr<INNER, KEEP>::type;
 // Write the inner ghost points' k among this thread's points: each point's own thread writes it, and
 // no thread takes a value from it (sources are never inner ghost points).
 template <int G, int NP>
@@ -135,7 +141,7 @@ __device__ __forceinline__ void keep_ghosts(double *f, const Vec<NP> (&k)[6], co
   }
 }
 template <int G, int NP, bool INNER, bool NT, bool KEEP>
-__device__ __forceinline__ void group(k_ptr<KEEP> kin, const double *y_n, double *y_run, double *out,
+__device__ __forceinline__ void group(k_ptr<INNER, KEEP> kin, const double *y_n, double *y_run, double *out,
                                       const double *__restrict__ rfm0, const double *__restrict__ rfm1,
                                       const bhah_kparams &p, const int2 *__restrict__ map,
                                       const int2 *__restrict__ pairs, const long q) {
@@ -245,7 +251,7 @@ __device__ __forceinline__ void group(k_ptr<KEEP> kin, const double *y_n, double
   if constexpr (KEEP) keep_ghosts<G, NP>(kin, k, Ntot, S, idx);
 }
 template <int NP, bool INNER, bool NT, bool KEEP>
-__device__ __forceinline__ void any_group(int G, k_ptr<KEEP> kin, const double *y_n, double *y_run,
+__device__ __forceinline__ void any_group(int G, k_ptr<INNER, KEEP> kin, const double *y_n, double *y_run,
                                           double *out, const double *__restrict__ rfm0,
                                           const double *__restrict__ rfm1, const bhah_kparams &p,
                                           const int2 *__restrict__ map, const int2 *__restrict__ pairs,
@@ -259,7 +265,7 @@ __device__ __forceinline__ void any_group(int G, k_ptr<KEEP> kin, const double *
 }  // namespace rk_SinhSpherical_symnone_KO1_fd4
 template <int NP, bool INNER, bool NT, bool KEEP>
 __global__ void __launch_bounds__(256)
-bssn_rk_det_SinhSpherical_symnone_KO1_fd4(rk_SinhSpherical_symnone_KO1_fd4::k_ptr<KEEP> kin, const double *y_n, double *y_run, double *out,
+bssn_rk_det_SinhSpherical_symnone_KO1_fd4(rk_SinhSpherical_symnone_KO1_fd4::k_ptr<INNER, KEEP> kin, const double *y_n, double *y_run, double *out,
                   const double *__restrict__ rfm0, const double *__restrict__ rfm1, const bhah_kparams p,
                   const int2 *__restrict__ map, const int2 *__restrict__ pairs) {
   rk_SinhSpherical_symnone_KO1_fd4::any_group<NP, INNER, NT, KEEP>((int)(blockIdx.x & 3u), kin, y_n, y_run, out, rfm0, rfm1, p, map, pairs,
@@ -897,8 +903,8 @@ bssn_initial_lambda_SinhSpherical_symnone_KO1_fd4(double *gfs, const double *__r
 #undef Rational_1_2
 #undef Rational_2_3
 
-template <bool KEEP>
-static hipError_t rk_det_launch_SinhSpherical_symnone_KO1_fd4(hipStream_t s, rk_SinhSpherical_symnone_KO1_fd4::k_ptr<KEEP> kin, const double *y_n, double *y_run, double *out,
+template <bool KEEP, typename K>
+static hipError_t rk_det_launch_SinhSpherical_symnone_KO1_fd4(hipStream_t s, K *kin, const double *y_n, double *y_run, double *out,
     const double *rfm0, const double *rfm1, const bhah_kparams &p, const int2 *map, const int2 *pairs) {
   const int np = (!(p.Ntot & 1) && !((reinterpret_cast<uintptr_t>(kin) | reinterpret_cast<uintptr_t>(y_n) |
                                       reinterpret_cast<uintptr_t>(y_run) | reinterpret_cast<uintptr_t>(out)) & 15))

@@ -13,6 +13,8 @@
 
 import os
 import re
+import shutil
+import subprocess
 
 import numpy as np
 import pytest
@@ -119,3 +121,18 @@ def test_phaseprobe_instrument_and_analyse():
     assert abs(res["waits"] - 5 * nph / tile) < 1e-12 and abs(res["phases"] - 20 * nph / tile) < 1e-12
     assert abs(res["prologue"] - 10 / tile) < 1e-12 and abs(res["algebra"] - 50 / tile) < 1e-12
     assert res["phase_ticks"] == [20] * nph and res["barrier_arrival_spread_ticks"] == 0
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_only_the_folded_rk_pass_takes_k_in_an_array_of_its_own(tmp_path):
+    """Without the fold the RK pass writes the stage over k, so its k must not be restrict."""
+    text = H.RK_PASS
+    types = text[text.index("template <bool INNER, bool KEEP>\nstruct KPtr"):text.index("// Write the inner ghost points")]
+    assert "group(k_ptr<INNER, KEEP> kin" in text and "bssn_rk_det_@TAG@(rk_@TAG@::k_ptr<INNER, KEEP> kin" in text
+    (tmp_path / "t.cpp").write_text(f"""#include <type_traits>
+{types}
+static_assert(std::is_same<k_ptr<false, false>, const double *>::value, "stage written over k");
+static_assert(std::is_same<k_ptr<true, true>, double *>::value, "k written at inner ghosts");
+static_assert(std::is_same<k_ptr<true, false>, const double *__restrict__>::value, "k only read");
+""")
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", str(tmp_path / "t.cpp")], check=True)
