@@ -915,11 +915,17 @@ static hipError_t rk_det_launch_SinhSpherical_symnone_KO1_fd4(hipStream_t s, K *
   const unsigned nt = units >= (1L << 17) ? 256 : 64;
   const dim3 g(4u * (unsigned)((units + nt - 1) / nt));
   // The running sum is not read again before the next substep, so it always streams past the
-  // caches.  The other arrays (five stage arrays in all) are read by the next kernels: caching
-  // them gains where a good part of them stays in the 256 MB last-level cache (7229 -> 6947 us
-  // per four steps at 127x63x62 fd6, 0.64 GB; 2297 -> 2003 at 256x64x16, 0.39 GB; 6958 -> 6925
-  // for an ensemble of 1.5 GB) and loses where none does (23493 -> 23839 at 192x96x96, 2.1 GB).
-  const bool nt_all = p.Ntot * (5 * 24 * 8L) > 1800000000L;
+  // caches.  The other arrays are read by the next kernels: caching them gains while a good part
+  // of them stays in the 256 MB last-level cache.  What counts is the interior (an inner ghost
+  // point takes the k of an interior one): streaming against caching, per step, takes 1.12 / 1.09 /
+  // 1.04 / 0.99 / 0.96 at 256 x 64 x 16 / 20 / 24 and 256 x 96 x 20 / 24 points phi-symmetric (262,000 to
+  // 590,000 interior points), 1.04 / 0.95 at 800x96x4 / 1200x128x4, 1.04 / 0.98 at 1600x128x2 /
+  // 2400x192x2; 1.06 / 1.01 / 0.997 / 0.98 / 0.96 at 112, 120, 128, 136 x half x half and 160x80x80 fd4;
+  // 1.024 / 1.005 / 0.990 / 0.96 / 0.98 / 0.99 at 112x56x56, 120x60x60, 127x63x62, 160x80x80,
+  // 192x96x96, 224x112x112 fd6.  Above 2.6 million phi-symmetric or fd4 points it is within 1.2%
+  // either way.
+  const long interior = (long)(p.Nx0 - 2 * p.NG) * (p.Nx1 - 2 * p.NG) * (p.Nx2 - 2 * p.NG);
+  const bool nt_all = interior > 470000;
 #define RK_LAUNCH(NP_, IN_, NT_)                                                                                     \
   if (np == NP_ && (map != nullptr) == IN_ && nt_all == NT_)                                                         \
     hipLaunchKernelGGL((bssn_rk_det_SinhSpherical_symnone_KO1_fd4<NP_, IN_, NT_, KEEP>), g, dim3(nt), 0, s, kin, y_n, y_run, out, rfm0, rfm1, p,   \

@@ -118,3 +118,62 @@ def test_radiation_lines_match_oracle(hip, oracle_lib, name, order):
     P.apply_bcs_outerradiation_and_inner(y, k)
     d = np.abs(k.cpu().numpy() - ref).reshape(24, -1).max(1) / np.abs(ref).reshape(24, -1).max(1)
     assert d.max() < 1e-12
+
+
+# The forms that stream every array (more than 470,000 interior points): pairs whose sources lie apart
+# (odd rows, three ghost zones) and together, single points, and without the folded inner condition
+# (extrapolation boundary, separate copy).
+STREAMED = {
+    "fd6_odd": dict(coord=2, Nxx=(121, 65, 62), fd_order=6, sym=0, KO=True, off=0),
+    "fd6_odd_unaligned": dict(coord=2, Nxx=(121, 65, 62), fd_order=6, sym=0, KO=True, off=1),
+    "fd6_even": dict(coord=2, Nxx=(122, 64, 62), fd_order=6, sym=0, KO=True, off=0),
+    "sym2_separate": dict(coord=1, Nxx=(480, 124, 8), fd_order=4, sym=4, KO=False, off=0, separate=True),
+    "fd4_extrapolation": dict(coord=2, Nxx=(122, 64, 62), fd_order=4, sym=0, KO=True, off=0, outer_bc=1),
+    "fd4_odd_extrapolation_unaligned": dict(coord=2, Nxx=(123, 65, 60), fd_order=4, sym=0, KO=True, off=1, outer_bc=1),
+}
+
+
+@pytest.mark.parametrize("name", list(STREAMED))
+def test_streamed_pass_equals_the_single_calls(hip, name):
+    """A step at the sizes where the pass streams, against the per-call functions with the RK4
+    combinations in torch.  Each stage then differs by the rounding of a fused multiply-add (an
+    ulp or two of its largest value), which a stage's right-hand side amplifies no further than the
+    whole steps the parity tests compare to 1e-10; same bound."""
+    import torch
+    from nrpy_amd.runtime import OUTER_BC_EXTRAPOLATION
+
+    c = STREAMED[name]
+    kw = {"outer_bc": c["outer_bc"]} if "outer_bc" in c else {}
+    assert not kw or kw["outer_bc"] == OUTER_BC_EXTRAPOLATION
+    assert c["Nxx"][0] * c["Nxx"][1] * c["Nxx"][2] > 470000
+    P = _patch(c, c.get("separate", False), setup_on_device=True, **kw)
+    y = P.new_gfs()
+    P.initial_data_brill_lindquist(y, 0.5, (0.1, 0.2, 0.5), 0.4, (-0.1, 0.0, -0.6))
+    # terms of every kind alive: smooth waves over the grid, different in each gridfunction
+    x = [torch.linspace(0.0, 1.0, n, dtype=torch.float64, device="cuda") for n in P.Nx]
+    for g in range(24):
+        y[g] += 1e-2 * torch.sin((2 + g % 3) * x[0] + g) * torch.cos((1 + g % 4) * x[1] + g)[:, None] \
+            * torch.cos(2 * x[2] + g)[:, None, None]
+    P.apply_bcs_outerextrap_and_inner(y)
+    P.enforce_detgammabar_equals_detgammahat(y)
+    S = _state(P, y, c["off"])
+    S.steps(1, P.dt, use_graph=False)
+
+    aux, k, stage, total = P.new_gfs(6), P.new_gfs(), y, y
+    for w, a in ((1, 0.5), (2, 0.5), (2, 1.0), (1, None)):
+        P.Ricci_eval(stage, aux)
+        P.rhs_eval(aux, stage, k)
+        if not kw:
+            P.apply_bcs_outerradiation_and_inner(stage, k)
+        total = total + (w * P.dt / 6.0) * k
+        stage = total if a is None else y + (a * P.dt) * k
+        P.enforce_detgammabar_equals_detgammahat(stage)
+        if kw:
+            P.apply_bcs_outerextrap_and_inner(stage)
+            P.enforce_detgammabar_equals_detgammahat(stage)
+    torch.cuda.synchronize()
+    d = (S.y_n - stage).abs().reshape(24, -1).amax(1) / stage.abs().reshape(24, -1).amax(1)
+    moved = (stage - y).abs().reshape(24, -1).amax(1) / stage.abs().reshape(24, -1).amax(1)
+    print(name, "step against single calls", d.max().item(), "step against its start", moved.min().item())
+    assert torch.isfinite(S.y_n).all() and moved.min() > 1e-8
+    assert d.max() < 1e-10
