@@ -946,25 +946,32 @@ def _group_bounds(lb: str, k: int, ngroups: int) -> str:
 # Candidate schedules built per workload, from the general to the preferred one: a patch runs
 # the last of its list that takes its size (``default_schedule`` in bhah_hip.hip) until another
 # is selected.  The plain one-thread-per-point schedule comes first (any size and alignment).
-# What decides between the forms, measured per launch on MI355X:
+# What decides between the forms, measured per launch on MI355X (smooth data with noise):
 #   * _dmo takes rows of any length; _dma needs even ones and has a box two values narrower
-#     where the stencils reach NGHOSTS: rhs fd6 691 against 791 us at 192x96x96, 185 against 188
-#     at 128x64x64 and 127x63x62 (the plain schedule: 1027 us there).
-#   * _tp forms mixed derivatives in two passes within a wave (``lds_kernel``): rhs fd6 691
-#     against 749 us at 192x96x96, Ricci fd6 269 against 336, Ricci fd4 132 against 151 at
-#     160x80x80; the fd4 right-hand side gains little (74.9 against 75.5 us at 96x48x48).
+#     where the stencils reach NGHOSTS: rhs fd6 694 against 779 us at 192x96x96, 186 against 197
+#     at 128x64x64, 23.7 against 24.2 at 64x32x32 (plain: 3580, 1030, 115).  Ricci fd6's boxes have
+#     the same loads in both forms: 281 against 282 us, 87.7 against 86.7, 11.9 both, and within
+#     0.5% in whole steps from 64x32x32 to 192x96x96.
+#   * _tp forms mixed derivatives in two passes within a wave (``lds_kernel``): rhs fd6 694
+#     against 769 us at 192x96x96 and 186 against 211 at 128x64x64, Ricci fd6 281 against 389 and 88
+#     against 117 (there 128-thread tiles, too); Ricci fd4 132 against 151 at 160x80x80; the fd4
+#     right-hand side gains little (74.9 against 75.5 us at 96x48x48).
 #   * Small workgroups suit the kernels whose boxes are small: a wave then waits for its own
 #     box instead of three other waves', and several workgroups of a CU are at different
 #     points.  Ricci fd6, 128 threads against 256: 269 against 286 us at 192x96x96;
-#     phi-symmetric, 64 threads: Ricci 23.0 against 29.4 at 256x64x16, rhs (no xx2 halo) 42.9
-#     against 59.3.  The 3D right-hand side's boxes reach three or four points every way;
-#     there a 128-thread tile stages two thirds more halo and loses (843 against 691 us).
+#     phi-symmetric, 64 threads: Ricci 24.0 against 31.9 at 256x64x16 and 6.5 against 7.9 at
+#     72x12x2, rhs (no xx2 halo) 40.6 against 59.7 and 9.6 against 11.7.  The 3D right-hand side's
+#     boxes reach three or four points every way; there a 128-thread tile stages two thirds more
+#     halo and loses (843 against 691 us).
+# The forms between the first and the last are the fastest at no size measured.  They stay for what
+# selects them: _u32 takes rows and arrays of any parity and alignment at 0.4 to 0.9 of the plain
+# schedule's time, the 16x8x2 tiles and _lr40 are the second forms that the batched kernels, the
+# blocked tile order and the tuner's choice are checked on.
 FULL_CANDIDATES = {
-    "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_mi_xcd", "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk",
+    "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk",
             "p1_lb1_sj_L16x4x4x1_d4_dmo_rb1_io_pg_ub_sa_lr48_di_tp_ir_eb_mi_blk_xcd",
             "p1_lb1_sj_L16x4x4x1_d4_dma_rb1_io_pg_ub_sa_lr48_di_tp_mi_xcd_blk"],
-    "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_lr40_mi_xcd",
-              "r1_lb1_sj_L16x4x2x1_d3_dmo_rb1_io_pg_lr48_di_tp_mi_xcd", "r1_lb1_sj_L16x4x2x1_d3_dma_rb1_io_pg_lr48_di_tp_mi_xcd"],
+    "ricci": ["r1_lb1", "r1_lb1_sj_L16x4x2x1_d3_dmo_rb1_io_pg_lr48_di_tp_mi_xcd", "r1_lb1_sj_L16x4x2x1_d3_dma_rb1_io_pg_lr48_di_tp_mi_xcd"],
 }
 FULL_FD4_CANDIDATES = {
     "rhs": ["p1_lb1", "p1_lb1_sj_L16x4x4x1_d5_dmo_rb1_io_pg_ub_sa_lr48_di_tp_ir_eb_mi_xcd"],
@@ -978,8 +985,8 @@ SMALL_CANDIDATES = {"rhs": ["p1_lb1", "p1_lb1_sl_lf_pf16_u32_w2", "p1_lb1_sj_L16
 
 # The staged constraints kernel of every build (the plain one in bssn_kernels takes what this one
 # does not: input that is not 16-byte aligned, 2^29 points and more).  27 first and second
-# derivatives' worth of LDS reads a point; the tile and ring are those of the fd6 Ricci kernel.  100 us
-# at 128x64x64 fd6 against 453 us for the plain kernel.
+# derivatives' worth of LDS reads a point; 64-thread tiles and three ring slots.  94.8 us at 128x64x64 fd6
+# against 453 us for the plain kernel.
 CONSTRAINTS_STAGED = "k1_lb1_L16x2x2x1_d3_dmo_rb1_io_pg_lr40_di_mi_xcd"
 
 CAND_SIG = ("dim3 g, dim3 b, hipStream_t s, const double *in, const double *aux, double *out, "

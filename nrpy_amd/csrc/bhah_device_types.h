@@ -19,10 +19,8 @@ struct bhah_kparams {
 // substep.
 struct bhah_member {
   bhah_kparams kp;
-  const double *rfm0, *rfm1, *xx0;
+  const double *rfm0, *rfm1;
   double *arr[5];
-  int coord;
-  double AMPL, SINHW;
   const double *rad;  // r(xx0), dxx0/dr
   const int *inner_map, *inner_pairs;  // sources of the inner points, for the RK pass
 };

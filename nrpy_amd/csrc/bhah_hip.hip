@@ -1365,7 +1365,9 @@ const struct {
     {"Spherical_sym2_KO0_fd4", BHAH_KERNEL_RICCI, "r1_lb1_sj_L16x4x4x1_d2_dma_xcd"},
     {"Spherical_sym2_KO0_fd4", BHAH_KERNEL_RICCI, "r1_lb1_sj_L16x8x2x1_d3_dma_rb1_mi"},
     {"SinhSpherical_symnone_KO1_fd6", BHAH_KERNEL_RHS, "p1_lb1_sj_L16x4x4x1_d4_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk"},
+    {"SinhSpherical_symnone_KO1_fd6", BHAH_KERNEL_RHS, "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_mi_xcd"},
     {"SinhSpherical_symnone_KO1_fd6", BHAH_KERNEL_RICCI, "r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg2_mi_xcd"},
+    {"SinhSpherical_symnone_KO1_fd6", BHAH_KERNEL_RICCI, "r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_lr40_mi_xcd"},
     {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RHS, "p1_lb1_sl_lf_pf16_u32_w2"},
     {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RHS, "p1_lb1_sj_L16x8x2x1_d3_dma_rb1"},
     {"SinhSpherical_symnone_KO1_fd4", BHAH_KERNEL_RHS, "p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8"},
@@ -3019,7 +3021,6 @@ int bhah_hip_ensemble_bind(bhah_ensemble *E, const bhah_MoL_gridfunctions *gfs, 
     M.kp = P->kp(dt ? dt[m] : P->dt, 0);
     M.rfm0 = P->d_rfm0;
     M.rfm1 = P->d_rfm1;
-    M.xx0 = P->d_xx0;
     M.rad = P->d_rad;
     M.inner_map = P->d_inner_map;
     M.inner_pairs = P->d_inner_pairs;
@@ -3030,9 +3031,6 @@ int bhah_hip_ensemble_bind(bhah_ensemble *E, const bhah_MoL_gridfunctions *gfs, 
     M.arr[4] = g.auxevol_gfs;
     for (int a = 0; a < 4; a++)
       if ((uintptr_t)M.arr[a] & 15) aligned = false;
-    M.coord = P->d.coord;
-    M.AMPL = P->d.grid_physical_size;
-    M.SINHW = P->d.SINHW;
   }
   E->bound = false;  // until the device has the new arrays and the list that fits them
   E->invalidate_graph();

@@ -16,8 +16,10 @@ FD4_RICCI = ["r1_lb1_pf16_u32", "r1_lb1_sj_L16x4x4x1_d2_dma_xcd", "r1_lb1_sj_L16
 RETIRED = {
     (1, 4, 4, False): {RHS: ["p1_lb1_sj_L16x8x2x1_d3_dma_rb1_pg8_ub_mi"],
                        RICCI: ["r1_lb1_sj_L16x4x4x1_d2_dma_xcd", "r1_lb1_sj_L16x8x2x1_d3_dma_rb1_mi"]},
-    (2, 6, 0, True): {RHS: ["p1_lb1_sj_L16x4x4x1_d4_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk"],
-                      RICCI: ["r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg2_mi_xcd"]},
+    (2, 6, 0, True): {RHS: ["p1_lb1_sj_L16x4x4x1_d4_dma_rb1_io_pg_ub_sa_lr40_di_mi_xcd_blk",
+                            "p1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_ub_mi_xcd"],
+                      RICCI: ["r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg2_mi_xcd",
+                              "r1_lb1_sj_L16x4x4x1_d3_dma_rb1_io_pg_lr40_mi_xcd"]},
     (2, 4, 0, True): {RHS: FD4_RHS, RICCI: FD4_RICCI},
 }
 
