@@ -2,10 +2,10 @@
 the step with the separate copy (BHAH_HIP_SEPARATE_INNER_BC=1 at patch creation): the same
 state bit for bit, eagerly and through the cached graph, at the default schedules and tile.
 
-The fold needs every pair of points (2q, 2q+1) to find both sources of its k in one 16-byte-
-aligned pair; the first case (fd6, four ghost zones, even rows) meets that, which the test
-checks from the patch's inner boundary lists, so the folded pass is the one compared.  The
-second case (fd4, three ghost zones) does not, and its step keeps the separate copy."""
+In the first case (fd6, four ghost zones, even rows) every pair of points (2q, 2q+1) finds both
+sources of its k in one 16-byte-aligned pair; in the second (fd4, three ghost zones) some pairs'
+sources lie apart and are taken with two 8-byte loads.  The test checks from the patch's inner
+boundary lists which form it compares."""
 
 import os
 
@@ -25,7 +25,7 @@ CASES = {
 
 
 def pairs_fit(P) -> bool:
-    """Whether both points of every pair take k from one aligned pair (the fold's condition)."""
+    """Whether both points of every pair take k from one aligned pair."""
     dst, src, _ = P.inner_bc()
     n = int(np.prod(P.Nx))
     s = np.arange(n, dtype=np.int64)
