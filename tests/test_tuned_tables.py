@@ -46,3 +46,12 @@ def test_tuner_times_tiles_on_the_schedules_that_run_in_them(hip, monkeypatch):
                         log=lambda s: None)
     assert at_tile == [("p1_lb1", "r1_lb1")] * len(autotune.TILES)
     assert out["tile"] in [list(t) for t in autotune.TILES]
+
+
+@pytest.mark.parametrize("Nxx", [(72, 12, 2), (151, 33, 10), (256, 64, 16)])
+def test_phi_symmetric_plain_schedules_run_in_the_tile_their_table_chose(Nxx):
+    """32x8: rows of 151 points fill 5 x 5 x 10 workgroups, one round of the 256 CUs; 64x4 takes 3 x 9
+    x 10, two rounds (Ricci and right-hand side 80 against 136 us there; never slower elsewhere)."""
+    from nrpy_amd.runtime import PatchConfig
+
+    assert autotune.load_choice(PatchConfig(coord=1, Nxx=Nxx, fd_order=4, symmetry_axes=4))["tile"] == [32, 8]
