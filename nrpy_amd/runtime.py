@@ -214,11 +214,13 @@ def _check(rc: int) -> None:
         raise BHaHError(f"bhah_hip error {rc}: {msg}")
 
 
-def _schedule_index(find, handle, kind: int, name_or_index) -> int:
+def _schedule_index(names, find, handle, kind: int, name_or_index) -> int:
     """Index of a schedule given by index or name (names of schedules that earlier builds had and
     this one replaces included); ValueError for a name the build never had."""
     if not isinstance(name_or_index, str):
         return int(name_or_index)
+    if name_or_index in names:
+        return names.index(name_or_index)
     idx = find(handle, kind, name_or_index.encode())
     if idx == BHAH_ERR_ARG:
         raise ValueError(load_library().bhah_hip_last_error().decode())
@@ -368,7 +370,8 @@ class Patch:
         return [self.lib.bhah_hip_patch_schedule_name(self.handle, kind, i).decode() for i in range(n)]
 
     def select_schedule(self, kind: int, name_or_index):
-        idx = _schedule_index(self.lib.bhah_hip_patch_find_schedule, self.handle, kind, name_or_index)
+        idx = _schedule_index(self.schedules(kind), self.lib.bhah_hip_patch_find_schedule, self.handle, kind,
+                              name_or_index)
         _check(self.lib.bhah_hip_patch_select_schedule(self.handle, kind, idx))
 
     def schedule(self, kind: int) -> str:
@@ -579,7 +582,8 @@ class Ensemble:
         return self.members[0].schedules(kind)
 
     def select_schedule(self, kind: int, name_or_index):
-        idx = _schedule_index(self.lib.bhah_hip_ensemble_find_schedule, self.handle, kind, name_or_index)
+        idx = _schedule_index(self.schedules(kind), self.lib.bhah_hip_ensemble_find_schedule, self.handle, kind,
+                              name_or_index)
         _check(self.lib.bhah_hip_ensemble_select_schedule(self.handle, kind, idx))
         self.choice[kind] = idx
 

@@ -90,3 +90,17 @@ def test_stored_table_with_an_unknown_name_warns(hip, monkeypatch):
     with pytest.warns(UserWarning, match="p9_lb1"):
         autotune.apply_tuned(P)
     assert (P.schedule(RHS), P.schedule(RICCI)) == before
+
+
+def test_refusals_keep_their_errors(hip):
+    from nrpy_amd.runtime import CARTESIAN, SYSTEM_WAVE, BHaHError, Patch, PatchConfig
+
+    W = Patch(PatchConfig(system=SYSTEM_WAVE, coord=CARTESIAN, Nxx=(4, 4, 4), fd_order=4, symmetry_axes=0,
+                          grid_physical_size=10.0, wavespeed=1.0))
+    with pytest.raises(BHaHError, match="not a BSSN patch"):
+        W.select_schedule(RHS, "p1_lb1")
+    P = Patch(_cfg((1, 4, 4, False), (24, 6, 2)), tuned=False)
+    with pytest.raises(BHaHError, match="unknown kernel kind"):
+        P.select_schedule(7, "p1_lb1")
+    with pytest.raises(BHaHError, match="out of range"):
+        P.select_schedule(RHS, len(P.schedules(RHS)))
